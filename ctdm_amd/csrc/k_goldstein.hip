@@ -5,11 +5,9 @@
 //   1. k_gs_residues  one thread per pixel: the reference's wrapped differences with its float /
 //                     double promotions, summed in float, thresholded at +-6.
 //   2. branch cuts, deterministic raster order (the reference runs its search for all residues
-//      concurrently, which is racy; the raster order makes it reproducible). Three phases:
-//      k_gs_rank + k_gs_cand list every residue's first hits on the initial charges in parallel (one
-//      thread per residue), k_gs_commit (one wavefront per map, presence at 1 bit per pixel, in LDS when
-//      it fits, else in global memory) walks the residues in order and takes the first listed hit still
-//      present, and k_gs_draw draws the chosen cuts in parallel.
+//      concurrently, which is racy; the raster order makes it reproducible): k_gs_pair (one workgroup per
+//      map) pairs the residues, with rows side by side where no decision can reach another's, and k_gs_draw
+//      draws the chosen cuts in parallel.
 //   3. flood fill: level-synchronous breadth-first search over non-cut pixels from a fixed start; each
 //                     new pixel takes k from its first neighbour of the previous level in the order
 //                     right, left, below, above. Maps whose cut bits fit in LDS (up to 1.3 M pixels):
@@ -23,6 +21,7 @@
 // built with -ffp-contract=off (the _rn intrinsics are plain operations that the compiler would
 // otherwise fuse into FMAs), matching the host specification compiled without contraction.
 #include <climits>
+#include <type_traits>
 
 #include "internal.hpp"
 
@@ -61,7 +60,9 @@ __device__ __forceinline__ void pixel_of_grid(int W, int& x, int& y, long long& 
 }
 
 // ---------------------------------------------------------------- 1. residues
-__global__ void k_gs_residues(const float* __restrict__ phi, int batch, int H, int W, int8_t* __restrict__ res)
+// Also starts the cut mask: a residue on the border is its own cut, every other pixel is clear.
+__global__ void k_gs_residues(const float* __restrict__ phi, int batch, int H, int W, int8_t* __restrict__ res,
+                              uint8_t* __restrict__ cuts)
 {
     const long long n = (long long)H * W;
     int i, j;
@@ -79,6 +80,7 @@ __global__ void k_gs_residues(const float* __restrict__ phi, int batch, int H, i
         q = s >= 6.0f ? 1 : (s <= -6.0f ? -1 : 0);
     }
     res[g] = q;
+    cuts[g] = q != 0 && (i == 0 || j == 0);
 }
 
 // ---------------------------------------------------------------- 2. branch cuts
@@ -107,398 +109,387 @@ __device__ __forceinline__ unsigned nonzero_bits(const uint8_t* __restrict__ m, 
     return v;
 }
 
-// Word w of the bit array of a residue map's negative charges (bit b: pixel 32 w + b; pixels past n: 0).
-__device__ __forceinline__ unsigned negative_bits(const int8_t* __restrict__ m, long long n, int w)
+// Words w of the bit arrays of a residue map's charges, x: positive, y: negative (bit b: pixel 32 w + b;
+// pixels past n: 0). Bytes are 0, 1 or -1: bit 0 tells a charge, bit 7 its sign, and a multiplication moves
+// the four flags of a 32-bit load (bits 0, 8, 16, 24) to bits 28-31 without carries.
+__device__ __forceinline__ uint2 charge_bits(const int8_t* __restrict__ m, long long n, int w)
 {
     const long long p0 = (long long)w * 32;
-    int8_t q[32];
+    unsigned any = 0, neg = 0;
+    if (p0 + 32 <= n && ((reinterpret_cast<uintptr_t>(m + p0) & 15) == 0)) {
+        const uint4 a = *reinterpret_cast<const uint4*>(m + p0);
+        const uint4 b = *reinterpret_cast<const uint4*>(m + p0 + 16);
+        const unsigned q[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-    for (int k = 0; k < 32; ++k) q[k] = m[min(p0 + k, n - 1)];
-    unsigned v = 0;
+        for (int k = 0; k < 8; ++k) {
+            any |= (((q[k] & 0x01010101u) * 0x10204080u) >> 28) << (4 * k);
+            neg |= ((((q[k] >> 7) & 0x01010101u) * 0x10204080u) >> 28) << (4 * k);
+        }
+    } else {
+        int8_t q[32];
 #pragma unroll
-    for (int k = 0; k < 32; ++k) v |= (unsigned)(p0 + k < n && q[k] < 0) << k;
-    return v;
+        for (int k = 0; k < 32; ++k) q[k] = m[min(p0 + k, n - 1)];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+            any |= (unsigned)(p0 + k < n && q[k] != 0) << k;
+            neg |= (unsigned)(p0 + k < n && q[k] < 0) << k;
+        }
+    }
+    return make_uint2(any & ~neg, neg);
 }
 
-// Charges still present: 1 bit per pixel, 32 pixels per word. A charge keeps its sign until it is
-// removed, so the sign is read from the residue map. The words live in LDS when a map's words fit
-// (maps up to 1.3 M pixels in 160 KiB), else in global memory; either way one wavefront reads and
-// clears them (in global memory through atomics at device scope, which bypass the vector L1).
+// ---------------------------------------------------------------- 2b. branch cuts: rows in a pipeline
+// The search visits the residues in raster order: a residue that is still present takes the first point of
+// its box scan (rings of radius 1, 2, ..., below R) that is a border point or a present charge of the opposite
+// sign, and both charges are removed. A residue on the border takes itself; no other residue removes it (the
+// border is met first), so those are left out here and marked as cuts beside the residues (k_gs_residues).
+//
+// A decision only reads and changes pixels within its reach (the ring of its hit), so rows can run side by
+// side when each stays behind the one above. One workgroup per map, one group of GS_LANES lanes per row in
+// flight. Each group publishes the pixel up to which its row is decided (raster index; a wave's LDS
+// operations execute in order, so removals precede the index that covers them). With c the first column the
+// row above has not published and rho a bound on every reach, a residue at column x takes a hit on ring r
+// once x + r + rho < c, and a row publishes at most c - rho - 1. If every reach is at most rho, its scan then
+// sees
+//   - every earlier residue's removals: undecided ones lie at columns >= c in the row above and further right
+//     in the rows before, so they change columns >= c - rho only;
+//   - no later residue's: those decided changed columns < x - rho.
+// so all decisions are those of the raster order. A hit beyond rho ends the attempt, and the map starts again
+// with 4 rho, then with R, which no reach exceeds. A small rho keeps the rows close together and more of them
+// in flight; it follows the residue density, as the nearest opposite charges are close where residues are
+// many. Reaches over maps of 8 Gaussians plus uniform noise of +-a pi: at most 7 at densities 0.28 (a = 0.8;
+// one in 150 000 is 6) and 0.20 (0.7), 10 at 0.10 (0.6, 256^2), 12 at 0.09, 16 at 0.04 (0.55), each ring
+// further 3 to 15 times rarer, so a second attempt stays below one map in a hundred.
+//
+// Bound: the chain of dependent decisions along the front (about 2 300 steps for 512 rows of density 0.28,
+// 13 decisions side by side). In a step a group reads the row above's index, its row's next 31 pixels and the
+// opposite charges on rings 1-3 of the pixel it stands on (one LDS round trip), looks the first hit up (another)
+// and removes the pair; the work of a step is done on vectors of rows, one instruction for the eight rows of a
+// wave, since a wavefront alone on its SIMD takes about five cycles per instruction whatever its lanes do.
+// Measured: 64 maps of 512^2 at density 0.28 in 1.0 ms, one 256^2 map at 0.10 in 0.46 ms, against 7.6 and
+// 0.74 ms for one wavefront per map that visited the residues one after the other.
+constexpr int GS_LANES = 8;                       // lanes per row: rows -3 .. 3 around it (the last lane idle)
+constexpr int GS_WAVES = 4;                       // wavefronts per map
+constexpr int GS_ROWS = GS_WAVES * 64 / GS_LANES; // rows in flight
+constexpr int GS_LEFT = INT_MIN;                  // published by a group that leaves its rows undecided
+
+// The charges still present as two bit arrays, positive and negative, with the border's bits set in both; nw
+// words each, one spare word before them and two after. In LDS when they fit (maps up to 0.65 M pixels), else in global memory, read and
+// cleared by atomics at device scope, which bypass the vector L1.
 template <bool LDSW>
-struct Presence {
-    unsigned* w;
-    __device__ __forceinline__ unsigned get(int i) const
+struct Charges {
+    unsigned* w;   // positive charges, then negative ones from word nw + 3
+    int nw;
+    __device__ __forceinline__ unsigned ld(int i) const
     {
         if constexpr (LDSW)
-            return w[i];
+            return __hip_atomic_load(w + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         else
             return __hip_atomic_load(w + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __device__ __forceinline__ bool at(int pix) const { return (get(pix >> 5) >> (pix & 31)) & 1u; }
-    __device__ __forceinline__ void clear(int pix) const
+    // first word of the charges of one sign
+    __device__ __forceinline__ int plane(bool negative) const { return negative ? nw + 3 : 0; }
+    __device__ __forceinline__ void clear(int p, bool negative) const
     {
-        const unsigned m = ~(1u << (pix & 31));
+        unsigned* a = w + plane(negative) + (p >> 5);
+        const unsigned m = ~(1u << (p & 31));
         if constexpr (LDSW)
-            atomicAnd(w + (pix >> 5), m);
+            atomicAnd(a, m);
         else
-            __hip_atomic_fetch_and(w + (pix >> 5), m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_and(a, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void set_border(int p) const
+    {
+        for (int s = 0; s < 2; ++s) {
+            if constexpr (LDSW)
+                atomicOr(w + plane(s) + (p >> 5), 1u << (p & 31));
+            else
+                __hip_atomic_fetch_or(w + plane(s) + (p >> 5), 1u << (p & 31), __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
 };
 
-// ---------------------------------------------------------------- 2b. branch cuts in three phases
-// The same result as the raster-order search, with most of the work in parallel. Charges only ever
-// disappear, and a border point is always a hit, so the first hit of a residue's scan at the time it is
-// processed is the first point of its scan that was a hit initially and is still present. Hence:
-//   1. every residue (in parallel) lists the first GS_K hits of its scan on the initial charges, stopping
-//      at a border point (always valid) or when the box radius runs out;
-//   2. one wavefront per map walks the residues in raster order and takes the first listed hit that is
-//      still present; only when all GS_K listed charges are gone does it scan again (a full rescan from
-//      radius 1 finds the same point as continuing the scan: the earlier points are all non-hits now);
-//   3. the chosen cuts are drawn in parallel (cut pixels are only ever set to 1).
-constexpr int GS_K = 4;
-constexpr int GS_META_SELF = 8;        // residue on the border: balanced by a one-pixel cut
-constexpr int GS_META_TERM = 16;       // the list ends with a border point
-constexpr int GS_META_EXHAUSTED = 32;  // the scan reached the largest box without GS_K hits or a border
-constexpr int GS_META_NEG = 64;        // the residue's charge is -1
-
-// Residues per block of 1024 pixels.
-__global__ __launch_bounds__(1024) void k_gs_count(const int8_t* __restrict__ res, long long n, int nblk,
-                                                   int* __restrict__ blkcnt)
+// Position q of ring r's scan order, unclipped: left column top to bottom, then the columns between on the
+// top and bottom rows in turn, then the right column top to bottom.
+__device__ __forceinline__ void ring_position(int r, int q, int& dx, int& dy)
 {
-    __shared__ int wc[16];
-    const long long map = blockIdx.x / nblk, blk = blockIdx.x % nblk;
-    const long long p = blk * 1024 + threadIdx.x;
-    const bool q = p < n && res[map * n + p] != 0;
-    const unsigned long long m = __ballot(q);
-    if ((threadIdx.x & 63) == 0) wc[threadIdx.x >> 6] = __popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int w = 0; w < 16; ++w) t += wc[w];
-        blkcnt[blockIdx.x] = t;
+    const int side = 2 * r + 1, q2 = q - side, nmid = 2 * (side - 2);
+    dx = q < side ? -r : (q2 < nmid ? 1 - r + (q2 >> 1) : r);
+    dy = q < side ? q - r : (q2 < nmid ? ((q2 & 1) ? r : -r) : q2 - nmid - r);
+}
+
+// The scan of one residue beyond ring 3 by a whole wavefront, 64 positions of the scan order per round (the
+// first hit is the lowest lane with one). Returns the hit's pixel, -1 for no hit; sets `far` for a hit beyond ring
+// rho, or none up to it. No ring is clipped before the one that touches the border, which holds a hit, so the
+// first round (ring 4 and 32 positions of ring 5, fixed offsets) needs no look at the borders.
+template <bool LDSW>
+__device__ int gs_scan(const Charges<LDSW>& ch, int H, int W, int R, int p, int i, int j, int opp, int lane, int rho,
+                       bool& far)
+{
+    if (R <= 4) return -1;
+    int rc = 4, o0 = 0;  // next position: ring rc, index o0
+    if (R > 5 && rho >= 5) {
+        int dx, dy;
+        ring_position(lane < 32 ? 4 : 5, lane & 31, dx, dy);
+        const int q = p + dx + W * dy;
+        const unsigned wq = min((unsigned)(q >> 5), (unsigned)ch.nw);
+        const unsigned long long hit = __ballot((ch.ld(opp + (int)wq) >> (q & 31)) & 1u);
+        if (hit) {
+            const int l = __builtin_ctzll(hit);
+            return __builtin_amdgcn_readlane(q, l);
+        }
+        rc = 5;
+        o0 = 32;
     }
-}
-
-// Exclusive scan of the block counts of one map (one thread per map; a few hundred blocks).
-__global__ void k_gs_scan(int* __restrict__ blkcnt, int nblk, int batch, int* __restrict__ nres)
-{
-    const int map = blockIdx.x * blockDim.x + threadIdx.x;
-    if (map >= batch) return;
-    int acc = 0;
-    for (int b = 0; b < nblk; ++b) {
-        const int v = blkcnt[(long long)map * nblk + b];
-        blkcnt[(long long)map * nblk + b] = acc;
-        acc += v;
-    }
-    nres[map] = acc;
-}
-
-// Phase 1a: one thread per pixel; each residue writes its pixel at its raster rank (rec_pm.x).
-__global__ __launch_bounds__(1024) void k_gs_rank(const int8_t* __restrict__ res, int H, int W, int nblk,
-                                                  const int* __restrict__ blkoff, int2* __restrict__ rec_pm)
-{
-    __shared__ int wc[16];
-    const long long n = (long long)H * W;
-    const long long map = blockIdx.x / nblk, blk = blockIdx.x % nblk;
-    const long long p = blk * 1024 + threadIdx.x;
-    const int q = p < n ? res[map * n + p] : 0;
-    const unsigned long long m = __ballot(q != 0);
-    const int lane = threadIdx.x & 63;
-    if (lane == 0) wc[threadIdx.x >> 6] = __popcll(m);
-    __syncthreads();
-    if (q == 0) return;
-    int rank = blkoff[blockIdx.x] + __popcll(m & ((1ull << lane) - 1ull));
-    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) rank += wc[w];
-    rec_pm[map * n + rank] = make_int2((int)p, 0);
-}
-
-// Phase 1b: one thread per residue (raster rank), so that the scans fill whole wavefronts; the record
-// gets the residue's list. A listed hit is encoded as kind << 30 | target pixel (kind 1: column border,
-// cut along the row; 2: row border, cut along the column; 3: opposite charge), kind 0 with the
-// residue's own pixel for a border residue.
-__global__ __launch_bounds__(1024) void k_gs_cand(const int8_t* __restrict__ res, int H, int W, int nblk,
-                                                  const int* __restrict__ nres, int2* __restrict__ rec_pm,
-                                                  int4* __restrict__ rec_c)
-{
-    const long long n = (long long)H * W;
-    const long long map = blockIdx.x / nblk, rank = (blockIdx.x % nblk) * 1024 + threadIdx.x;
-    if (rank >= nres[map]) return;
-    const long long o = map * n + rank;
-    const int8_t* r = res + map * n;
-    const long long p = rec_pm[o].x;
-    const int q = r[p];
-    const int i = (int)(p % W), j = (int)(p / W);
-    int cand[GS_K] = {0, 0, 0, 0};
-    int cnt = 0, meta = 0;
-    if (i <= 0 || i >= W - 1 || j <= 0 || j >= H - 1) {
-        meta = GS_META_SELF;  // its one listed hit is itself (kind 0), which no commit removes
-        cand[0] = (int)p;
-        cnt = 1;
-    } else {
-        const int R = min(901, W / 2);
-        bool stop = false;
-        int rr = 1;
-        for (; rr < R && !stop; ++rr) {
-            const int m1 = max(i - rr, 0), m2 = min(i + rr, W - 1);
-            const int n1 = max(j - rr, 0), n2 = min(j + rr, H - 1);
-            for (int mm = m1; mm <= m2 && !stop; ++mm) {
-                const int ndel = (mm == m1 || mm == m2) ? 1 : (n2 - n1);
-                for (int nn = n1; nn <= n2 && !stop; nn += ndel) {
-                    unsigned c = 0;
-                    bool hit = true;
-                    if (mm <= 0 || mm >= W - 1) {
-                        c = (1u << 30) | (unsigned)(mm + W * j);
-                        meta |= GS_META_TERM;
-                    } else if (nn <= 0 || nn >= H - 1) {
-                        c = (2u << 30) | (unsigned)(i + W * nn);
-                        meta |= GS_META_TERM;
-                    } else if (q * r[mm + (long long)W * nn] == -1) {
-                        c = (3u << 30) | (unsigned)(mm + W * nn);
-                    } else {
-                        hit = false;
-                    }
-                    if (hit) {
-                        cand[cnt++] = (int)c;
-                        stop = (meta & GS_META_TERM) || cnt == GS_K;
-                    }
-                }
+    while (rc < R) {
+        if (rc > rho) {
+            far = true;
+            return -1;
+        }
+        int lr = R, lq = 0;  // lanes past the last ring scan nothing
+        int start = 0, rr = rc, off = o0;
+        while (start < 64 && rr < R) {
+            const int P = 2 * (min(j + rr, H - 1) - max(j - rr, 0) + 1) +
+                          2 * (min(i + rr, W - 1) - max(i - rr, 0) - 1);
+            const int take = min(P - off, 64 - start);
+            if (lane >= start && lane < start + take) {
+                lr = rr;
+                lq = off + lane - start;
+            }
+            start += take;
+            off += take;
+            if (off == P) {
+                ++rr;
+                off = 0;
             }
         }
-        if (!stop) meta |= GS_META_EXHAUSTED;
+        int c = 0;
+        bool here = false;
+        if (lr < R) {
+            const int m1 = max(i - lr, 0), m2 = min(i + lr, W - 1);
+            const int n1 = max(j - lr, 0), n2 = min(j + lr, H - 1);
+            const int nrow = n2 - n1 + 1, nmid = 2 * (m2 - m1 - 1);
+            const int q2 = lq - nrow;
+            const bool left = lq < nrow, mid = !left && q2 < nmid;
+            const int mm = left ? m1 : (mid ? m1 + 1 + (q2 >> 1) : m2);
+            const int nn = left ? n1 + lq : (mid ? ((q2 & 1) ? n2 : n1) : n1 + (q2 - nmid));
+            const int q = mm + W * nn;
+            c = q;
+            here = (ch.ld(opp + (q >> 5)) >> (q & 31)) & 1u;
+        }
+        const unsigned long long hit = __ballot(here);
+        if (hit) {
+            const int l = __builtin_ctzll(hit);
+            far = __builtin_amdgcn_readlane(lr, l) > rho;
+            return __builtin_amdgcn_readlane(c, l);
+        }
+        rc = rr;
+        o0 = off;
     }
-    rec_pm[o] = make_int2((int)p, meta | cnt | (q < 0 ? GS_META_NEG : 0));
-    rec_c[o] = make_int4(cand[0], cand[1], cand[2], cand[3]);
+    return -1;
 }
 
-__device__ __forceinline__ int sel4(const int4& v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : (k == 2 ? v.z : v.w)); }
+// Minimum over the eight lanes of a row's group.
+__device__ __forceinline__ unsigned group_min(unsigned v)
+{
+    static_assert(GS_LANES == 8, "group reduction");
+    auto step = [&](auto ctrl) {
+        const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(-1, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
+        v = o < v ? o : v;
+    };
+    step(std::integral_constant<int, 0xb1>{});   // quad_perm 1 0 3 2
+    step(std::integral_constant<int, 0x4e>{});   // quad_perm 2 3 0 1
+    step(std::integral_constant<int, 0x141>{});  // mirrored within 8 lanes
+    return v;
+}
 
-// Phase 2: one wavefront per map, residues in raster order. Residues are taken 64 at a time, one per
-// lane. Each lane reads, once per batch, whether its residue and its listed hits are still present;
-// those flags are kept as wave-wide lane masks (one for the residues, one per list position), so a
-// residue's choice is a few scalar bit tests, and after each commit the masks lose the lanes whose
-// residue or listed hit that commit removed (vector compares of the two removed pixels against every
-// lane's pixels). Each committing lane keeps its choice in a register and a mask records which lanes
-// committed; the pairs are written (in commit order, which is lane order) and their charges cleared
-// once at the end of the batch, so the loop itself issues no memory operation. A residue whose listed charges are all gone clears the batch's
-// charges so far (clearing twice is harmless) and scans again on the current charges (the signs of
-// the charges it meets come from the residue map).
+// Scan key of the point (dx, dy) on rings 1-3, ordered as the scan: order << 10 | ring << 8 | dx + 8 << 4 | dy + 8.
+constexpr unsigned GS_NONE = 0xffffu;
+__device__ __forceinline__ unsigned ring_key(int dx, int dy)
+{
+    const int r = max(abs(dx), abs(dy)), side = 2 * r + 1;
+    const int q = dx == -r ? dy + r : (dx == r ? side + 2 * (side - 2) + dy + r : side + 2 * (dx + r - 1) + (dy > 0));
+    return (unsigned)((q + (r == 1 ? 0 : (r == 2 ? 8 : 24))) << 10 | r << 8 | (dx + 8) << 4 | (dy + 8));
+}
+
 template <bool LDSW>
-__global__ __launch_bounds__(64) void k_gs_commit(const int8_t* __restrict__ res, int H, int W,
-                                                  const int* __restrict__ nres, const int2* __restrict__ rec_pm,
-                                                  const int4* __restrict__ rec_c, unsigned* __restrict__ gwords,
-                                                  int sign_lds, int2* __restrict__ pairs, int* __restrict__ npairs)
+__global__ __launch_bounds__(64 * GS_WAVES) void k_gs_pair(const int8_t* __restrict__ res, int H, int W,
+                                                           unsigned* __restrict__ gwords, int2* __restrict__ pairs,
+                                                           int* __restrict__ rowpairs)
 {
     extern __shared__ unsigned lwords[];
-    const int lane = threadIdx.x;
+    // prog[first lane of a group]: its published index (the other lanes write the words beside it, which
+    // costs less than masking them)
+    __shared__ int prog[64 * GS_WAVES], failed, nres;
+    __shared__ unsigned short first_key[8 * 128];  // [row dy + 3][charges at dx = -3 .. 3]: key of the first hit
+    constexpr int NT = 64 * GS_WAVES;
+    const int tid = threadIdx.x, lane = tid & 63, l = lane % GS_LANES, slot = tid / GS_LANES;
     const long long n = (long long)H * W;
     const int nw = (int)((n + 31) / 32);
-    const Presence<LDSW> pr{LDSW ? lwords : gwords + (long long)blockIdx.x * nw};
     const int8_t* r = res + blockIdx.x * n;
-    for (int w = lane; w < nw; w += 64) pr.w[w] = nonzero_bits(reinterpret_cast<const uint8_t*>(r), n, w);
-    // sign bits (1: charge -1) after the presence bits when both fit: rescans then read no residue map
-    const unsigned* sg = lwords + nw;
-    if (sign_lds)
-        for (int w = lane; w < nw; w += 64) lwords[nw + w] = negative_bits(r, n, w);
-    if constexpr (!LDSW) __threadfence();
-    __syncthreads();
-    const int total = nres[blockIdx.x];
-    const int2* pm = rec_pm + blockIdx.x * n;
-    const int4* rc = rec_c + blockIdx.x * n;
-    int2* out = pairs + blockIdx.x * n;
+    int2* out = pairs + blockIdx.x * n;  // row y's choices start at out[y W], nrow[y] of them
+    int* nrow = rowpairs + (long long)blockIdx.x * H;
+    const Charges<LDSW> ch{(LDSW ? lwords : gwords + (long long)blockIdx.x * 2 * (nw + 3)) + 1, nw};
     const int R = min(901, W / 2);
-    int emitted = 0;
-    int2 nxt_pm = lane < total ? pm[lane] : make_int2(0, 0);
-    int4 nxt_c = lane < total ? rc[lane] : make_int4(0, 0, 0, 0);
-    // The first batch's records are waited for here, so that no batch waits for the records of the one
-    // after it (loaded at its start) before its own work.
-    __builtin_amdgcn_s_waitcnt(0);
-    for (int base = 0; base < total; base += 64) {
-        const int2 mypm = nxt_pm;
-        const int4 myc = nxt_c;
-        const int nidx = base + 64 + lane;  // the next batch's records load while this one commits
-        nxt_pm = nidx < total ? pm[nidx] : make_int2(0, 0);
-        nxt_c = nidx < total ? rc[nidx] : make_int4(0, 0, 0, 0);
-        const bool in = lane < min(64, total - base);
-        const int cn = mypm.y & 7;
-        // cpix[k]: the pixel of the k-th listed hit when it is a charge (a commit can remove it), else -1
-        // (presence is read for every lane and position, at pixel 0 where there is nothing to read, so
-        // that the five reads issue together)
-        int cpix[GS_K];
-        bool hv[GS_K];
-#pragma unroll
-        for (int k = 0; k < GS_K; ++k) {
-            const unsigned c = (unsigned)sel4(myc, k);
-            cpix[k] = (c >> 30) == 3u ? (int)(c & 0x3fffffffu) : -1;
-            const bool pres = pr.at(max(cpix[k], 0));
-            hv[k] = in && k < cn && (cpix[k] < 0 || pres);
+    for (int e = tid; e < 8 * 128; e += NT) {
+        unsigned best = GS_NONE;
+        const int dy = (e >> 7) - 3;
+        for (int k = 0; k < 7; ++k) {
+            const int dx = k - 3, rg = max(abs(dx), abs(dy));
+            if (dy <= 3 && rg > 0 && rg < R && ((e >> k) & 1)) best = min(best, ring_key(dx, dy));
         }
-        const bool rpres = pr.at(mypm.x);
-        unsigned long long live = __ballot(in && rpres);
-        unsigned long long h0 = __ballot(hv[0]), h1 = __ballot(hv[1]), h2 = __ballot(hv[2]), h3 = __ballot(hv[3]);
-        // this batch's commits: the lanes whose residue committed (commits go in lane order) and, in each
-        // such lane, its choice
-        unsigned long long done = 0;
-        int mych = 0;
-        while (live) {
-            const int l = __ffsll((long long)live) - 1;
-            const unsigned long long bit = 1ull << l;
-            live &= ~bit;
-            const int p = __builtin_amdgcn_readlane(mypm.x, l);
-            // the first listed hit still present (a residue on the border lists itself, kind 0); -1 when
-            // there is none (no choice encodes to -1: pixels stay below 2^30 - 1). Scalar selects, no branch.
-            const int c0 = __builtin_amdgcn_readlane(myc.x, l), c1 = __builtin_amdgcn_readlane(myc.y, l);
-            const int c2 = __builtin_amdgcn_readlane(myc.z, l), c3 = __builtin_amdgcn_readlane(myc.w, l);
-            // (instruction order, held by scheduling barriers: the five reads first, so that their
-            // latencies overlap, then the vector compares that need only p, then the scalar selects,
-            // then the compares that need the choice, and the mask updates last)
-            __builtin_amdgcn_sched_barrier(0);
-            const unsigned long long e0 = __ballot(cpix[0] == p), e1 = __ballot(cpix[1] == p);
-            const unsigned long long e2 = __ballot(cpix[2] == p), e3 = __ballot(cpix[3] == p);
-            __builtin_amdgcn_sched_barrier(0);
-            // The selects as scalar-ALU assembly: s_and_b64 sets SCC to (mask & bit) != 0, which
-            // s_cselect_b32 reads directly (compiled code inserts an s_cmp before each select). Scalar
-            // registers only, no memory access; SCC is declared clobbered.
-            int chosen;
-            unsigned long long tsel;
-            asm volatile(
-                "s_and_b64 %[t], %[b], %[h3]\n\t"
-                "s_cselect_b32 %[ch], %[c3], -1\n\t"
-                "s_and_b64 %[t], %[b], %[h2]\n\t"
-                "s_cselect_b32 %[ch], %[c2], %[ch]\n\t"
-                "s_and_b64 %[t], %[b], %[h1]\n\t"
-                "s_cselect_b32 %[ch], %[c1], %[ch]\n\t"
-                "s_and_b64 %[t], %[b], %[h0]\n\t"
-                "s_cselect_b32 %[ch], %[c0], %[ch]"
-                : [ch] "=&s"(chosen), [t] "=&s"(tsel)
-                : [b] "s"(bit), [h0] "s"(h0), [h1] "s"(h1), [h2] "s"(h2), [h3] "s"(h3), [c0] "s"(c0), [c1] "s"(c1),
-                  [c2] "s"(c2), [c3] "s"(c3)
-                : "scc");
-            bool found = chosen != -1;
-            if (__builtin_expect(!found, 0)) {
-                const int meta = __builtin_amdgcn_readlane(mypm.y, l);
-                if (meta & (GS_META_TERM | GS_META_EXHAUSTED)) continue;  // nothing within reach: unbalanced
-                // every listed charge is gone: scan again on the current charges
-                if ((done >> lane) & 1ull) {
-                    pr.clear(mypm.x);
-                    if (((unsigned)mych >> 30) == 3u) pr.clear(mych & 0x3fffffff);
-                }
-                if constexpr (!LDSW) __builtin_amdgcn_s_waitcnt(0);
-                const int q = (meta & GS_META_NEG) ? -1 : 1;
-                const int i = p % W, j = p / W;
-                // The box rings 1, 2, ... (radius below R) in scan order, 64 positions per round: each
-                // lane takes the next position (ring lr, index lq on that ring), several rings per round
-                // while they are short; the first hit in scan order is the lowest lane with a hit. Rings
-                // that no border clips have 8 r positions, so a first round 4 or more pixels from every
-                // border takes rings 1-3 and the first 16 positions of ring 4 with a fixed lane layout.
-                const bool inner = R > 4 && i >= 4 && i <= W - 5 && j >= 4 && j <= H - 5;
-                int rc = 1, off0 = 0;  // next position to scan: ring rc, index off0
-                while (!found && rc < R) {
-                    int lr = R, lq = 0;  // lanes past the last ring scan nothing
-                    int start = 0, rr = rc, off = off0;
-                    if (rc == 1 && inner) {
-                        lr = lane < 8 ? 1 : (lane < 24 ? 2 : (lane < 48 ? 3 : 4));
-                        lq = lane - (lane < 8 ? 0 : (lane < 24 ? 8 : (lane < 48 ? 24 : 48)));
-                        start = 64;
-                        rr = 4;
-                        off = 16;
-                    }
-                    while (start < 64 && rr < R) {
-                        const int P = 2 * (min(j + rr, H - 1) - max(j - rr, 0) + 1) +
-                                      2 * (min(i + rr, W - 1) - max(i - rr, 0) - 1);
-                        const int take = min(P - off, 64 - start);
-                        if (lane >= start && lane < start + take) {
-                            lr = rr;
-                            lq = off + lane - start;
-                        }
-                        start += take;
-                        off += take;
-                        if (off == P) {
-                            ++rr;
-                            off = 0;
-                        }
-                    }
-                    int c = 0;
-                    bool hit_here = false;
-                    if (lr < R) {
-                        // ring lr's positions: its left column top to bottom, then the columns between
-                        // alternately on its top and bottom rows, then its right column top to bottom
-                        const int m1 = max(i - lr, 0), m2 = min(i + lr, W - 1);
-                        const int n1 = max(j - lr, 0), n2 = min(j + lr, H - 1);
-                        const int nrow = n2 - n1 + 1, nmid = 2 * (m2 - m1 - 1);
-                        const int q2 = lq - nrow;
-                        const bool left = lq < nrow, mid = !left && q2 < nmid;
-                        const int mm = left ? m1 : (mid ? m1 + 1 + (q2 >> 1) : m2);
-                        const int nn = left ? n1 + lq : (mid ? ((q2 & 1) ? n2 : n1) : n1 + (q2 - nmid));
-                        const int pp = mm + W * nn;
-                        const bool opposite =
-                            sign_lds ? ((int)((sg[pp >> 5] >> (pp & 31)) & 1u) == (q > 0)) : (r[pp] == -q);
-                        const bool present = pr.at(pp) && opposite;
-                        if (mm <= 0 || mm >= W - 1) {
-                            c = (int)((1u << 30) | (unsigned)(mm + W * j));
-                            hit_here = true;
-                        } else if (nn <= 0 || nn >= H - 1) {
-                            c = (int)((2u << 30) | (unsigned)(i + W * nn));
-                            hit_here = true;
-                        } else if (present) {
-                            c = (int)((3u << 30) | (unsigned)pp);
-                            hit_here = true;
-                        }
-                    }
-                    const unsigned long long hit = __ballot(hit_here);
-                    if (hit) {
-                        chosen = __builtin_amdgcn_readlane(c, __ffsll((long long)hit) - 1);
-                        found = true;
-                    }
-                    rc = rr;
-                    off0 = off;
-                }
-                if (!found) continue;  // nothing within reach: the residue stays unbalanced
-            }
-            mych = lane == l ? chosen : mych;
-            done |= bit;
-            // the masks follow the two removed charges (pixels are >= 0; -2 never matches, and
-            // cpix[k] = -1 marks a hit that no commit can remove)
-            const int pix = ((unsigned)chosen >> 30) == 3u ? (chosen & 0x3fffffff) : -2;
-            const unsigned long long el = __ballot(mypm.x == pix);
-            const unsigned long long f0 = __ballot(cpix[0] == pix), f1 = __ballot(cpix[1] == pix);
-            const unsigned long long f2 = __ballot(cpix[2] == pix), f3 = __ballot(cpix[3] == pix);
-            __builtin_amdgcn_sched_barrier(0);
-            live &= ~el;
-            h0 &= ~(e0 | f0);
-            h1 &= ~(e1 | f1);
-            h2 &= ~(e2 | f2);
-            h3 &= ~(e3 | f3);
-        }
-        // the batch's pairs, in commit order, and its charges cleared for the later batches
-        if ((done >> lane) & 1ull) {
-            const int slot = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(done >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((unsigned)done, 0u));
-            out[emitted + slot] = make_int2(mypm.x, mych);
-            pr.clear(mypm.x);
-            if (((unsigned)mych >> 30) == 3u) pr.clear(mych & 0x3fffffff);
-        }
-        if constexpr (!LDSW) __builtin_amdgcn_s_waitcnt(0);
-        emitted += __popcll(done);
+        first_key[e] = (unsigned short)best;
     }
-    if (lane == 0) npairs[blockIdx.x] = emitted;
+    const int off = W * (l - 3) - 3;  // this lane's row around a pixel, from dx = -3
+    const unsigned short* const keys = first_key + (l << 7);
+    // group g starts on row 1 + g (those past the map publish the same, as the first row reads the last group)
+    const int start = (int)min((1ll + slot) * W, (long long)INT_MAX);
+    int* const my_prog = &prog[tid];
+    const int* const above = &prog[(slot + GS_ROWS - 1) % GS_ROWS * GS_LANES];
+    if (tid == 0) nres = 0;
+    __syncthreads();
+    int rho = 0;  // set from the density on the first attempt
+    for (int attempt = 0;; ++attempt) {
+        int mine = 0;
+        for (int w = tid - 1; w < nw + 2; w += NT) {
+            const uint2 b = w >= 0 && w < nw ? charge_bits(r, n, w) : make_uint2(0, 0);
+            ch.w[w] = b.x;
+            ch.w[nw + 3 + w] = b.y;
+            mine += __popc(b.x | b.y);
+        }
+        if (attempt == 0 && mine) atomicAdd(&nres, mine);
+        prog[tid] = start;
+        if (tid == 0) failed = 0;
+        if constexpr (!LDSW) __threadfence();
+        __syncthreads();
+        for (int y = tid; y < H; y += NT) {
+            ch.set_border(y * W);
+            ch.set_border(y * W + W - 1);
+        }
+        for (int x = tid; x < W; x += NT) {
+            ch.set_border(x);
+            ch.set_border((H - 1) * W + x);
+        }
+        if constexpr (!LDSW) __threadfence();
+        __syncthreads();
+        rho = attempt == 0 ? (nres >= 0.25f * n ? 8 : (nres >= 0.1f * n ? 12 : (nres >= 0.05f * n ? 20 : 40)))
+                           : (attempt == 1 ? 4 * rho : R);  // no scan reaches R
+        // Per row in flight (equal in all lanes of its group): the row, its first pixel and the end of its
+        // interior, the pixel it stands on (the first undecided one), whether a charge is expected there and its
+        // sign, the published index and the choices so far. Groups without a row stand still on a valid pixel.
+        int y = 1 + slot;
+        bool active = y <= H - 2 && nres > 0, known = false, qn = false;
+        int row0 = active ? y * W : 0, hi = row0 + W - 1, pos = row0 + 1, pub = start, np = 0;
+        // Every step moves the topmost undecided row on (it waits for nothing), and a group that leaves its
+        // rows publishes GS_LEFT, which the group after it passes on: the loop ends.
+        while (__ballot(active)) {
+            const int v = __hip_atomic_load(above, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if constexpr (!LDSW) __builtin_amdgcn_s_waitcnt(0);  // the index before the charges it covers
+            asm volatile("" ::: "memory");
+            const int wi = pos >> 5;
+            const unsigned a0 = ch.ld(wi), a1 = ch.ld(wi + 1), b0 = ch.ld(nw + 3 + wi), b1 = ch.ld(nw + 4 + wi);
+            // the seven pixels of this lane's row (outside the map: any words, those rings come after a border hit)
+            const int opp = ch.plane(!qn), ring = pos + off;
+            const int wr = opp + max(min(ring >> 5, nw), -1);
+            const unsigned r0 = ch.ld(wr), r1 = ch.ld(wr + 1);
+            asm volatile("" ::: "memory");
+            const unsigned best = group_min(keys[__builtin_amdgcn_alignbit(r1, r0, ring) & 127u]);
+            // the row's charges from pos on (bit b: pixel pos + b)
+            const int nb = min(31, hi - pos);
+            const unsigned neg = __builtin_amdgcn_alignbit(b1, b0, pos);
+            unsigned any = __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(a1, a0, pos) | neg, 0, nb);
+            const bool all = v >= row0;                           // the row above is decided
+            const int lim = all ? INT_MAX - 2 * rho : v + W;      // else: below the pixel under its published index
+            const bool here = active && known && (any & 1u);
+            const int dx = (int)((best >> 4) & 15u) - 8, dy = (int)(best & 15u) - 8;
+            bool decided = here && best != GS_NONE && pos + (int)((best >> 8) & 3u) + rho < lim;
+            int t = pos + dx + (LDSW ? __mul24(W, dy) : W * dy);
+            bool pair = (unsigned)(pos - row0 + dx - 1) < (unsigned)(W - 2) && (unsigned)(y + dy - 1) < (unsigned)(H - 2);
+            // no hit on rings 1-3: the rest of the scan, once every ring up to rho is settled
+            bool far = false;
+            for (unsigned long long slow = __ballot(here && best == GS_NONE && pos + 2 * rho < lim); slow;) {
+                const int f = __builtin_ctzll(slow);
+                slow &= ~(((1ull << GS_LANES) - 1) << (f & ~(GS_LANES - 1)));
+                bool beyond = false;
+                const int sp = __builtin_amdgcn_readlane(pos, f);
+                const int c = gs_scan(ch, H, W, R, sp, sp - __builtin_amdgcn_readlane(row0, f),
+                                      __builtin_amdgcn_readlane(y, f), __builtin_amdgcn_readlane(opp, f), lane, rho,
+                                      beyond);
+                if ((lane ^ f) < GS_LANES) {
+                    t = c;
+                    const int tx = c % W, ty = c / W;
+                    pair = tx > 0 && tx < W - 1 && ty > 0 && ty < H - 1;
+                    decided = !beyond;
+                    far = beyond;
+                }
+            }
+            if (decided) {
+                any &= ~1u;
+                if (t >= 0) {  // else nothing within reach: the residue stays unbalanced
+                    // the residue goes, and the charge it takes; a border point stays
+                    const unsigned dt = (unsigned)(t - pos);
+                    if (pair && dt < 31u) any &= ~(1u << dt);
+                    if (l == 0 || (l == 1 && pair)) {
+                        ch.clear(l ? t : pos, l ? !qn : qn);
+                        out[row0 + np] = make_int2(pos, t);
+                    }
+                    ++np;
+                }
+            }
+            // the next charge, and how far the row is decided
+            known = any != 0;
+            const int nx = known ? __builtin_ctz(any) : nb;
+            qn = (neg >> nx) & 1u;
+            pos += nx;
+            pub = pub == GS_LEFT ? GS_LEFT : max(pub, min(pos, lim - rho - 1));
+            if (active && all && pos >= hi) {
+                pub = row0 + W;
+                if (l == 0) nrow[y] = np;
+                active = y + GS_ROWS <= H - 2;
+                if (active) {
+                    y += GS_ROWS;
+                    row0 = y * W;
+                    hi = row0 + W - 1;
+                    pos = row0 + 1;
+                    known = false;
+                    np = 0;
+                }
+            }
+            if (active && (far || v == GS_LEFT)) {
+                if (far) failed = 1;
+                active = false;
+                pub = GS_LEFT;
+            }
+            if constexpr (!LDSW) __builtin_amdgcn_s_waitcnt(0);  // removals before the index that covers them
+            asm volatile("" ::: "memory");
+            __hip_atomic_store(my_prog, pub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        __syncthreads();
+        if (!failed) break;
+        __syncthreads();  // every wave has read the flag before the next attempt clears it
+    }
+    for (int y = tid; y < H; y += NT)
+        if (nres == 0 || y == 0 || y == H - 1) nrow[y] = 0;
 }
 
-// Phase 3: one thread per chosen cut; cut pixels are only set, so the order does not matter.
-__global__ void k_gs_draw(const int2* __restrict__ pairs, const int* __restrict__ npairs, int H, int W,
+// The chosen cuts: one thread per choice, one grid row per row of the map (cut pixels are only set, so the
+// order does not matter).
+__global__ void k_gs_draw(const int2* __restrict__ pairs, const int* __restrict__ rowpairs, int H, int W,
                           uint8_t* __restrict__ cuts)
 {
     const long long n = (long long)H * W;
-    const long long map = blockIdx.y;
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= npairs[map]) return;
-    const int2 pr = pairs[map * n + k];
+    const long long map = blockIdx.z;
+    const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x), y = blockIdx.y;
+    if (k >= rowpairs[map * H + y]) return;
+    const int2 pr = pairs[map * n + (long long)y * W + k];
     uint8_t* cut = cuts + map * n;
-    const int p = pr.x, kind = (int)((unsigned)pr.y >> 30), t = pr.y & 0x3fffffff;
-    if (kind == 0) {
-        cut[p] = 1;
-        return;
-    }
-    const int r1 = p % W, c1 = p / W, r2 = t % W, c2 = t / W;
+    const int p = pr.x, r1 = p % W, c1 = p / W;
+    // to an opposite charge straight; to a column border along the row, else to a row border along the column
+    int r2 = pr.y % W, c2 = pr.y / W;
+    if (r2 == 0 || r2 == W - 1) c2 = c1;
+    else if (c2 == 0 || c2 == H - 1) r2 = r1;
+    const long long t = r2 + (long long)W * c2;
     cut[p] = 1;
     cut[t] = 1;
     const float dR = (float)(r2 - r1), dC = (float)(c2 - c1);
@@ -849,36 +840,23 @@ void goldstein(Ctx& c, const float* wrapped, int batch, int H, int W, int8_t* re
     int* qa = (int*)c.buf("gs.qa", sizeof(int) * tot);
     int* qb = (int*)c.buf("gs.qb", sizeof(int) * tot);
     const dim3 pgrid((unsigned)((W + 255) / 256), (unsigned)H, (unsigned)batch);  // per-pixel kernels
-    hipLaunchKernelGGL(k_gs_residues, pgrid, dim3(256), 0, c.stream, wrapped, batch, H, W, r);
+    hipLaunchKernelGGL(k_gs_residues, pgrid, dim3(256), 0, c.stream, wrapped, batch, H, W, r, ct);
     const long long nw = (n + 31) / 32, nb = (n + 31) / 32;
     const size_t lds_max = (size_t)(c.max_lds > 0 ? c.max_lds : 64 * 1024);
-    // branch cuts in three phases: candidates in parallel, raster-order commit, drawing
-    const size_t commit_lds = sizeof(unsigned) * (size_t)nw;
-    const int nblk = (int)((n + 1023) / 1024);
-    int* blk = (int*)c.buf("gs.blk", sizeof(int) * (size_t)nblk * batch);
-    int* nres = (int*)c.buf("gs.nres", sizeof(int) * (size_t)batch);
-    int* npairs = (int*)c.buf("gs.npairs", sizeof(int) * (size_t)batch);
-    int2* rec_pm = (int2*)c.buf("gs.recpm", sizeof(int2) * (size_t)tot);
-    int4* rec_c = (int4*)c.buf("gs.recc", sizeof(int4) * (size_t)tot);
+    // branch cuts: the pairs of the raster-order search, then their cuts
+    const size_t words = 2 * ((size_t)nw + 3) * sizeof(unsigned);  // the charges' two bit arrays
+    int* npairs = (int*)c.buf("gs.npairs", sizeof(int) * (size_t)batch * H);
     int2* pairs = (int2*)c.buf("gs.pairs", sizeof(int2) * (size_t)tot);
-    hipLaunchKernelGGL(k_gs_count, dim3((unsigned)(nblk * batch)), dim3(1024), 0, c.stream, r, n, nblk, blk);
-    hipLaunchKernelGGL(k_gs_scan, dim3((batch + 63) / 64), dim3(64), 0, c.stream, blk, nblk, batch, nres);
-    hipLaunchKernelGGL(k_gs_rank, dim3((unsigned)(nblk * batch)), dim3(1024), 0, c.stream, r, H, W, nblk, blk,
-                       rec_pm);
-    hipLaunchKernelGGL(k_gs_cand, dim3((unsigned)(nblk * batch)), dim3(1024), 0, c.stream, r, H, W, nblk, nres,
-                       rec_pm, rec_c);
-    if (commit_lds <= lds_max) {  // presence bits in LDS, and the sign bits beside them when they fit
-        const int sign_lds = 2 * commit_lds <= lds_max;
-        hipLaunchKernelGGL(k_gs_commit<true>, dim3(batch), dim3(64), (sign_lds ? 2 : 1) * commit_lds, c.stream, r,
-                           H, W, nres, rec_pm, rec_c, nullptr, sign_lds, pairs, npairs);
-    } else {  // a map's presence bits exceed LDS: they stay in global memory
-        unsigned* gw = (unsigned*)c.buf("gs.words", sizeof(unsigned) * (size_t)nw * batch);
-        hipLaunchKernelGGL(k_gs_commit<false>, dim3(batch), dim3(64), 0, c.stream, r, H, W, nres, rec_pm, rec_c,
-                           gw, 0, pairs, npairs);
+    if (words + 4096 <= lds_max) {  // beside the kernel's own 3 KiB
+        hipLaunchKernelGGL(k_gs_pair<true>, dim3(batch), dim3(64 * GS_WAVES), words, c.stream, r, H, W, nullptr,
+                           pairs, npairs);
+    } else {
+        unsigned* gw = (unsigned*)c.buf("gs.words", words * batch);
+        hipLaunchKernelGGL(k_gs_pair<false>, dim3(batch), dim3(64 * GS_WAVES), 0, c.stream, r, H, W, gw, pairs,
+                           npairs);
     }
-    hipLaunchKernelGGL(k_gs_fill_u8, dim3(grid1d(tot, 256)), dim3(256), 0, c.stream, ct, tot);
-    hipLaunchKernelGGL(k_gs_draw, dim3((unsigned)((n + 255) / 256), (unsigned)batch), dim3(256), 0, c.stream,
-                       pairs, npairs, H, W, ct);
+    CTDM_CHECK_LAUNCH("k_gs_pair");
+    hipLaunchKernelGGL(k_gs_draw, pgrid, dim3(256), 0, c.stream, pairs, npairs, H, W, ct);
     CTDM_CHECK_LAUNCH("k_gs_draw");
     const size_t bits = sizeof(unsigned) * (size_t)nb;  // cut-or-visited bits
     // the queues get what LDS has left (>= 256 each); their entries pack x and y in 16 bits each
