@@ -17,7 +17,8 @@
 // REFCOMPAT_IDCT reproduces the reference IDCT literally (2N Hermitian completion with the (i+1)
 // twiddle on the right half, DCT_Unwrapping.cu:218-246), which needs a 2N-point transform.
 //
-// Batched path: three kernels per batch
+// Batched path: three kernels per batch, each transforming two real lines as one complex line (line a + i
+// line b; the transform of a real line is conjugate-symmetric, so the two are told apart afterwards)
 //   1. k_uw_rows_fwd: RHS on the fly + DCT-II along x          -> D1[b][y][kx]
 //   2. k_uw_cols:     DCT-II along y, / lambda, DCT-III along y -> D2[b][y][kx]
 //   3. k_uw_rows_inv: DCT-III along x (+ congruence)           -> out[b][y][x]
@@ -26,6 +27,7 @@
 
 #include <cmath>
 #include <mutex>
+#include <tuple>
 
 namespace ctdm {
 
@@ -35,11 +37,20 @@ enum : unsigned { F_SINCOS = CTDM_UNWRAP_SINCOS, F_REF_EIG = CTDM_UNWRAP_REFCOMP
 
 static constexpr float kPI = 3.14159265358979323846f;
 
-// Reference wrap of NumericDerivative1 (DCT_Unwrapping.cu:378-379).
+// Reference wrap of NumericDerivative1 (DCT_Unwrapping.cu:378-379), s = sign(t):
+// t - 2 pi s floor(|pi s + t| / 2 pi). |pi s + t| is u = pi + |t| (0 for t = 0), and floor(u / 2 pi) is 0 below
+// 2 pi and 1 below 4 pi also after rounding (a float below 2 pi k, divided by 2 pi, rounds below k), so
+// differences of less than three half periods, all that wrapped maps have, need no division; the others (and
+// infinities and NaN) take the formula as it stands. Bit-identical to it.
 __device__ __forceinline__ float wrapdiff(float t)
 {
-    const float s = (t > 0.f) ? 1.f : ((t < 0.f) ? -1.f : 0.f);
-    return t - 2.f * kPI * s * floorf(fabsf(kPI * s + t) / (2.f * kPI));
+    const float u = kPI + fabsf(t);
+    float r = u >= 2.f * kPI ? t - copysignf(2.f * kPI, t) : t;
+    if (!(u < 4.f * kPI)) {
+        const float s = (t > 0.f) ? 1.f : ((t < 0.f) ? -1.f : 0.f);
+        r = t - 2.f * kPI * s * floorf(fabsf(kPI * s + t) / (2.f * kPI));
+    }
+    return r;
 }
 
 // RHS at (i, j) of an N x N map.
@@ -62,118 +73,166 @@ __device__ __forceinline__ float rhs_at(const float* __restrict__ p, int N, int 
     return (c1 - c2) + (c3 - c4);
 }
 
-// The same from rows staged in LDS: st holds map rows y0 - 1 .. y0 + G (row r of st is map row y0 - 1 + r;
-// rows outside the map are never read, since the borders take no difference there).
-__device__ __forceinline__ float rhs_staged(const float* st, int N, int i, int j, int y0, bool sincos)
-{
-    const float* row = st + (j - y0 + 1) * N;
-    const float c = row[i];
-    if (sincos) {
-        float r = 0.f;
-        if (i < N - 1) r += sinf(row[i + 1] - c);
-        if (i > 0) r += sinf(row[i - 1] - c);
-        if (j < N - 1) r += sinf(row[i + N] - c);
-        if (j > 0) r += sinf(row[i - N] - c);
-        return r;
-    }
-    const float c1 = (i == N - 1) ? 0.f : wrapdiff(row[i + 1] - c);
-    const float c2 = (i == 0) ? 0.f : wrapdiff(c - row[i - 1]);
-    const float c3 = (j == N - 1) ? 0.f : wrapdiff(row[i + N] - c);
-    const float c4 = (j == 0) ? 0.f : wrapdiff(c - row[i - N]);
-    return (c1 - c2) + (c3 - c4);
-}
-
 // Makhoul source index: position n of v holds x[src(n)].
 __device__ __forceinline__ int mk_src(int n, int N) { return n < N / 2 ? 2 * n : 2 * (N - 1 - n) + 1; }
 
-// ---------------------------------------------------------------- 1. RHS + DCT-II along x
-// mode 0: input is a wrapped map, RHS computed on the fly; mode 1: input used as is (adjoint).
-template <int N, int G>
-__global__ __launch_bounds__(G* Plan<N>::T) void k_uw_rows_fwd(const float* __restrict__ in, int batch,
-                                                              int mode, int sincos,
-                                                              const float2* __restrict__ tw_n,
-                                                              const float2* __restrict__ tw_4n,
-                                                              float* __restrict__ out)
-{
-    constexpr int T = Plan<N>::T;
-    __shared__ float2 lds[G * LdsSize<N>::value];
-    const int g = threadIdx.x / T, t = threadIdx.x % T;
-    const long long row = (long long)blockIdx.x * G + g;
-    const bool valid = row < (long long)batch * N;
-    const long long b = valid ? row / N : 0;
-    const int y = valid ? (int)(row % N) : 0;
-    const float* map = in + b * N * N;
-    float2* s = lds + g * LdsSize<N>::value;
-    auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
-    // When a workgroup's G rows are consecutive rows of one map, those rows and their neighbours above
-    // and below are first staged into the (still unused) LDS area with coalesced float4 loads: the
-    // transform's first stage, which evaluates the right-hand side, reads every input before its first
-    // write into the area, so the staged rows and the transform can share it.
-    constexpr bool STAGE = N % G == 0 && (G + 2) * N <= 2 * G * LdsSize<N>::value && N % 4 == 0;
-    if constexpr (STAGE) {
-        float* st = reinterpret_cast<float*>(lds);
-        const long long row0 = (long long)blockIdx.x * G;
-        const bool wg_valid = row0 < (long long)batch * N;  // N % G == 0: all G rows valid or none
-        const int y0 = (int)(row0 % N);
-        const float* m0 = in + (wg_valid ? row0 / N : 0) * N * N;
-        const int r_lo = y0 == 0 ? 1 : 0, r_hi = (y0 + G == N) ? G : G + 1;  // staged rows r_lo .. r_hi
-        if (wg_valid) {
-            const int nv = (r_hi - r_lo + 1) * (N / 4);
-            const float4* src = reinterpret_cast<const float4*>(m0 + (long long)(y0 - 1 + r_lo) * N);
-            float4* dst = reinterpret_cast<float4*>(st + r_lo * N);
-            for (int e = threadIdx.x; e < nv; e += G * T) dst[e] = src[e];
-        }
-        __syncthreads();
-        auto gl = [&](int n) -> float2 {
-            if (!valid) return make_float2(0.f, 0.f);
-            const int x = mk_src(n, N);
-            return make_float2(mode == 0 ? rhs_staged(st, N, x, y, y0, sincos) : st[(y - y0 + 1) * N + x], 0.f);
-        };
-        Plan<N>::template run<-1>(t, s, tw_n, gl, gs);
-    } else {
-        auto gl = [&](int n) -> float2 {
-            if (!valid) return make_float2(0.f, 0.f);
-            const int x = mk_src(n, N);
-            return make_float2(mode == 0 ? rhs_at(map, N, x, y, sincos) : map[x + N * y], 0.f);
-        };
-        Plan<N>::template run<-1>(t, s, tw_n, gl, gs);
-    }
-    __syncthreads();
-    if (!valid) return;
-    const float s0 = sqrtf(1.f / N), s1 = sqrtf(2.f / N);
-    float* dst = out + row * N;
-    for (int k = t; k < N; k += T) {
-        const float2 V = s[lds_pad(k)];
-        const float2 w = tw_4n[k];  // exp(-i pi k / 2N)
-        dst[k] = (V.x * w.x - V.y * w.y) * (k == 0 ? s0 : s1);
-    }
-}
+// Makhoul position of x[i] in v (the inverse of mk_src).
+__device__ __forceinline__ int mk_pos(int i, int N) { return i & 1 ? N - 1 - (i >> 1) : i >> 1; }
 
-// DCT-III of one line held as real coefficients `X` (LDS, N floats) into `s`, final values handed to
-// put(n, value). refcompat selects the reference's literal 2N construction (requires LdsSize<2N>).
-template <int N, int DIR_UNUSED = 0>
-struct Dct3 {
-    template <class Put>
-    __device__ __forceinline__ static void exact(int t, const float* X, float2* s, const float2* tw_n,
-                                                 const float2* tw_4n, Put& put)
+// Transform and workgroup of a pair of lines of length N: T threads per pair with a radix plan of their own,
+// GP row pairs or CP column pairs per workgroup. More threads per line than Plan<N> has, so that a thread's share
+// is short (4 or 8 points): these kernels wait for memory and for their own chains far more than they compute,
+// and the workgroups are small so that a few maps still spread over the chip (24 maps of 192^2: right-hand side
+// and first transform 13.1 us, with Plan<192>'s 16 threads 17.5 us; 45 of 128^2: 8.1 against 11.8 us).
+template <int N, int T_, int GP_, int... R>
+struct PairOf {
+    static constexpr int T = T_, GP = GP_, CP = 8;
+    static constexpr int NT = T * GP, NC = T * CP;       // threads of a row / column workgroup
+    static constexpr int R0 = std::get<0>(std::make_tuple(R...)), J = N / T;
+    static_assert(N / R0 == T, "the first stage's elements of thread t are t + r T");
+    template <int DIR, class TW, class GL, class GS>
+    __device__ __forceinline__ static void run(int t, float2* s, const TW& tw, GL& gl, GS& gs)
     {
-        // 1 / sqrt(1/N) and 1 / sqrt(2/N) (compile-time constants): the un-normalisation multiplies
-        const float r0 = 1.f / sqrtf(1.f / N), r1 = 1.f / sqrtf(2.f / N);
-        auto gl = [&](int k) -> float2 {
-            const float ck = X[k] * (k == 0 ? r0 : r1);
-            const float cn = (k == 0) ? 0.f : X[N - k] * r1;
-            const float2 w = tw_4n[k];  // exp(-i pi k/2N); we need exp(+i pi k/2N) = conj
-            // (ck - i cn) * (w.x - i w.y)
-            return make_float2(ck * w.x - cn * w.y, -ck * w.y - cn * w.x);
-        };
-        const float inv = 1.f / N;
-        auto gs = [&](int n, float2 v) {
-            const int x = mk_src(n, N);
-            put(x, v.x * inv);
-        };
-        Plan<N>::template run<+1>(t, s, tw_n, gl, gs);
+        Stockham<N, T, DIR, 1, R...>::run(t, s, tw, gl, gs);
     }
 };
+template <int N>
+struct Pair;
+template <>
+struct Pair<32> : PairOf<32, 8, 8, 4, 8> {};
+template <>
+struct Pair<64> : PairOf<64, 16, 4, 4, 4, 4> {};
+template <>
+struct Pair<128> : PairOf<128, 32, 8, 4, 4, 8> {};
+template <>
+struct Pair<192> : PairOf<192, 24, 8, 8, 8, 3> {};
+template <>
+struct Pair<256> : PairOf<256, 32, 8, 8, 8, 4> {};
+
+// The DCT-II coefficients k of two lines a, b from Z = FFT(v_a + i v_b): V_a = (Z[k] + conj Z[-k]) / 2,
+// V_b = (Z[k] - conj Z[-k]) / 2i, X = s Re(w V) with w = exp(-i pi k / 2N).
+template <int N>
+__device__ __forceinline__ float2 dct2_pair(const float2* s, int k, float2 w)
+{
+    const float2 z = s[lds_pad(k)], m = s[lds_pad(k == 0 ? 0 : N - k)];
+    const float sc = 0.5f * (k == 0 ? sqrtf(1.f / N) : sqrtf(2.f / N));
+    const float ax = z.x + m.x, ay = z.y - m.y, bx = z.y + m.y, by = m.x - z.x;
+    return make_float2((ax * w.x - ay * w.y) * sc, (bx * w.x - by * w.y) * sc);
+}
+
+// Element k of the DCT-III's transform input of two lines whose coefficients c = (a, b) stand in s:
+// V_a + i V_b with V = exp(i pi k / 2N) (C_k - i C_{N-k}), C = X / s, C_N = 0.
+template <int N>
+__device__ __forceinline__ float2 dct3_pair(const float2* s, int k, float2 w)
+{
+    const float r0 = 1.f / sqrtf(1.f / N), r1 = 1.f / sqrtf(2.f / N);
+    const float2 c = cscale(s[lds_pad(k)], k == 0 ? r0 : r1);
+    const float2 n = k == 0 ? make_float2(0.f, 0.f) : cscale(s[lds_pad(N - k)], r1);
+    // (c - i n) (w.x - i w.y) for each line
+    const float ar = c.x * w.x - n.x * w.y, ai = -c.x * w.y - n.x * w.x;
+    const float br = c.y * w.x - n.y * w.y, bi = -c.y * w.y - n.y * w.x;
+    return make_float2(ar - bi, ai + br);
+}
+
+// ---------------------------------------------------------------- 1. RHS + DCT-II along x
+enum : int { RHS_WRAP = 0, RHS_SIN = 1, RHS_NONE = 2 };  // RHS of a wrapped map, or the input as it is (adjoint)
+
+// A workgroup's 2 GP rows lie in one map. First each thread forms the right-hand side of blocks of 4 x 4 or 4 x 2 pixels
+// straight from the map (every difference within the block once: 2.5 or 2.75 per pixel instead of the 4 of the
+// stencil) and puts two rows of it as one complex line in Makhoul order; then the lines
+// are transformed. Bound by the chain load - differences - transform of one round of workgroups. 60 maps of
+// 256^2: 13.4 us, one map 7.3 us; 26.2 and 15.4 us when each thread evaluated the whole stencil for the 16 pixels
+// of its transform, with a division in each difference, in 80 KiB of unrolled code.
+template <int N, int RHS>
+__global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_fwd(const float* __restrict__ in,
+                                                            const float2* __restrict__ tw_n,
+                                                            const float2* __restrict__ tw_4n, float* __restrict__ out)
+{
+    using PR = Pair<N>;
+    constexpr int T = PR::T, GP = PR::GP, NT = PR::NT, GR = 2 * GP, Q = N / 4;
+    constexpr int CR = Q * GR / 4 >= NT ? 4 : 2;  // rows of a thread's block
+    static_assert(N % GR == 0 && GR % CR == 0, "a workgroup's rows lie in one map");
+    __shared__ float2 lds[GP * LdsSize<N>::value];
+    __shared__ float2 twl[LdsSize<N>::value];
+    TwStager<N, NT> tws;
+    tws.fetch(tw_n);
+    const int g = threadIdx.x / T, t = threadIdx.x % T;
+    const long long row0 = (long long)blockIdx.x * GR;
+    const int y0 = (int)(row0 % N);
+    const float* map = in + (row0 - y0) * N;
+    float2 w[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) w[j] = tw_4n[t + j * T];
+    for (int e = threadIdx.x; e < Q * (GR / CR); e += NT) {
+        const int x = 4 * (e % Q), r = CR * (e / Q), y = y0 + r;
+        const float* p = map + (long long)y * N + x;
+        float v[CR + 2][4], l[CR], rt[CR];  // rows y - 1 .. y + CR and the pixels beside the block
+#pragma unroll
+        for (int k = 0; k < CR + 2; ++k) {
+            if (RHS == RHS_NONE && (k == 0 || k == CR + 1)) continue;
+            // rows and columns past the map are not used: the border rows and columns stand in for them
+            const int yy = min(max(y + k - 1, 0), N - 1);
+            const float4 q = *reinterpret_cast<const float4*>(map + (long long)yy * N + x);
+            v[k][0] = q.x;
+            v[k][1] = q.y;
+            v[k][2] = q.z;
+            v[k][3] = q.w;
+        }
+        float rho[CR][4];
+        if constexpr (RHS == RHS_NONE) {
+#pragma unroll
+            for (int k = 0; k < CR; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) rho[k][i] = v[k + 1][i];
+        } else {
+#pragma unroll
+            for (int k = 0; k < CR; ++k) {
+                l[k] = p[k * N - (x > 0)];
+                rt[k] = p[k * N + (x + 4 < N ? 4 : 3)];
+            }
+            auto step = [](float d) { return RHS == RHS_SIN ? sinf(d) : wrapdiff(d); };
+            float up[4];  // differences to the row above
+#pragma unroll
+            for (int i = 0; i < 4; ++i) up[i] = y == 0 ? 0.f : step(v[1][i] - v[0][i]);
+#pragma unroll
+            for (int k = 0; k < CR; ++k) {
+                const float* c = v[k + 1];
+                float left = x == 0 ? 0.f : step(c[0] - l[k]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float nx = i < 3 ? c[i < 3 ? i + 1 : 3] : rt[k];
+                    const float right = i == 3 && x + 4 == N ? 0.f : step(nx - c[i]);
+                    const float down = k == CR - 1 && y + CR == N ? 0.f : step(v[k + 2][i] - c[i]);
+                    rho[k][i] = RHS == RHS_SIN ? ((right - left) + down) - up[i] : (right - left) + (down - up[i]);
+                    left = right;
+                    up[i] = down;
+                }
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < CR / 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                lds[(r / 2 + h) * LdsSize<N>::value + lds_pad(mk_pos(x + i, N))] =
+                    make_float2(rho[2 * h][i], rho[2 * h + 1][i]);
+    }
+    tws.put(twl);
+    const TwPad twp{twl};
+    __syncthreads();
+    float2* s = lds + g * LdsSize<N>::value;
+    auto gl = [&](int n) -> float2 { return s[lds_pad(n)]; };
+    auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
+    PR::template run<-1>(t, s, twp, gl, gs);
+    __syncthreads();
+    float* dst = out + (row0 + 2 * g) * N;
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) {
+        const int k = t + j * T;
+        const float2 X = dct2_pair<N>(s, k, w[j]);
+        dst[k] = X.x;
+        dst[N + k] = X.y;
+    }
+}
 
 // Reference IDCT of one line (countIDCT + inverse 2N FFT + cufft2float), dTemp = 1/sqrt(2N).
 template <int N, class Put>
@@ -201,21 +260,89 @@ __device__ __forceinline__ void idct_refcompat(int t, const float* X, float2* s,
 }
 
 // ---------------------------------------------------------------- 2. columns: DCT-II, / lambda, DCT-III
-// LDS per column: one complex area (LdsSize<LN>). The N real coefficients between the two transforms
-// are held in registers while the area is read, then written into it as floats: the DCT-III reads them
-// only in its first stage, before its first write to the area. One area per column keeps 60 maps of
-// 256 columns within one round of workgroups.
-template <int N, int C, int LN>
-__global__ __launch_bounds__(C* Plan<LN>::T) void k_uw_cols(const float* __restrict__ in, int batch,
-                                                            unsigned flags, const double* __restrict__ eig,
-                                                            const float2* __restrict__ tw_n,
-                                                            const float2* __restrict__ tw_2n,
-                                                            const float2* __restrict__ tw_4n,
-                                                            float* __restrict__ out)
+// C pairs of neighbouring columns per workgroup, one float2 per row of a pair (C * 8 bytes of a row side by
+// side). 60 maps of 256^2: 14.7 us (22.8 with one real column per transform), one map 7.1 us (9.5). The coefficient pairs between the two transforms are held in registers while the area is read, then
+// written into it: the DCT-III reads them before its first write. For the adjoint: `num`, the exact sin^2 table,
+// also multiplies by the stencil's own eigenvalue (the Laplacian of the solution, without the stencil), and
+// `dc` receives each map's mean.
+template <int N>
+__global__ __launch_bounds__(Pair<N>::NC) void k_uw_cols(const float2* __restrict__ in, unsigned flags,
+                                                        const double* __restrict__ eig,
+                                                        const float2* __restrict__ tw_n,
+                                                        const float2* __restrict__ tw_4n, float2* __restrict__ out,
+                                                        const double* __restrict__ num, float* __restrict__ dc)
 {
-    constexpr int TL = Plan<LN>::T;  // threads per column (sized for the longest transform used)
+    using PR = Pair<N>;
+    constexpr int T = PR::T, C = PR::CP, H = N / 2;
+    constexpr int LS = LdsStride<N, C>::value;
+    __shared__ float2 lds[C * LS];
+    __shared__ float2 twl[LdsSize<N>::value];
+    TwStager<N, PR::NC> tws;
+    tws.fetch(tw_n);
+    const int cidx = threadIdx.x % C, t = threadIdx.x / C;
+    constexpr int tiles = H / C;
+    const long long b = blockIdx.x / tiles;
+    const int c = (blockIdx.x % tiles) * C + cidx;  // columns 2c and 2c + 1
+    const float2* col = in + b * N * H + c;
+    float2* s = lds + cidx * LS;
+    StageRegs<N, T, PR::R0> x;
+#pragma unroll
+    for (int r = 0; r < PR::R0; ++r) x.v[0][r] = col[mk_src(t + r * T, N) * H];
+    float2 w[PR::J];
+    double ey[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) {
+        w[j] = tw_4n[t + j * T];
+        ey[j] = eig[t + j * T];
+    }
+    const double e0 = eig[2 * c], e1 = eig[2 * c + 1];
+    __builtin_amdgcn_sched_barrier(0);  // every load is under way before the first wait
+    tws.put(twl);
+    const TwPad twp{twl};
+    auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
+    PR::template run<-1>(t, s, twp, x, gs);
+    __syncthreads();
+    const bool refeig = flags & F_REF_EIG;
+    float2 xv[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) {
+        const int ky = t + j * T;
+        const float2 X = dct2_pair<N>(s, ky, w[j]);
+        const double l0 = refeig ? e0 + ey[j] - 4.0 : -4.0 * (e0 + ey[j]);
+        const double l1 = refeig ? e1 + ey[j] - 4.0 : -4.0 * (e1 + ey[j]);
+        // X / lambda as a product with the hardware reciprocal (v_rcp_f32, about 1 ulp) of the eigenvalue sum
+        // formed in double: two ulps at most, in place of a double division
+        xv[j].x = c == 0 && ky == 0 ? 0.f : X.x * __builtin_amdgcn_rcpf((float)l0);
+        xv[j].y = X.y * __builtin_amdgcn_rcpf((float)l1);
+        if (num) {
+            const double n = num[ky];
+            xv[j].x *= (float)(-4.0 * (num[2 * c] + n));
+            xv[j].y *= (float)(-4.0 * (num[2 * c + 1] + n));
+        }
+        if (dc && c == 0 && ky == 0) dc[b] = X.x * (1.f / N);
+    }
+    __syncthreads();  // every read of the transform's output precedes the coefficients' writes
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) s[lds_pad(t + j * T)] = xv[j];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
+    float2* dcol = out + b * N * H + c;
+    auto gs2 = [&](int n, float2 v) { dcol[mk_src(n, N) * H] = cscale(v, 1.f / N); };
+    PR::template run<+1>(t, s, twp, x, gs2);
+}
+
+// The same for one column per transform with the reference's 2N-point IDCT.
+template <int N, int C>
+__global__ __launch_bounds__(C* Plan<2 * N>::T) void k_uw_cols_ref(const float* __restrict__ in, unsigned flags,
+                                                                  const double* __restrict__ eig,
+                                                                  const float2* __restrict__ tw_n,
+                                                                  const float2* __restrict__ tw_2n,
+                                                                  const float2* __restrict__ tw_4n,
+                                                                  float* __restrict__ out)
+{
+    constexpr int LN = 2 * N, TL = Plan<LN>::T;  // threads per column (sized for the longer transform)
     constexpr int LS = LdsStride<LN, C>::value;
-    static_assert(2 * LdsSize<LN>::value >= N, "coefficients must fit the complex area");
     constexpr int J = (N + TL - 1) / TL;  // coefficients per thread
     __shared__ float2 lds[C * LS];
     const int cidx = threadIdx.x % C, t = threadIdx.x / C;
@@ -239,13 +366,7 @@ __global__ __launch_bounds__(C* Plan<LN>::T) void k_uw_cols(const float* __restr
             const float2 V = s[lds_pad(ky)];
             const float2 w = tw_4n[ky];
             const float Xv = (V.x * w.x - V.y * w.y) * (ky == 0 ? s0 : s1);
-            double lam;
-            if (refeig)
-                lam = eig[kx] + eig[ky] - 4.0;
-            else
-                lam = -4.0 * (eig[kx] + eig[ky]);
-            // Xv / lambda as a product with the hardware reciprocal (v_rcp_f32, about 1 ulp) of the
-            // eigenvalue sum formed in double: two ulps at most, in place of a double division
+            const double lam = refeig ? eig[kx] + eig[ky] - 4.0 : -4.0 * (eig[kx] + eig[ky]);
             xv[j] = (kx == 0 && ky == 0) ? 0.f : Xv * __builtin_amdgcn_rcpf((float)lam);
         }
     }
@@ -258,113 +379,225 @@ __global__ __launch_bounds__(C* Plan<LN>::T) void k_uw_cols(const float* __restr
     __syncthreads();
     float* dcol = out + b * N * N + kx;
     auto put = [&](int y, float v) { dcol[(long long)y * N] = v; };
-    if (flags & F_REF_IDCT) {
-        if constexpr (LN == 2 * N) idct_refcompat<N>(t, X, s, tw_2n, tw_4n, put);
-    } else {
-        Dct3<N>::exact(t, X, s, tw_n, tw_4n, put);
-    }
+    idct_refcompat<N>(t, X, s, tw_2n, tw_4n, put);
 }
 
 // ---------------------------------------------------------------- 3. rows: DCT-III along x
-template <int N, int G, int LN>
-__global__ __launch_bounds__(G* Plan<LN>::T) void k_uw_rows_inv(const float* __restrict__ in, int batch,
-                                                                unsigned flags,
-                                                                const float* __restrict__ wrapped,
-                                                                const float2* __restrict__ tw_n,
-                                                                const float2* __restrict__ tw_2n,
-                                                                const float2* __restrict__ tw_4n,
-                                                                float* __restrict__ out)
+// Congruence: the value of the class w + 2 pi Z nearest to v.
+__device__ __forceinline__ float congruent(float v, float w) { return w + 2.f * kPI * rintf((v - w) / (2.f * kPI)); }
+
+// Coefficients of a workgroup's 2 GP rows (two neighbouring rows per pair) into its LDS areas.
+template <int N>
+__device__ __forceinline__ void load_row_pairs(const float* __restrict__ rows, float2* lds, int ls)
 {
-    constexpr int TL = Plan<LN>::T;
+    constexpr int Q = N / 4, E = Q * Pair<N>::GP;
+    for (int e = threadIdx.x; e < E; e += Pair<N>::NT) {
+        const int g = e / Q, x = 4 * (e % Q);
+        const float4 a = *reinterpret_cast<const float4*>(rows + 2 * g * N + x);
+        const float4 b = *reinterpret_cast<const float4*>(rows + (2 * g + 1) * N + x);
+        float2* s = lds + g * ls;
+        s[lds_pad(x)] = make_float2(a.x, b.x);
+        s[lds_pad(x + 1)] = make_float2(a.y, b.y);
+        s[lds_pad(x + 2)] = make_float2(a.z, b.z);
+        s[lds_pad(x + 3)] = make_float2(a.w, b.w);
+    }
+}
+
+template <int N>
+__global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_inv(const float* __restrict__ in, const float* __restrict__ wrapped,
+                                                            const float2* __restrict__ tw_n,
+                                                            const float2* __restrict__ tw_4n, float* __restrict__ out)
+{
+    using PR = Pair<N>;
+    constexpr int T = PR::T, GP = PR::GP, Q = N / 4, LS = LdsSize<N>::value;
+    __shared__ float2 lds[GP * LS];
+    __shared__ float2 twl[LS];
+    TwStager<N, PR::NT> tws;
+    tws.fetch(tw_n);
+    const int g = threadIdx.x / T, t = threadIdx.x % T;
+    const long long base = (long long)blockIdx.x * 2 * GP * N;
+    float2 w[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) w[j] = tw_4n[t + j * T];
+    load_row_pairs<N>(in + base, lds, LS);
+    tws.put(twl);
+    const TwPad twp{twl};
+    __syncthreads();
+    float2* s = lds + g * LS;
+    StageRegs<N, T, PR::R0> x;
+#pragma unroll
+    for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
+    auto gs = [&](int n, float2 v) { s[lds_pad(mk_src(n, N))] = cscale(v, 1.f / N); };
+    PR::template run<+1>(t, s, twp, x, gs);
+    __syncthreads();
+    for (int e = threadIdx.x; e < Q * GP; e += PR::NT) {
+        const int gg = e / Q, c = 4 * (e % Q);
+        const float2* p = lds + gg * LS;
+        const float2 v0 = p[lds_pad(c)], v1 = p[lds_pad(c + 1)], v2 = p[lds_pad(c + 2)], v3 = p[lds_pad(c + 3)];
+        const long long o = base + 2 * gg * N + c;
+        float4 a = make_float4(v0.x, v1.x, v2.x, v3.x), b = make_float4(v0.y, v1.y, v2.y, v3.y);
+        if (wrapped) {
+            const float4 wa = *reinterpret_cast<const float4*>(wrapped + o);
+            const float4 wb = *reinterpret_cast<const float4*>(wrapped + o + N);
+            a = make_float4(congruent(a.x, wa.x), congruent(a.y, wa.y), congruent(a.z, wa.z), congruent(a.w, wa.w));
+            b = make_float4(congruent(b.x, wb.x), congruent(b.y, wb.y), congruent(b.z, wb.z), congruent(b.w, wb.w));
+        }
+        *reinterpret_cast<float4*>(out + o) = a;
+        *reinterpret_cast<float4*>(out + o + N) = b;
+    }
+}
+
+// The same for one row per transform with the reference's 2N-point IDCT.
+template <int N, int G>
+__global__ __launch_bounds__(G* Plan<2 * N>::T) void k_uw_rows_inv_ref(const float* __restrict__ in, int batch,
+                                                                      const float* __restrict__ wrapped,
+                                                                      const float2* __restrict__ tw_2n,
+                                                                      const float2* __restrict__ tw_4n,
+                                                                      float* __restrict__ out)
+{
+    constexpr int LN = 2 * N, TL = Plan<LN>::T;
     __shared__ float2 lds[G * LdsSize<LN>::value];
     const int g = threadIdx.x / TL, t = threadIdx.x % TL;
     const long long row = (long long)blockIdx.x * G + g;
     const bool valid = row < (long long)batch * N;
     const long long r = valid ? row : 0;
-    float2* s = lds + g * LdsSize<LN>::value;
-    // The DCT-III's first stage reads coefficients k and N - k of the row straight from the input (the
-    // row's 1 KiB stays in cache); no LDS copy, so 60 maps of 256 rows fit one round of workgroups.
-    const float* X = in + r * N;
-    const bool cong = (flags & F_CONGRUENT) && wrapped;
     auto put = [&](int x, float v) {
-        if (!valid) return;
-        if (cong) {
-            const float w = wrapped[r * N + x];
-            v = w + 2.f * kPI * rintf((v - w) / (2.f * kPI));
-        }
-        out[r * N + x] = v;
+        if (valid) out[r * N + x] = wrapped ? congruent(v, wrapped[r * N + x]) : v;
     };
-    if (flags & F_REF_IDCT) {
-        if constexpr (LN == 2 * N) idct_refcompat<N>(t, X, s, tw_2n, tw_4n, put);
-    } else {
-        Dct3<N>::exact(t, X, s, tw_n, tw_4n, put);
-    }
+    idct_refcompat<N>(t, in + r * N, lds + g * LdsSize<LN>::value, tw_2n, tw_4n, put);
 }
 
 // Rows of the last unwrapping pass fused with the row pass of the Rytov spectrum (k_rytov_rows of the
-// reconstruction module, same transform and twiddles): each row's DCT-III result, after the congruence
-// step, goes to the unwrapped map (when wanted) and stays in the row's LDS area as floats (the DCT-III's
-// last stage writes only after its barrier), where the forward row transform of u = logamp + i phi
-// reads it. Row spectra: P[r][k].
-template <int N, int G>
-__global__ __launch_bounds__(G* Plan<N>::T) void k_uw_rows_inv_rytov(const float* __restrict__ in, int batch,
-                                                                      unsigned flags,
-                                                                      const float* __restrict__ wrapped,
-                                                                      const float* __restrict__ la,
-                                                                      const float2* __restrict__ tw_n,
-                                                                      const float2* __restrict__ tw_4n,
-                                                                      float* __restrict__ out,
-                                                                      float2* __restrict__ P)
+// reconstruction module, same transform and twiddles): the DCT-III's two rows, after the congruence step, go to
+// the unwrapped map (when wanted) and stay in LDS as floats, one row in each of the pair's two areas (the
+// DCT-III's last stage writes only after its barrier), where the forward row transforms of u = logamp + i phi
+// read them. Row spectra: P[r][k].
+template <int N>
+__global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_inv_rytov(const float* __restrict__ in,
+                                                                  const float* __restrict__ wrapped,
+                                                                  const float* __restrict__ la,
+                                                                  const float2* __restrict__ tw_n,
+                                                                  const float2* __restrict__ tw_4n,
+                                                                  float* __restrict__ out, float2* __restrict__ P)
 {
-    constexpr int TL = Plan<N>::T;
-    static_assert(2 * LdsSize<N>::value >= N, "the phase row must fit the complex area");
-    __shared__ float2 lds[G * LdsSize<N>::value];
-    const int g = threadIdx.x / TL, t = threadIdx.x % TL;
-    const long long row = (long long)blockIdx.x * G + g;
-    const bool valid = row < (long long)batch * N;
-    const long long r = valid ? row : 0;
-    float2* s = lds + g * LdsSize<N>::value;
-    float* ph = reinterpret_cast<float*>(s);
-    const float* X = in + r * N;
-    const bool cong = (flags & F_CONGRUENT) && wrapped;
-    auto put = [&](int x, float v) {
-        if (cong) {
-            const float w = wrapped[r * N + x];
-            v = w + 2.f * kPI * rintf((v - w) / (2.f * kPI));
-        }
-        ph[x] = v;
-        if (valid && out) out[r * N + x] = v;
-    };
-    Dct3<N>::exact(t, X, s, tw_n, tw_4n, put);
+    using PR = Pair<N>;
+    constexpr int T = PR::T, GP = PR::GP, LS = LdsSize<N>::value;
+    __shared__ float2 lds[2 * GP * LS];
+    const int g = threadIdx.x / T, t = threadIdx.x % T;
+    const long long base = (long long)blockIdx.x * 2 * GP * N;
+    float2 w[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) w[j] = tw_4n[t + j * T];
+    load_row_pairs<N>(in + base, lds, 2 * LS);
     __syncthreads();
-    auto gl = [&](int x) -> float2 { return make_float2(la[r * N + x], ph[x]); };
-    auto gs = [&](int k, float2 v) {
-        if (valid) P[r * N + k] = v;
+    float2* s = lds + g * 2 * LS;
+    StageRegs<N, T, PR::R0> x;
+#pragma unroll
+    for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
+    const long long ra = base + 2 * g * N;
+    float* pa = reinterpret_cast<float*>(s);
+    float* pb = reinterpret_cast<float*>(s + LS);
+    auto gs = [&](int n, float2 v) {
+        const int c = mk_src(n, N);
+        float a = v.x * (1.f / N), b = v.y * (1.f / N);
+        if (wrapped) {
+            a = congruent(a, wrapped[ra + c]);
+            b = congruent(b, wrapped[ra + N + c]);
+        }
+        pa[c] = a;
+        pb[c] = b;
+        if (out) {
+            out[ra + c] = a;
+            out[ra + N + c] = b;
+        }
     };
-    Plan<N>::template run<-1>(t, s, tw_n, gl, gs);
+    PR::template run<+1>(t, s, tw_n, x, gs);
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const float* ph = h ? pb : pa;
+        const float* l = la + ra + h * N;
+        float2* dst = P + ra + h * N;
+        auto gl = [&](int c) -> float2 { return make_float2(l[c], ph[c]); };
+        auto gs2 = [&](int k, float2 v) { dst[k] = v; };
+        PR::template run<-1>(t, s + h * LS, tw_n, gl, gs2);
+    }
 }
 
-// Adjoint helper: (weighted) zero-flux Laplacian, g_in = sum_nbr w_pn (v_n - v_p); weights
-// cos(phi_n - phi_p) for SINCOS, 1 otherwise.
-__global__ void k_uw_stencil(const float* __restrict__ v, const float* __restrict__ phi, int batch,
-                             int N, int sincos, float* __restrict__ out)
+// Adjoint of the right-hand side at a solution v = P g: the zero-flux stencil sum_nbr w_pn (v_n - v_p) with
+// weights cos(phi_n - phi_p). With `g` and `mean` (P exact) the unweighted part is known, as the stencil undoes
+// P up to the mean, and only sum (cos - 1) (v_n - v_p) is taken from v: v is smooth and large where g is rough,
+// so its differences carry its rounding, here times 1 - cos. Four pixels of a row per thread.
+__global__ __launch_bounds__(256) void k_uw_stencil(const float* __restrict__ v, const float* __restrict__ phi, int N,
+                                                    long long quads, const float* g, const float* __restrict__ mean,
+                                                    float* out)  // out may be g
 {
-    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (long long)batch * N * N) return;
-    const long long b = g / ((long long)N * N);
-    const int k = (int)(g % ((long long)N * N)), i = k % N, j = k / N;
-    const float* vv = v + b * N * N;
-    const float* pp = phi + b * N * N;
-    float acc = 0.f;
-    auto term = [&](int kn) {
-        const float w = sincos ? cosf(pp[kn] - pp[k]) : 1.f;
-        acc += w * (vv[kn] - vv[k]);
+    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= quads) return;
+    const int Q = N / 4;
+    const long long row = e / Q, b = row / N;
+    const int x = 4 * (int)(e - row * Q), y = (int)(row - b * N);
+    const long long o = row * N + x;
+    auto quad = [&](const float* m, long long k, float (&q)[4]) {
+        const float4 f = *reinterpret_cast<const float4*>(m + k);
+        q[0] = f.x;
+        q[1] = f.y;
+        q[2] = f.z;
+        q[3] = f.w;
     };
-    if (i < N - 1) term(k + 1);
-    if (i > 0) term(k - 1);
-    if (j < N - 1) term(k + N);
-    if (j > 0) term(k - N);
-    out[g] = acc;
+    // past the border a pixel stands in for its neighbour: no difference, whatever the weight
+    const long long ou = o - (y > 0 ? N : 0), od = o + (y < N - 1 ? N : 0);
+    float vc[4], vu[4], vd[4], pc[4], pu[4], pd[4];
+    quad(v, o, vc);
+    quad(v, ou, vu);
+    quad(v, od, vd);
+    quad(phi, o, pc);
+    quad(phi, ou, pu);
+    quad(phi, od, pd);
+    const long long ol = o - (x > 0), orr = o + (x + 4 < N ? 4 : 3);
+    const float one = g ? 1.f : 0.f;
+    auto flux = [&](float dp, float dv) { return (cosf(dp) - one) * dv; };
+    float left = flux(pc[0] - phi[ol], vc[0] - v[ol]);  // flux from the left neighbour into pixel 0
+    float r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float pn = i < 3 ? pc[i < 3 ? i + 1 : 3] : phi[orr], vn = i < 3 ? vc[i < 3 ? i + 1 : 3] : v[orr];
+        const float right = flux(pn - pc[i], vn - vc[i]);
+        r[i] = ((right - left) + flux(pd[i] - pc[i], vd[i] - vc[i])) + flux(pu[i] - pc[i], vu[i] - vc[i]);
+        left = right;
+    }
+    if (g) {
+        const float m = mean[b];
+        float gc[4];
+        quad(g, o, gc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] += gc[i] - m;
+    }
+    *reinterpret_cast<float4*>(out + o) = make_float4(r[0], r[1], r[2], r[3]);
+}
+
+// Each map minus its mean (the sums in double), one workgroup per map of n values.
+__global__ __launch_bounds__(1024) void k_uw_sub_mean(const float* in, float* out, int n)  // out may be in
+{
+    __shared__ double red[16];
+    const float* m = in + (size_t)blockIdx.x * n;
+    float* o = out + (size_t)blockIdx.x * n;
+    double sum = 0.0;
+    for (int i = 4 * threadIdx.x; i < n; i += 4096) {
+        const float4 f = *reinterpret_cast<const float4*>(m + i);
+        sum += ((double)f.x + f.y) + ((double)f.z + f.w);
+    }
+    for (int w = 32; w > 0; w >>= 1) sum += __shfl_xor(sum, w);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    double tot = 0.0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) tot += red[w];
+    const float mean = (float)(tot / n);
+    for (int i = 4 * threadIdx.x; i < n; i += 4096) {
+        const float4 f = *reinterpret_cast<const float4*>(m + i);
+        *reinterpret_cast<float4*>(o + i) = make_float4(f.x - mean, f.y - mean, f.z - mean, f.w - mean);
+    }
 }
 
 // ---------------------------------------------------------------- FastUnwrapping's map conventions
@@ -437,35 +670,53 @@ static const double* eig_table(Ctx& c, int N, bool refcompat, bool existing = fa
     return d;
 }
 
-template <int N, int LN>
-static void run_cols(Ctx& c, const float* in, int batch, unsigned flags, float* out, bool existing)
+template <int N>
+static void run_rows_fwd(Ctx& c, const float* in, int batch, int rhs, float* out)
 {
-    constexpr int C = (256 / Plan<LN>::T) < N ? (256 / Plan<LN>::T) : N;
-    const double* eig = eig_table(c, N, flags & F_REF_EIG, existing);
-    const float2* tw2 = (LN == 2 * N) ? c.tw(2 * N) : c.tw(N);
-    hipLaunchKernelGGL((k_uw_cols<N, C, LN>), dim3(batch * (N / C)), dim3(C * Plan<LN>::T), 0, c.stream,
-                       in, batch, flags, eig, c.tw(N), tw2, c.tw(4 * N), out);
-    CTDM_CHECK_LAUNCH("k_uw_cols");
-}
-
-template <int N, int LN>
-static void run_rows_inv(Ctx& c, const float* in, int batch, unsigned flags, const float* wrapped,
-                         float* out)
-{
-    constexpr int G = 256 / Plan<LN>::T;
-    const float2* tw2 = (LN == 2 * N) ? c.tw(2 * N) : c.tw(N);
-    hipLaunchKernelGGL((k_uw_rows_inv<N, G, LN>), dim3(grid1d((long long)batch * N, G)), dim3(G * Plan<LN>::T),
-                       0, c.stream, in, batch, flags, wrapped, c.tw(N), tw2, c.tw(4 * N), out);
-    CTDM_CHECK_LAUNCH("k_uw_rows_inv");
+    using PR = Pair<N>;
+    const dim3 grid((unsigned)((long long)batch * N / (2 * PR::GP))), block(PR::NT);
+    const float2 *tw = c.tw(N), *tw4 = c.tw(4 * N);
+    if (rhs == RHS_WRAP)
+        hipLaunchKernelGGL((k_uw_rows_fwd<N, RHS_WRAP>), grid, block, 0, c.stream, in, tw, tw4, out);
+    else if (rhs == RHS_SIN)
+        hipLaunchKernelGGL((k_uw_rows_fwd<N, RHS_SIN>), grid, block, 0, c.stream, in, tw, tw4, out);
+    else
+        hipLaunchKernelGGL((k_uw_rows_fwd<N, RHS_NONE>), grid, block, 0, c.stream, in, tw, tw4, out);
+    CTDM_CHECK_LAUNCH("k_uw_rows_fwd");
 }
 
 template <int N>
-static void run_rows_fwd(Ctx& c, const float* in, int batch, int mode, bool sincos, float* out)
+static void run_cols(Ctx& c, const float* in, int batch, unsigned flags, float* out, bool existing,
+                     const double* num = nullptr, float* dc = nullptr)
 {
-    constexpr int G = 256 / Plan<N>::T;
-    hipLaunchKernelGGL((k_uw_rows_fwd<N, G>), dim3(grid1d((long long)batch * N, G)), dim3(G * Plan<N>::T), 0,
-                       c.stream, in, batch, mode, (int)sincos, c.tw(N), c.tw(4 * N), out);
-    CTDM_CHECK_LAUNCH("k_uw_rows_fwd");
+    const double* eig = eig_table(c, N, flags & F_REF_EIG, existing);
+    if (flags & F_REF_IDCT) {
+        constexpr int C = (256 / Plan<2 * N>::T) < N ? (256 / Plan<2 * N>::T) : N;
+        hipLaunchKernelGGL((k_uw_cols_ref<N, C>), dim3(batch * (N / C)), dim3(C * Plan<2 * N>::T), 0, c.stream, in,
+                           flags, eig, c.tw(N), c.tw(2 * N), c.tw(4 * N), out);
+    } else {
+        using PR = Pair<N>;
+        hipLaunchKernelGGL((k_uw_cols<N>), dim3(batch * (N / 2 / PR::CP)), dim3(PR::NC), 0, c.stream,
+                           (const float2*)in, flags, eig, c.tw(N), c.tw(4 * N), (float2*)out, num, dc);
+    }
+    CTDM_CHECK_LAUNCH("k_uw_cols");
+}
+
+// wrapped: the map to be congruent to, or null.
+template <int N>
+static void run_rows_inv(Ctx& c, const float* in, int batch, unsigned flags, const float* wrapped, float* out)
+{
+    if (!(flags & F_CONGRUENT)) wrapped = nullptr;
+    if (flags & F_REF_IDCT) {
+        constexpr int G = 256 / Plan<2 * N>::T;
+        hipLaunchKernelGGL((k_uw_rows_inv_ref<N, G>), dim3(grid1d((long long)batch * N, G)), dim3(G * Plan<2 * N>::T),
+                           0, c.stream, in, batch, wrapped, c.tw(2 * N), c.tw(4 * N), out);
+    } else {
+        using PR = Pair<N>;
+        hipLaunchKernelGGL((k_uw_rows_inv<N>), dim3((unsigned)((long long)batch * N / (2 * PR::GP))), dim3(PR::NT), 0,
+                           c.stream, in, wrapped, c.tw(N), c.tw(4 * N), out);
+    }
+    CTDM_CHECK_LAUNCH("k_uw_rows_inv");
 }
 
 // Intermediate spectra of one solve: context scratch, or (allocation-free entry point) the fixed
@@ -474,6 +725,8 @@ struct Work {
     float* D1 = nullptr;
     float* D2 = nullptr;
     bool existing = false;
+    const double* num = nullptr;  // adjoint only (k_uw_cols)
+    float* dc = nullptr;
 };
 
 // Whole solve for one size: mode 0 (wrapped input) or 1 (raw input, adjoint).
@@ -485,18 +738,9 @@ static void solve(Ctx& c, const float* in, int batch, unsigned flags, int mode, 
         w.D1 = (float*)c.buf("uw.D1", sizeof(float) * (size_t)batch * N * N);
         w.D2 = (float*)c.buf("uw.D2", sizeof(float) * (size_t)batch * N * N);
     }
-    run_rows_fwd<N>(c, in, batch, mode, flags & F_SINCOS, w.D1);
-    if (flags & F_REF_IDCT) {
-        if constexpr (N <= 256) {
-            run_cols<N, 2 * N>(c, w.D1, batch, flags, w.D2, w.existing);
-            run_rows_inv<N, 2 * N>(c, w.D2, batch, flags, wrapped, out);
-        } else {
-            fail(CTDM_EUNSUPPORTED, "REFCOMPAT_IDCT needs N <= 256");
-        }
-    } else {
-        run_cols<N, N>(c, w.D1, batch, flags, w.D2, w.existing);
-        run_rows_inv<N, N>(c, w.D2, batch, flags, wrapped, out);
-    }
+    run_rows_fwd<N>(c, in, batch, mode == 1 ? RHS_NONE : (flags & F_SINCOS ? RHS_SIN : RHS_WRAP), w.D1);
+    run_cols<N>(c, w.D1, batch, flags, w.D2, w.existing, w.num, w.dc);
+    run_rows_inv<N>(c, w.D2, batch, flags, wrapped, out);
 }
 
 static void solve_any(Ctx& c, const float* in, int batch, int N, unsigned flags, int mode,
@@ -604,13 +848,14 @@ template <int N>
 static void uw_rytov(Ctx& c, const float* wrapped, float* unwrapped, const float* logamp, int batch, unsigned flags,
                      float2* P)
 {
-    constexpr int G = 256 / Plan<N>::T;
+    using PR = Pair<N>;
     float* D1 = (float*)c.buf("uw.D1", sizeof(float) * (size_t)batch * N * N);
     float* D2 = (float*)c.buf("uw.D2", sizeof(float) * (size_t)batch * N * N);
-    run_rows_fwd<N>(c, wrapped, batch, 0, flags & F_SINCOS, D1);
-    run_cols<N, N>(c, D1, batch, flags, D2, false);
-    hipLaunchKernelGGL((k_uw_rows_inv_rytov<N, G>), dim3(grid1d((long long)batch * N, G)), dim3(G * Plan<N>::T), 0,
-                       c.stream, D2, batch, flags, wrapped, logamp, c.tw(N), c.tw(4 * N), unwrapped, P);
+    run_rows_fwd<N>(c, wrapped, batch, flags & F_SINCOS ? RHS_SIN : RHS_WRAP, D1);
+    run_cols<N>(c, D1, batch, flags, D2, false);
+    hipLaunchKernelGGL((k_uw_rows_inv_rytov<N>), dim3((unsigned)((long long)batch * N / (2 * PR::GP))), dim3(PR::NT),
+                       0, c.stream, D2, flags & F_CONGRUENT ? wrapped : nullptr, logamp, c.tw(N), c.tw(4 * N),
+                       unwrapped, P);
     CTDM_CHECK_LAUNCH("k_uw_rows_inv_rytov");
 }
 
@@ -645,12 +890,36 @@ void unwrap_dct_adjoint(Ctx& c, const float* wrapped, const float* g_out, float*
         CTDM_HIP(hipMemcpyAsync(g_in, g_out, sizeof(float) * n, hipMemcpyDeviceToDevice, c.stream));
         return;
     }
-    // J = D_rho * P with P the (symmetric) Poisson operator and D_rho the (symmetric) linearised
-    // RHS stencil, so J^T g = D_rho (P g).
+    // J = P D with P the (symmetric) Poisson operator and D the (symmetric) linearised RHS stencil, so
+    // J^T g = D (P g). Without SINCOS D is the Laplacian, which the DCT diagonalises: with the exact eigenvalues
+    // D P is the identity but for the mean, with the reference's it is the ratio of the two eigenvalues. With
+    // SINCOS the stencil's weights are cos of the phase differences.
+    CTDM_REQUIRE(batch > 0, "unwrap_dct_adjoint: negative batch");
+    if (!(M == 32 || M == 64 || M == 128 || M == 192 || M == 256))
+        fail(CTDM_EUNSUPPORTED, "unwrap size " + std::to_string(M) + " has no kernel");
+    const bool refeig = flags & F_REF_EIG;
+    if (!(flags & F_SINCOS)) {
+        if (!refeig) {
+            hipLaunchKernelGGL(k_uw_sub_mean, dim3(batch), dim3(1024), 0, c.stream, g_out, g_in, M * M);
+            CTDM_CHECK_LAUNCH("k_uw_sub_mean");
+            return;
+        }
+        Work w;
+        w.D1 = (float*)c.buf("uw.D1", sizeof(float) * n);
+        w.D2 = (float*)c.buf("uw.D2", sizeof(float) * n);
+        w.num = eig_table(c, M, false);
+        solve_any(c, g_out, batch, M, F_REF_EIG, 1, nullptr, g_in, w);
+        return;
+    }
     float* tmp = (float*)c.buf("uw.adj", sizeof(float) * n);
-    solve_any(c, g_out, batch, M, flags & F_REF_EIG, 1, nullptr, tmp);
-    hipLaunchKernelGGL(k_uw_stencil, dim3(grid1d((long long)n, 256)), dim3(256), 0, c.stream, tmp, wrapped, batch,
-                       M, (int)(flags & F_SINCOS), g_in);
+    Work w;
+    w.D1 = (float*)c.buf("uw.D1", sizeof(float) * n);
+    w.D2 = (float*)c.buf("uw.D2", sizeof(float) * n);
+    if (!refeig) w.dc = (float*)c.buf("uw.dc", sizeof(float) * (size_t)batch);
+    solve_any(c, g_out, batch, M, flags & F_REF_EIG, 1, nullptr, tmp, w);
+    const long long quads = (long long)n / 4;
+    hipLaunchKernelGGL(k_uw_stencil, dim3(grid1d(quads, 256)), dim3(256), 0, c.stream, tmp, wrapped, M, quads,
+                       refeig ? nullptr : g_out, (const float*)w.dc, g_in);
     CTDM_CHECK_LAUNCH("k_uw_stencil");
 }
 
