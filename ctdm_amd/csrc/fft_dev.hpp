@@ -352,6 +352,17 @@ __device__ __forceinline__ int xcd_block(int i, int n)
     return (i & 7) * per + (i >> 3);
 }
 
+// Stores an element (8-byte aligned) straight through this XCD's L2, as a device-scope relaxed store.
+// An ordinary store leaves the line dirty in the L2 of the XCD that ran the workgroup, and it is written
+// back when the kernel ends, while nothing else runs, or when another XCD asks for it. Where the next kernel
+// reads the data from other XCDs, writing it through moves that time under the rest of the kernel.
+__device__ __forceinline__ void store_through(float2* p, float2 v)
+{
+    unsigned long long u;
+    __builtin_memcpy(&u, &v, sizeof u);
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Radix plans per transform length. T = threads cooperating on one transform.
 template <int N>
 struct Plan;
