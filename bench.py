@@ -34,10 +34,10 @@ A, H, V, ITERS = 60, 1024, 256, 10
 # runs, FETCH_SIZE then WRITE_SIZE, scaled by the copy yardstick); its machine-readable line names the
 # libctdm.so build it measured. The profiler cannot run inside this process.
 TRAFFIC_PROFILE = ROOT / "profiles" / "traffic_config2_pmc.md"
-PASS_KEYS = {0: "k_vol_x", 1: "k_vol_y", 2: "k_vol_zdc"}
-PASS_NAMES = {0: "k_vol_x (inverse x-FFT + projection + forward x-FFT)",
+PASS_KEYS = {0: "k_vol_xy", 1: "k_vol_y", 2: "k_vol_zy"}
+PASS_NAMES = {0: "k_vol_xy (half of the inverse y-FFT, inverse x-FFT + projection + forward x-FFT, half of the y-FFT)",
               1: "k_vol_y (y-FFT)",
-              2: "k_vol_zdc (z-FFT + data consistency + inverse z-FFT)"}
+              2: "k_vol_zy (half of the y-FFT, z-FFT + data consistency + inverse z-FFT, half of the inverse y-FFT)"}
 
 
 def lib_sha16() -> str:
@@ -133,8 +133,8 @@ def main() -> int:
         log(f"batched {ms:.3f} ms/vol ({value:.1f} vol/s), plain {ms_plain:.2f} ms/vol, max|dn| {dn:.2e}")
 
     # roofline of the dominant kernel: live HIP-event timing of each fused volume pass inside the
-    # loop's own sequence (x, y, z+dc, y) on the stream the kernels run on
-    per_vol = {0: ITERS, 1: 2 * ITERS + 1, 2: ITERS}  # launches per volume of each pass
+    # loop's own sequence (xy, zy) on the stream the kernels run on
+    per_vol = {0: ITERS + 1, 1: 1, 2: ITERS}  # launches per volume of each pass
     lms, lbytes = ctx.time_loop(V, 2 * ITERS)
     kernels = {}
     for k in (0, 1, 2):

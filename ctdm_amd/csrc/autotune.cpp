@@ -1,9 +1,9 @@
-// Autotuner: for every requested volume side, times each fused volume pass (x with projection,
-// y, z with data consistency) with 8 and 16 pencils per workgroup on this device, inside the
+// Autotuner: for every requested volume side, times each fused volume pass (xy with projection,
+// y, zy with data consistency) with both tile sizes on this device, inside the
 // positivity loop's own pass sequence (ctdm_time_loop; each pass reads what the previous one wrote),
-// and keeps the faster choice (for y and z+dc, 8 pencils only when clearly faster) in the context
+// and keeps the faster choice (for y and zy, 8 only when clearly faster) in the context
 // (used by every later launch of that side, including graph captures made afterwards); then the sweep
-// direction of the x and y passes (forward, or one of them walking the z planes backwards so that it
+// direction of the xy and y passes (forward, or one of them walking the z planes backwards so that it
 // starts on the planes the previous pass wrote last), the radix plan of the y pass and the pencils per
 // workgroup of the gridding pass. An explicit call re-times every side; a reconstruction asking for
 // tuning only times sides not tuned yet. The choices are also kept per (device architecture, side) for
@@ -57,10 +57,10 @@ std::string autotune(Ctx& c, const int* sizes, int nsizes, bool force)
             }
             t.ms[k][0] = m[0];
             t.ms[k][1] = m[1];
-            // y and z+dc pencils are strided: 8 of them write 64-byte halves of 128-byte lines, which
-            // costs more inside a replayed reconstruction than in this short timed sequence (measured
-            // in a graph: z+dc 54.9 us at 8 pencils against 50.7 us at 16, where this timing had the two
-            // within 1 %). Those passes take 8 pencils only on a clear margin; x rows are contiguous.
+            // 8 y pencils write 64-byte halves of 128-byte lines, which costs more inside a replayed
+            // reconstruction than in this short timed sequence, and the zy pass's two tiles lie within the
+            // timing's spread at the sides where both fill the device (128^3: 14.3 and 14.7 us). These
+            // take 8 only on a clear margin.
             const double margin = k == 0 ? 1.0 : 0.97;
             t.pencils[k] = m[0] < margin * m[1] ? 8 : 16;
             char line[200];
@@ -68,9 +68,9 @@ std::string autotune(Ctx& c, const int* sizes, int nsizes, bool force)
                           names[k], m[0], m[1], t.pencils[k], bytes[k] / (1e6 * std::min(m[0], m[1])));
             rep << line;
         }
-        // Sweep directions: the loop sequence timed with the x pass, then the y passes, walking the z
-        // planes backwards (outputs are identical; only the order of the tiles changes), kept when the
-        // iteration (x + 2 y + z+dc) is at least 1 % faster than with both forward.
+        // Sweep directions: the sequence timed with the xy pass, then the y pass, walking the z
+        // planes backwards (outputs are identical; only the order of the tiles changes), kept when
+        // the three together are at least 1 % faster than with both forward.
         static const int combos[3][2] = {{0, 0}, {1, 0}, {0, 1}};
         int best = 0;
         for (int v = 0; v < 3; ++v) {
@@ -78,26 +78,27 @@ std::string autotune(Ctx& c, const int* sizes, int nsizes, bool force)
             t.rev[1] = combos[v][1];
             double ms[3], bytes[3];
             time_loop(c, V, kIters, ms, bytes);
-            t.sweep_ms[v] = ms[0] + 2.0 * ms[1] + ms[2];
+            t.sweep_ms[v] = ms[0] + ms[1] + ms[2];
             if (t.sweep_ms[v] < (best == 0 ? 0.99 : 1.0) * t.sweep_ms[best]) best = v;
         }
         t.rev[0] = combos[best][0];
         t.rev[1] = combos[best][1];
         char line[240];
-        std::snprintf(line, sizeof line, "V=%d sweep  fwd %.4f ms  x-rev %.4f ms  y-rev %.4f ms per iteration -> %s\n", V,
+        std::snprintf(line, sizeof line, "V=%d sweep  fwd %.4f ms  x-rev %.4f ms  y-rev %.4f ms -> %s\n", V,
                       t.sweep_ms[0], t.sweep_ms[1], t.sweep_ms[2], best == 0 ? "fwd" : (best == 1 ? "x-rev" : "y-rev"));
         rep << line;
-        // Radix plan of the y pass: the alternative factorisation is kept when its y launches are at
-        // least 5 % faster inside the loop sequence. It rounds differently, so the choice must not hang on the
-        // timing's own spread (a few per cent of the few microseconds a small volume's pass takes), or two
-        // tunings of one side would give volumes that differ in the last bits.
-        for (int pv = 0; pv < 2; ++pv) {
-            t.yplan = pv;
+        // Radix plan of the y pass: the alternative factorisation is kept when its slowest of three timings leads
+        // the base plan's fastest by 10 %. It rounds differently, so the choice must not hang on the timing's own
+        // spread (a few per cent of the few microseconds a small volume's pass takes), or two tunings of one side would
+        // give volumes that differ in the last bits; and the pass runs once per reconstruction.
+        for (int r = 0; r < 6; ++r) {
+            t.yplan = r & 1;
             double ms[3], bytes[3];
-            time_loop(c, V, kIters, ms, bytes);
-            t.yplan_ms[pv] = ms[1];
+            time_loop(c, V, 4 * kIters, ms, bytes);
+            if (r < 2 || (t.yplan == 0 ? ms[1] < t.yplan_ms[0] : ms[1] > t.yplan_ms[1]))
+                t.yplan_ms[t.yplan] = ms[1];
         }
-        t.yplan = t.yplan_ms[1] < 0.95 * t.yplan_ms[0] ? 1 : 0;
+        t.yplan = t.yplan_ms[1] < 0.9 * t.yplan_ms[0] ? 1 : 0;
         std::snprintf(line, sizeof line, "V=%d y plan  base %.4f ms  alternative %.4f ms -> %s\n", V, t.yplan_ms[0],
                       t.yplan_ms[1], t.yplan ? "alternative" : "base");
         rep << line;

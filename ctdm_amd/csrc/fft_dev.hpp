@@ -264,12 +264,29 @@ struct TwStager {
     }
 };
 
+// A TwPad for transforms whose T threads lie in one wave (T divides 64, groups aligned): the stages then
+// only order the wave's own LDS accesses, which execute in program order, and its waves never wait for each other.
+struct TwWave : TwPad {};
+template <class TW>
+__device__ __forceinline__ void stage_sync(const TW&)
+{
+    __syncthreads();
+}
+__device__ __forceinline__ void stage_sync(const TwWave&)
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // Cooperative N-point transform by T threads of one transform; threads with t >= T only take part
 // in the barriers (so a workgroup sized for a longer transform can run a shorter one).
 // gload(i) supplies input element i (called in the first stage), gstore(i, v) receives output
 // element i (called in the last stage); intermediate stages exchange through the LDS area `s`
 // (LdsSize<N>::value float2). Every thread of the workgroup must call this with the same template
-// arguments: it contains __syncthreads().
+// arguments: it contains __syncthreads() (with a TwWave table, every thread of the wave). A RegFile in place
+// of gstore receives the last stage's outputs: slot (p, r) holds element j + r N/R, j = t + p T, R the last
+// radix, which is what the first stage of a transform that begins with R reads.
 template <int N, int T, int DIR, int L, int R, int... Rest>
 struct Stockham {
     template <class TW, class GLoad, class GStore>
@@ -281,6 +298,8 @@ struct Stockham {
         constexpr bool LAST = (sizeof...(Rest) == 0);
         constexpr bool REG_IN = FIRST && IsRegFile<GLoad>::value;
         if constexpr (REG_IN) static_assert(GLoad::P == P && GLoad::R == R, "register input must match the stage");
+        constexpr bool REG_OUT = LAST && IsRegFile<GStore>::value;
+        if constexpr (REG_OUT) static_assert(GStore::P == P && GStore::R == R, "register output must match the stage");
         float2 v[P][R];
 #pragma unroll
         for (int p = 0; p < P; ++p) {
@@ -302,7 +321,7 @@ struct Stockham {
                 }
             }
         }
-        __syncthreads();  // every read of this stage precedes any write into `s`
+        stage_sync(tw);  // every read of this stage precedes any write into `s`
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const int j = t + p * T;
@@ -323,7 +342,9 @@ struct Stockham {
                 float2* sb = s + (WR == 1 ? lds_pad(base) : lds_pad((j - k) * R) + k);
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    if constexpr (LAST)
+                    if constexpr (REG_OUT)
+                        gstore.v[p][r] = v[p][r];
+                    else if constexpr (LAST)
                         gstore(base + r * L, v[p][r]);
                     else if constexpr (WR == 1 || WR == 2)
                         sb[lds_pad(r * L)] = v[p][r];
@@ -335,7 +356,7 @@ struct Stockham {
             }
         }
         if constexpr (!LAST) {
-            __syncthreads();
+            stage_sync(tw);
             Stockham<N, T, DIR, L * R, Rest...>::run(t, s, tw, gload, gstore);
         }
     }

@@ -57,12 +57,12 @@ struct Ctx;
 
 // Per-size kernel choices picked by the autotuner (defaults are the untuned picks).
 struct Tune {
-    int pencils[4] = {16, 16, 16, 8};  // pencils per workgroup of the x, y, z+dc and gridding passes
-    int rev[2] = {0, 0};               // x and y passes sweep the z planes backwards
+    int pencils[4] = {16, 16, 16, 8};  // tile size of the xy, y, zy and gridding passes
+    int rev[2] = {0, 0};               // xy and y passes sweep the z planes backwards
     int yplan = 0;                     // radix plan of the y pass: 0 Plan<V>, 1 PlanAlt<V>
     bool tuned = false;
     double ms[4][2] = {};               // measured ms per launch for B = 8, 16 (after tuning)
-    double sweep_ms[3] = {};            // loop iteration (x + 2 y + z+dc) for sweeps (fwd, fwd), (rev, fwd), (fwd, rev)
+    double sweep_ms[3] = {};            // xy + y + zy for sweeps (fwd, fwd), (rev, fwd), (fwd, rev)
     double yplan_ms[2] = {};            // y pass per launch with either radix plan
     double grid_ms[2] = {};             // gridding pass per launch with 8 / 16 pencils
 };

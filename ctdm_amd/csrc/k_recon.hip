@@ -12,11 +12,11 @@
 //
 // Loop (HilbertTransform.cu:1940-1972): n = est_n(f); repeat { f = modify(n); F = FFT3(f);
 // F = F_meas on measured voxels; f = iFFT3(F); n = est_n(f) }, then the octant shift (:1974).
-// The fused schedule runs each iteration as 4 pencil passes over the volume:
-//   X: inverse x-FFT, 1/V^3, P = modify o est_n, forward x-FFT  (one read + one write)
-//   Y: forward y-FFT
-//   Z: forward z-FFT, data consistency from a compact per-pencil list, inverse z-FFT
-//   Y: inverse y-FFT
+// The fused schedule runs each iteration as two passes over the volume, with half of each y-FFT in either:
+//   XY: second half of the inverse y-FFT, inverse x-FFT, 1/V^3, P = modify o est_n, forward x-FFT, first
+//       half of the forward y-FFT  (one read + one write)
+//   ZY: second half of the forward y-FFT, forward z-FFT, data consistency from a compact per-pencil list,
+//       inverse z-FFT, first half of the inverse y-FFT
 // The unfused schedule (plain path) launches the reference's kernel sequence: modify, 3 FFT
 // passes, check, 3 FFT passes, scale, est_n.
 #include "fft_dev.hpp"
@@ -600,152 +600,300 @@ struct Tile {
     }
 };
 
-// How a volume pass stores (see store_through). The y and z passes give an XCD the same x blocks, the x pass
-// gives it rows: the next pass reads from other XCDs what the x pass writes and what the y pass before an x
-// pass writes (CROSS). Those two write through at every size. The other two stay within one L2 and write through
-// only while the volume fits the L2s together (16 MB at 128^3), where otherwise almost every line is still dirty
-// at the kernel's end. Whole reconstructions with ordinary stores / CROSS through / all through: 128^3 (45 maps)
-// 500 / 376 / 358 us, 192^3 (30 angles) 1086 / 1073 / 1076, 256^3 (fit) 9073 / 9022 / 9160.
-template <int V, bool CROSS>
-__device__ __forceinline__ void vol_store(float2* p, float2 v)
-{
-    if constexpr (CROSS || V <= 128)
-        store_through(p, v);
-    else
-        *p = v;
-}
-
-// X pass. MODE 0: P + forward (input real space); 1: inverse, scale, P, forward;
-// 2: inverse, scale, est_n, octant shift -> out; 3: est_n (+ shift) -> out.
+// Rows to n without an iteration. MODE 2: inverse x transform, scale, est_n, octant shift -> out;
+// 3: est_n (+ shift) -> out.
 template <int V, int B, int MODE>
-__global__ __launch_bounds__(B* Plan<V>::T) void k_vol_x(float2* __restrict__ W, float2* __restrict__ out,
+__global__ __launch_bounds__(B* Plan<V>::T) void k_vol_x(const float2* __restrict__ W, float2* __restrict__ out,
                                                          const float2* __restrict__ tw, Proj p, float scale,
-                                                         int shift, int rev)
+                                                         int shift)
 {
     constexpr int T = Plan<V>::T;
     __shared__ float2 lds[B * LdsSize<V>::value];
     __shared__ float2 twl[LdsSize<V>::value];
     TwStager<V, B * T> tws;
     tws.fetch(tw);
-    Tile<V, 0, B> tl(rev);
+    Tile<V, 0, B> tl;
     float2* s = lds + tl.b * LdsSize<V>::value;
-    float2* row = W + tl.base;
-    // modes 1 and 2: the row's elements are loaded before the table's LDS copy waits for the table
-    StageRegs<V, T, Plan<V>::R0> rin;
-    if constexpr (MODE == 1 || MODE == 2) load_first_stage<V, T, Plan<V>::R0>(rin, row, 1, tl.t);
-    __builtin_amdgcn_sched_barrier(0);
-    tws.put(twl);
-    const TwPad twp{twl};
+    const float2* row = W + tl.base;
     // destination row of the final n (octant shift)
     const int h = shift ? V / 2 : 0;
     const long long orow = ((long long)((tl.px + h) % V) + (long long)V * ((tl.py + h) % V)) * V;
     auto put_n = [&](int x, float2 v) { out[orow + (x + h) % V] = v; };
-    if constexpr (MODE == 0) {
-        auto gl = [&](int x) -> float2 { return project(row[x], p, 1.f); };
-        auto gs = [&](int k, float2 v) { vol_store<V, true>(row + k, v); };
-        Plan<V>::template run<-1>(tl.t, s, twp, gl, gs);
-    } else if constexpr (MODE == 3) {
+    if constexpr (MODE == 3) {
         for (int x = tl.t; x < V; x += Plan<V>::T) put_n(x, est_n(row[x], p));
     } else {
-        if constexpr (MODE == 1) {
-            auto gs = [&](int k, float2 v) { s[lds_pad(k)] = project(v, p, scale); };
-            Plan<V>::template run<+1>(tl.t, s, twp, rin, gs);
-            __syncthreads();
-            auto gl2 = [&](int k) -> float2 { return s[lds_pad(k)]; };
-            auto gs2 = [&](int k, float2 v) { vol_store<V, true>(row + k, v); };
-            Plan<V>::template run<-1>(tl.t, s, twp, gl2, gs2);
-        } else {
-            auto gs = [&](int k, float2 v) { put_n(k, est_n(cscale(v, scale), p)); };
-            Plan<V>::template run<+1>(tl.t, s, twp, rin, gs);
-        }
+        // the row's elements are loaded before the table's LDS copy waits for the table
+        StageRegs<V, T, Plan<V>::R0> rin;
+        load_first_stage<V, T, Plan<V>::R0>(rin, row, 1, tl.t);
+        __builtin_amdgcn_sched_barrier(0);
+        tws.put(twl);
+        const TwPad twp{twl};
+        auto gs = [&](int k, float2 v) { put_n(k, est_n(cscale(v, scale), p)); };
+        Plan<V>::template run<+1>(tl.t, s, twp, rin, gs);
     }
 }
 
-// Z pass with data consistency: forward z-FFT, replace measured voxels, inverse z-FFT.
-// Load order at kernel entry: the twiddle table and the pencil's list count, then the pencil's elements
-// (into the registers of the transform's first stage), then the list entries below the count (DC_PRE
-// per thread; longer lists finish in a loop) and the table's LDS copy. Those wait for the count and the
-// table only, so the data loads are in flight meanwhile, and no entry beyond the count is fetched (a
-// pencil's list averages a third of its capacity).
+// ---------------------------------------------------------------- the loop's two passes
+// Half of each y transform runs in the x pass and half in the z pass. With y = y0 + R2 r and ky = k1 + R1 k2
+// (V = R1 R2) the forward transform is R2 DFTs of length R1 over r, the factors exp(-2 pi i y0 k1 / V), and R1
+// DFTs of length R2 over y0; the inverse undoes them in reverse order. The DFTs over r stay within the rows
+// {y0 + R2 r} of one z plane (pass xy, which transforms those rows along x), the DFTs over y0 within the
+// (x, k1) pencils of all y0 and z (pass zy, which transforms them along z). One iteration reads and writes the
+// volume twice; with a y pass of its own in each direction it was four times. Per iteration, before (x + y + z +
+// y) and now (xy + zy), the streaming copy of the volume in brackets: 256^3 177 and 110 us (38.5), 192^3 92 and 70,
+// 128^3 31 and 26.5, 64^3 17.5 and 8.3.
+// Between the passes element (z, y0, k1, x) stands in the row pair of y0 and its neighbour y0 ^ 1, at slot k1:
+//   W[(z V + (y0 & ~1) + R2 k1) V + 2 x + (y0 & 1)],
+// rows that one xy workgroup both reads and writes, so the volume is transformed in place. Pairing two y0 doubles
+// the piece of a line that a zy workgroup of few x takes (16 bytes per x).
+template <int V>
+struct Split {
+    static constexpr int T = Plan<V>::T;
+    static constexpr int R1 = V / T >= 8 ? V / T : 8;  // 256: 16, 192: 12, 128, 64, 32: 8
+    static constexpr int R2 = V / R1;
+    static_assert(R1 * R2 == V && R2 % 2 == 0 && 64 % T == 0, "split of the y transform");
+    // Row spacing = T (mod 32) and area spacing = 16 (mod 32) float2: the 32 lanes of a half wave then cover every
+    // LDS bank once, with T lanes per row along x or z as well as with 16 columns of two neighbouring areas.
+    static constexpr int LS = (LdsSize<V>::value - T + 31) / 32 * 32 + T;
+    static constexpr int area(int rows) { return (rows * LS - 16 + 31) / 32 * 32 + 16; }
+    static __device__ long long at(int z, int y0, int k1, int x)  // of the pair's even member
+    {
+        return ((long long)z * V + (y0 & ~1) + R2 * k1) * V + 2 * x;
+    }
+};
+// Radix plan of a transform that reads the registers left by Plan<V>'s last stage.
+template <int V>
+using PlanAfter = std::conditional_t<V == 64 || V == 256, Plan<V>, PlanAlt<V>>;
+
+// xy pass: Y values of y0 (a multiple of 2) in one z plane, Y R1 rows of V per workgroup.
+// IN 0: rows of f, projected as they are read; 1: rows whose inverse x transform is due (y done); 2: rows of the
+// zy pass. OUT 0: on to the zy pass; 1: n = est_n, octant shift, to `out`.
+// The inverse x transform's last stage leaves each thread the elements that the forward one's first stage reads, so
+// the projection happens in registers. T lanes of one wave share a row: only the two changes between
+// columns and rows are workgroup barriers. Bound by vector issue (1645 instructions a wave at 256^3, about 45 us of
+// issue of the 50 us it takes). Y = 2 leaves two workgroups on a CU at 256^3, one loading while the other
+// computes; Y = 4 one: 50 and 73 us (192^3: 34 and 38, 128^3: 11.8 and 13.5). It writes through (see
+// store_through), since the zy pass reads every line on another XCD: with ordinary stores 128^3 takes 16.8 us and the
+// zy pass after it 18.8 instead of 14.7, 256^3 52.
+template <int V, int Y, int IN, int OUT>
+__global__ __launch_bounds__(Y* V, 4) void k_vol_xy(float2* __restrict__ W, float2* __restrict__ out,
+                                                 const float2* __restrict__ tw, Proj p, float scale, int shift, int rev)
+{
+    using S = Split<V>;
+    constexpr int T = S::T, R1 = S::R1, R2 = S::R2, LS = S::LS, AREA = S::area(R1), NT = Y * V;
+    static_assert(Y % 2 == 0 && R2 % Y == 0 && R1 * T == V, "a workgroup's rows and columns");
+    __shared__ float2 lds[Y * AREA];
+    __shared__ float2 twl[LdsSize<V>::value];
+    TwStager<V, NT> tws;
+    tws.fetch(tw);
+    const int blk = rev ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x;
+    const int z = blk / (R2 / Y), yb = blk % (R2 / Y) * Y;
+    // columns (x, y0), lanes walk the pair's members, then x
+    const int cy = (threadIdx.x / (2 * V)) * 2 + threadIdx.x % 2, cx = threadIdx.x / 2 % V;
+    float2* col = W + S::at(z, yb + cy, 0, cx) + cy % 2;
+    float2* cl = lds + cy * AREA + lds_pad(cx);
+    // rows, T lanes each
+    const int row = threadIdx.x / T, t = threadIdx.x % T;
+    const int y = yb + row / R1 + R2 * (row % R1);
+    float2* s = lds + (row / R1) * AREA + (row % R1) * LS;
+    constexpr long long KS = (long long)R2 * V;  // from slot k1 to the next, and from row r to the next
+    using First = StageRegs<V, T, Plan<V>::R0>;
+    using Mid = StageRegs<V, T, PlanAfter<V>::R0>;
+    const TwWave twp{{twl}};
+    Mid m;
+    auto invert = [&](auto& in) {
+        if constexpr (OUT == 0) {
+            Plan<V>::template run<+1>(t, s, twp, in, m);
+#pragma unroll
+            for (int q = 0; q < Mid::P; ++q)
+#pragma unroll
+                for (int r = 0; r < Mid::R; ++r) m.v[q][r] = project(m.v[q][r], p, scale);
+        } else {
+            const int h = shift ? V / 2 : 0;
+            float2* orow = out + ((long long)((y + h) % V) + (long long)V * ((z + h) % V)) * V;
+            auto gs = [&](int x, float2 v) { orow[(x + h) % V] = est_n(cscale(v, scale), p); };
+            Plan<V>::template run<+1>(t, s, twp, in, gs);
+        }
+    };
+    if constexpr (IN == 2) {
+        float2 a[R1];
+#pragma unroll
+        for (int k = 0; k < R1; ++k) a[k] = col[k * KS];
+        __builtin_amdgcn_sched_barrier(0);
+        tws.put(twl);
+        DFT<R1, +1>::run(a);
+#pragma unroll
+        for (int r = 0; r < R1; ++r) cl[r * LS] = a[r];
+        __syncthreads();
+        auto gl = [&](int x) -> float2 { return s[lds_pad(x)]; };
+        invert(gl);
+    } else {
+        const float2* src = W + ((long long)z * V + y) * V;
+        if constexpr (IN == 1) {
+            First f;
+            load_first_stage<V, T, Plan<V>::R0>(f, src, 1, t);
+            __builtin_amdgcn_sched_barrier(0);
+            tws.put(twl);
+            __syncthreads();
+            invert(f);
+        } else {
+            load_first_stage<V, T, PlanAfter<V>::R0>(m, src, 1, t);
+            __builtin_amdgcn_sched_barrier(0);
+            tws.put(twl);
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < Mid::P; ++q)
+#pragma unroll
+                for (int r = 0; r < Mid::R; ++r) m.v[q][r] = project(m.v[q][r], p, 1.f);
+        }
+    }
+    if constexpr (OUT == 0) {
+        auto gs = [&](int k, float2 v) { s[lds_pad(k)] = v; };
+        PlanAfter<V>::template run<-1>(t, s, twp, m, gs);
+        __syncthreads();
+        float2 a[R1];
+#pragma unroll
+        for (int r = 0; r < R1; ++r) a[r] = cl[r * LS];
+        DFT<R1, -1>::run(a);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) store_through(col + k * KS, a[k]);
+    }
+}
+
+typedef float F4 __attribute__((ext_vector_type(4), aligned(8)));  // two neighbouring elements of a volume
+
+// zy pass with data consistency, P values of x at one k1 per workgroup: the y0 half of the forward y transform,
+// forward z, replace measured voxels, inverse z, and the y0 half of the inverse y transform.
+// Load order at kernel entry: the twiddle table and the pencil's list count, then the columns' elements, then the
+// list entries below the count (DC_PRE per thread; longer lists finish in a loop): the data loads are in
+// flight meanwhile, and no entry beyond the count is fetched (a pencil's list averages a third of its capacity).
 // With tau != 1 a measured voxel moves only part of the way: F <- F + tau (m - F), the fit's
 // hit-preconditioned gradient step (see fit_pgd); tau == 1 is the exact replacement.
 // JT (the fit with its objective): before the step, each measured voxel adds h |F - m|^2 / 2 (h its
 // hit count, m the averaged measurement) to the workgroup's partial sum, written to dc.part[block].
-template <int V, int B, bool JT>
-__global__ __launch_bounds__(B* Plan<V>::T) void k_vol_zdc(float2* __restrict__ W, const float2* __restrict__ tw,
-                                                           DcList dc, float tau)
+// A workgroup's pieces of a line are 16 P bytes; the workgroups that share the line run side by side on one
+// XCD (xcd_block) and meet in its L2: reading and writing the volume in such pieces of 32 bytes takes 45.8 us at 256^3
+// (43.3 in whole lines, 126 without the remapping). P = 2 leaves two workgroups on a CU there, P = 4 one: 60
+// and 75 us (192^3: 36 and 46, 128^3: 14.7 and 14.3). The stores are ordinary: written through, the pieces
+// reach memory one by one (256^3: 126 us).
+template <int V, int P, bool JT>
+__global__ __launch_bounds__(P* Split<V>::R2* Split<V>::T, 4) void k_vol_zy(float2* __restrict__ W,
+                                                                         const float2* __restrict__ tw, DcList dc,
+                                                                         float tau)
 {
-    constexpr int T = Plan<V>::T;
+    using S = Split<V>;
+    constexpr int T = S::T, R1 = S::R1, R2 = S::R2, LS = S::LS, AREA = S::area(R2), NT = P * R2 * T;
     constexpr int DC_PRE = 4;
-    constexpr int LS = LdsStride<V, B>::value;
-    __shared__ float2 lds[B * LS];
+    constexpr int CP = (P * V + NT - 1) / NT;  // columns per thread
+    __shared__ float2 lds[P * AREA];
     __shared__ float2 twl[LdsSize<V>::value];
-    __shared__ double red[JT ? B * T : 1];
-    TwStager<V, B * T> tws;
+    __shared__ double red[JT ? NT : 1];
+    TwStager<V, NT> tws;
     tws.fetch(tw);
-    // list prefetch: lanes walk the entries of one pencil (contiguous in the list)
-    const int pb = threadIdx.x / T, k0 = threadIdx.x % T;
-    const int blk = Tile<V, 2, B>::block();
-    const long long dpencil = (long long)(blk % (V / B)) * B + pb + (long long)V * (blk / (V / B));
+    const int blk = xcd_block(blockIdx.x, gridDim.x);  // neighbouring x share lines
+    const int x0 = blk % (V / P) * P, k1 = blk / (V / P);
+    // pencils (x, k2), T lanes each
+    const int pen = threadIdx.x / T, t = threadIdx.x % T;
+    const long long dpencil = x0 + pen / R2 + (long long)V * (k1 + R1 * (pen % R2));
     const int n = min(dc.cnt[dpencil], dc.cap);  // a count never exceeds the list capacity
-    Tile<V, 2, B> tl;
-    float2* s = lds + tl.b * LS;
-    float2* pen = W + tl.base;
-    StageRegs<V, T, Plan<V>::R0> x;
-    load_first_stage<V, T, Plan<V>::R0>(x, pen, tl.stride, tl.t);
+    // columns (x, z), lanes walk x; y0 = 2 j and 2 j + 1 side by side
+    float2 a[CP][R2];
+#pragma unroll
+    for (int i = 0; i < CP; ++i) {
+        const int c = threadIdx.x + i * NT;
+        if (P * V % NT == 0 || c < P * V) {
+            const float2* src = W + S::at(c / P, 0, k1, x0 + c % P);
+#pragma unroll
+            for (int j = 0; j < R2 / 2; ++j) {
+                const F4 q = *reinterpret_cast<const F4*>(src + 2 * j * V);
+                a[i][2 * j] = make_float2(q.x, q.y);
+                a[i][2 * j + 1] = make_float2(q.z, q.w);
+            }
+        }
+    }
     __builtin_amdgcn_sched_barrier(0);  // keeps the data loads ahead of the waits for the count and the table
     tws.put(twl);
-    const TwPad twp{twl};
+    const TwWave twp{{twl}};
     // Branch-free: lanes past the count read the pencil's first entry (a line the others fetch anyway),
     // and the entries are used only below the count.
     int pz[DC_PRE], ph[DC_PRE];
     float2 pv[DC_PRE];
 #pragma unroll
     for (int r = 0; r < DC_PRE; ++r) {
-        const int k = k0 + r * T;
+        const int k = t + r * T;
         const long long e = dpencil * dc.cap + (k < n ? k : 0);
         pz[r] = dc.idx[e];
         pv[r] = dc.val[e];
         if constexpr (JT) ph[r] = dc.hit[e];
     }
-    double jacc = 0.0;
-    auto gs = [&](int k, float2 v) { s[lds_pad(k)] = v; };
-    Plan<V>::template run<-1>(tl.t, s, twp, x, gs);
+#pragma unroll
+    for (int i = 0; i < CP; ++i) {
+        const int c = threadIdx.x + i * NT;
+        if (P * V % NT == 0 || c < P * V) {
+            float2* cl = lds + (c % P) * AREA + lds_pad(c / P);
+#pragma unroll
+            for (int y0 = 1; y0 < R2; ++y0) a[i][y0] = cmul(a[i][y0], tw[y0 * k1]);
+            DFT<R2, -1>::run(a[i]);
+#pragma unroll
+            for (int k2 = 0; k2 < R2; ++k2) cl[k2 * LS] = a[i][k2];
+        }
+    }
     __syncthreads();
+    float2* s = lds + (pen / R2) * AREA + (pen % R2) * LS;
+    auto gl = [&](int k) -> float2 { return s[lds_pad(k)]; };
+    auto gs = [&](int k, float2 v) { s[lds_pad(k)] = v; };
+    Plan<V>::template run<-1>(t, s, twp, gl, gs);
+    stage_sync(twp);
+    double jacc = 0.0;
     {
-        float2* sp = lds + pb * LS;
         const bool relax = tau != 1.f;
         auto put = [&](int z, float2 m, int h) {  // each z appears once in a pencil's list
             if (relax || JT) {
-                const float2 F = sp[lds_pad(z)];
+                const float2 F = s[lds_pad(z)];
                 if constexpr (JT) {
                     const double dr = (double)F.x - m.x, di = (double)F.y - m.y;
                     jacc += 0.5 * h * (dr * dr + di * di);
                 }
                 if (relax) m = make_float2(F.x + tau * (m.x - F.x), F.y + tau * (m.y - F.y));
             }
-            sp[lds_pad(z)] = m;
+            s[lds_pad(z)] = m;
         };
 #pragma unroll
         for (int r = 0; r < DC_PRE; ++r) {
-            const int k = k0 + r * T;
+            const int k = t + r * T;
             const int z = pz[r];
             if (k < n && z >= 0 && z < V) put(z, pv[r], JT ? ph[r] : 0);
         }
-        for (int k = k0 + DC_PRE * T; k < n; k += T) {
+        for (int k = t + DC_PRE * T; k < n; k += T) {
             const long long e = dpencil * dc.cap + k;
             const int z = dc.idx[e];
             if (z >= 0 && z < V) put(z, dc.val[e], JT ? dc.hit[e] : 0);
         }
     }
     if constexpr (JT) {
-        const double tot = workgroup_sum<B * T>(jacc, red);  // its barriers also order the LDS updates
+        const double tot = workgroup_sum<NT>(jacc, red);
         if (threadIdx.x == 0) dc.part[blockIdx.x] = tot;
     }
+    stage_sync(twp);
+    Plan<V>::template run<+1>(t, s, twp, gl, gs);
     __syncthreads();
-    auto gl2 = [&](int k) -> float2 { return s[lds_pad(k)]; };
-    auto gs2 = [&](int z, float2 v) { vol_store<V, false>(pen + (long long)z * tl.stride, v); };
-    Plan<V>::template run<+1>(tl.t, s, twp, gl2, gs2);
+#pragma unroll
+    for (int i = 0; i < CP; ++i) {
+        const int c = threadIdx.x + i * NT;
+        if (P * V % NT == 0 || c < P * V) {
+            const float2* cl = lds + (c % P) * AREA + lds_pad(c / P);
+#pragma unroll
+            for (int k2 = 0; k2 < R2; ++k2) a[i][k2] = cl[k2 * LS];
+            DFT<R2, +1>::run(a[i]);
+            float2* dst = W + S::at(c / P, 0, k1, x0 + c % P);
+#pragma unroll
+            for (int j = 0; j < R2 / 2; ++j) {
+                const float2 u = j == 0 ? a[i][0] : cmul(a[i][2 * j], cconj(tw[2 * j * k1]));
+                const float2 v = cmul(a[i][2 * j + 1], cconj(tw[(2 * j + 1) * k1]));
+                *reinterpret_cast<F4*>(dst + 2 * j * V) = F4{u.x, u.y, v.x, v.y};
+            }
+        }
+    }
 }
 
 // Y pass (plain FFT along y).
@@ -770,7 +918,7 @@ __global__ __launch_bounds__(B* Plan<V>::T) void k_vol_y(float2* __restrict__ W,
     __builtin_amdgcn_sched_barrier(0);
     tws.put(twl);
     const TwPad twp{twl};
-    auto gs = [&](int k, float2 v) { vol_store<V, (DIR > 0)>(pen + (long long)k * tl.stride, v); };
+    auto gs = [&](int k, float2 v) { store_through(pen + (long long)k * tl.stride, v); };
     PL::template run<DIR>(tl.t, s, twp, x, gs);
 }
 
@@ -989,16 +1137,12 @@ struct VolOps {
     static constexpr int NT = B * Plan<V>::T;
     static dim3 grid() { return dim3((unsigned)((long long)V * V / B)); }
 
-    static void x(Ctx& c, int mode, float2* W, float2* out, const Proj& p, float scale, bool shift, int rev = 0)
+    static void x(Ctx& c, int mode, const float2* W, float2* out, const Proj& p, float scale, bool shift)
     {
-        const float2* tw = c.tw(V);
-        const int sh = shift;
-        switch (mode) {
-        case 0: vlaunch(c, &k_vol_x<V, B, 0>, grid(), dim3(NT), W, out, tw, p, scale, sh, rev); break;
-        case 1: vlaunch(c, &k_vol_x<V, B, 1>, grid(), dim3(NT), W, out, tw, p, scale, sh, rev); break;
-        case 2: vlaunch(c, &k_vol_x<V, B, 2>, grid(), dim3(NT), W, out, tw, p, scale, sh, rev); break;
-        default: vlaunch(c, &k_vol_x<V, B, 3>, grid(), dim3(NT), W, out, tw, p, scale, sh, rev); break;
-        }
+        if (mode == 2)
+            vlaunch(c, &k_vol_x<V, B, 2>, grid(), dim3(NT), W, out, c.tw(V), p, scale, (int)shift);
+        else
+            vlaunch(c, &k_vol_x<V, B, 3>, grid(), dim3(NT), W, out, c.tw(V), p, scale, (int)shift);
         CTDM_CHECK_LAUNCH("k_vol_x");
     }
     static void y(Ctx& c, float2* W, int dir, int rev = 0, int plan = 0)
@@ -1017,15 +1161,6 @@ struct VolOps {
         }
         CTDM_CHECK_LAUNCH("k_vol_y");
     }
-    static void zdc(Ctx& c, float2* W, const DcList& dc, float tau)
-    {
-        const float2* tw = c.tw(V);
-        if (dc.part && dc.hit)
-            vlaunch(c, &k_vol_zdc<V, B, true>, grid(), dim3(NT), W, tw, dc, tau);
-        else
-            vlaunch(c, &k_vol_zdc<V, B, false>, grid(), dim3(NT), W, tw, dc, tau);
-        CTDM_CHECK_LAUNCH("k_vol_zdc");
-    }
     // W == nullptr: the list only.
     static void grid_pass(Ctx& c, const float2* spec, const double* rows, int A, const EwaldGeom& g, bool ref,
                           float2* W, const DcList& dc)
@@ -1040,19 +1175,43 @@ struct VolOps {
     }
 };
 
+// The loop's passes for one tile size: G pairs of y0 (xy) or G pairs of x (zy) per workgroup.
+template <int V, int G>
+struct LoopOps {
+    using S = Split<V>;
+    static constexpr unsigned XY_BLOCKS = V * S::R2 / (2 * G), ZY_BLOCKS = V / (2 * G) * S::R1;
+    template <int IN, int OUT>
+    static void xy(Ctx& c, float2* W, float2* out, const Proj& p, float scale, bool shift, int rev)
+    {
+        vlaunch(c, &k_vol_xy<V, 2 * G, IN, OUT>, dim3(XY_BLOCKS), dim3(2 * G * V), W, out, c.tw(V), p, scale, (int)shift,
+                rev);
+        CTDM_CHECK_LAUNCH("k_vol_xy");
+    }
+    static void zy(Ctx& c, float2* W, const DcList& dc, float tau)
+    {
+        const dim3 g(ZY_BLOCKS), b(2 * G * S::R2 * S::T);
+        if (dc.part && dc.hit)
+            vlaunch(c, &k_vol_zy<V, 2 * G, true>, g, b, W, c.tw(V), dc, tau);
+        else
+            vlaunch(c, &k_vol_zy<V, 2 * G, false>, g, b, W, c.tw(V), dc, tau);
+        CTDM_CHECK_LAUNCH("k_vol_zy");
+    }
+};
+
 // Runtime choice of B per pass kind (autotuned; 16 by default).
 enum PassKind { PASS_X = 0, PASS_Y = 1, PASS_ZDC = 2, PASS_GRID = 3, NPASS = 4, PASS_COPY = 4 };
 
 template <int V>
 struct Vol {
     static int pick(Ctx& c, PassKind k) { return c.tuning(V).pencils[k] == 8 ? 8 : 16; }
-    // Sweep direction of the x and y passes (tuned): both walk the z planes in tile order, so running
-    // one of them backwards starts each pass on the planes the previous one wrote last.
-    static void x(Ctx& c, int mode, float2* W, float2* out, const Proj& p, float scale, bool shift)
+    // Sweep direction of the xy and y passes (tuned): both walk the z planes in tile order, so running
+    // one of them backwards starts it on the planes the previous pass wrote last.
+    template <int IN, int OUT>
+    static void xy(Ctx& c, float2* W, float2* out, const Proj& p, float scale, bool shift)
     {
         const int rev = c.tuning(V).rev[0];
-        if (pick(c, PASS_X) == 8) VolOps<V, 8>::x(c, mode, W, out, p, scale, shift, rev);
-        else VolOps<V, 16>::x(c, mode, W, out, p, scale, shift, rev);
+        if (pick(c, PASS_X) == 8) LoopOps<V, 2>::template xy<IN, OUT>(c, W, out, p, scale, shift, rev);
+        else LoopOps<V, 1>::template xy<IN, OUT>(c, W, out, p, scale, shift, rev);
     }
     static void y(Ctx& c, float2* W, int dir)
     {
@@ -1060,10 +1219,14 @@ struct Vol {
         if (pick(c, PASS_Y) == 8) VolOps<V, 8>::y(c, W, dir, rev, plan);
         else VolOps<V, 16>::y(c, W, dir, rev, plan);
     }
-    static void zdc(Ctx& c, float2* W, const DcList& dc, float tau = 1.f)
+    static unsigned zy_blocks(Ctx& c)
     {
-        if (pick(c, PASS_ZDC) == 8) VolOps<V, 8>::zdc(c, W, dc, tau);
-        else VolOps<V, 16>::zdc(c, W, dc, tau);
+        return pick(c, PASS_ZDC) == 8 ? LoopOps<V, 2>::ZY_BLOCKS : LoopOps<V, 1>::ZY_BLOCKS;
+    }
+    static void zy(Ctx& c, float2* W, const DcList& dc, float tau = 1.f)
+    {
+        if (pick(c, PASS_ZDC) == 8) LoopOps<V, 2>::zy(c, W, dc, tau);
+        else LoopOps<V, 1>::zy(c, W, dc, tau);
     }
     static void grid_pass(Ctx& c, const float2* spec, const double* rows, int A, const EwaldGeom& g, bool ref,
                           float2* W, const DcList& dc)
@@ -1071,30 +1234,26 @@ struct Vol {
         if (pick(c, PASS_GRID) == 8) VolOps<V, 8>::grid_pass(c, spec, rows, A, g, ref, W, dc);
         else VolOps<V, 16>::grid_pass(c, spec, rows, A, g, ref, W, dc);
     }
-    // Loop after the initial inverse transform of the measured spectrum is in W up to the x pass:
-    // `first_x_mode` 0 if W holds real-space f, 1 if W still needs its inverse x-FFT. The z step is
-    // the data-consistency replacement (tau = 1) or the fit's relaxed step F <- F + tau (m - F).
-    // `jpart` (the fit with its objective): iteration it's z pass writes its workgroup partial sums to
-    // jpart + it * jstride.
+    // Loop from W = f in real space (`first_x` false), or W = f with its inverse x transform due (true).
+    // The zy pass applies the data-consistency replacement (tau = 1) or the fit's relaxed step
+    // F <- F + tau (m - F). `jpart` (the fit with its objective): iteration it's zy pass writes its workgroup
+    // partial sums to jpart + it * jstride.
     static void loop(Ctx& c, float2* W, float2* n_out, const DcList& dc, const Proj& p, int iters, bool shift,
-                     int first_x_mode, float tau = 1.f, double* jpart = nullptr, int jstride = 0)
+                     bool first_x, float tau = 1.f, double* jpart = nullptr, int jstride = 0)
     {
         const float s = (float)(1.0 / ((double)V * V * V));
         if (iters == 0) {
-            if (first_x_mode == 0)
-                x(c, 3, W, n_out, p, 1.f, shift);
-            else
-                x(c, 2, W, n_out, p, s, shift);
+            VolOps<V, 16>::x(c, first_x ? 2 : 3, W, n_out, p, s, shift);
             return;
         }
-        x(c, first_x_mode, W, n_out, p, s, shift);
+        if (first_x) xy<1, 0>(c, W, n_out, p, s, shift);
+        else xy<0, 0>(c, W, n_out, p, s, shift);
         for (int it = 0; it < iters; ++it) {
-            y(c, W, -1);
             DcList d = dc;
             d.part = jpart ? jpart + (size_t)it * jstride : nullptr;
-            zdc(c, W, d, tau);
-            y(c, W, +1);
-            x(c, it + 1 < iters ? 1 : 2, W, n_out, p, s, shift);
+            zy(c, W, d, tau);
+            if (it + 1 < iters) xy<2, 0>(c, W, n_out, p, s, shift);
+            else xy<2, 1>(c, W, n_out, p, s, shift);
         }
     }
 };
@@ -1108,7 +1267,7 @@ static void positivity_fused_v(Ctx& c, float2* f, const float2* Fm, const float*
     hipLaunchKernelGGL(k_dc_build, dim3(grid1d((long long)V * V, 256)), dim3(256), 0, c.stream, Fm, hits, V,
                        (int)ref, dc);
     CTDM_CHECK_LAUNCH("k_dc_build");
-    Vol<V>::loop(c, f, n, dc, p, iters, !(flags & CTDM_POS_NO_SHIFT), 0);
+    Vol<V>::loop(c, f, n, dc, p, iters, !(flags & CTDM_POS_NO_SHIFT), false);
 }
 
 void positivity_fused(Ctx& c, float2* f, const float2* Fm, const float* hits, float2* n, int V, int iters,
@@ -1137,7 +1296,7 @@ static void volume_batched_v(Ctx& c, const float2* spec, const double* rows, int
     float2* W = (float2*)c.buf("vol.W", sizeof(float2) * (size_t)V * V * V);
     Vol<V>::grid_pass(c, spec, rows, A, g, flags & CTDM_DC_REFCOMPAT, W, dc);
     Vol<V>::y(c, W, +1);
-    Vol<V>::loop(c, W, n_out, dc, make_proj(g), iters, !(flags & CTDM_POS_NO_SHIFT), 1);
+    Vol<V>::loop(c, W, n_out, dc, make_proj(g), iters, !(flags & CTDM_POS_NO_SHIFT), true);
 }
 
 void volume_batched(Ctx& c, const float2* spec, const double* rows, int A, int V, const ctdm_optics& o,
@@ -1190,7 +1349,7 @@ static void fit_pgd_v(Ctx& c, float2* f, const float2* spec, const double* rows,
     double* jdev = nullptr;
     int jstride = 0;
     if (objective && iters > 0) {
-        const int gblk = V * V / Vol<V>::pick(c, PASS_GRID), zblk = V * V / Vol<V>::pick(c, PASS_ZDC);
+        const int gblk = V * V / Vol<V>::pick(c, PASS_GRID), zblk = (int)Vol<V>::zy_blocks(c);
         jstride = zblk;
         ml.hit = (short*)c.buf("pgd.hit", sizeof(short) * (size_t)V * V * ml.cap);
         ml.part = (double*)c.buf("pgd.cpart", sizeof(double) * gblk);
@@ -1203,7 +1362,7 @@ static void fit_pgd_v(Ctx& c, float2* f, const float2* spec, const double* rows,
     } else {
         Vol<V>::grid_pass(c, spec, rows, A, g, false, nullptr, ml);  // m-bar = H^-1 G^T m per measured voxel
     }
-    Vol<V>::loop(c, f, n, ml, make_proj(g), iters, !(flags & CTDM_POS_NO_SHIFT), 0, tau, jpart, jstride);
+    Vol<V>::loop(c, f, n, ml, make_proj(g), iters, !(flags & CTDM_POS_NO_SHIFT), false, tau, jpart, jstride);
     if (jpart) {
         hipLaunchKernelGGL(k_sum_rows, dim3(iters), dim3(256), 0, c.stream, jpart, jstride, (const double*)jdev,
                            jdev + 1);
@@ -1286,10 +1445,10 @@ static double time_pass_v(Ctx& c, int kind, int B, int reps, double* bytes)
             hipLaunchKernelGGL(k_copy_vol, dim3(copy_grid), dim3(256), 0, c.stream, (const float4*)W, (float4*)nbuf, n4);
             CTDM_CHECK_LAUNCH("k_copy_vol");
             break;
-        case PASS_X: B == 8 ? VolOps<V, 8>::x(c, 1, W, nbuf, p, 1.f / (float)vol, true)
-                            : VolOps<V, 16>::x(c, 1, W, nbuf, p, 1.f / (float)vol, true); break;
+        case PASS_X: B == 8 ? LoopOps<V, 2>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true, 0)
+                            : LoopOps<V, 1>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true, 0); break;
         case PASS_Y: B == 8 ? VolOps<V, 8>::y(c, W, (r & 1) ? 1 : -1) : VolOps<V, 16>::y(c, W, (r & 1) ? 1 : -1); break;
-        case PASS_ZDC: B == 8 ? VolOps<V, 8>::zdc(c, W, dc, 1.f) : VolOps<V, 16>::zdc(c, W, dc, 1.f); break;
+        case PASS_ZDC: B == 8 ? LoopOps<V, 2>::zy(c, W, dc, 1.f) : LoopOps<V, 1>::zy(c, W, dc, 1.f); break;
         default: fail(CTDM_EINVAL, "time_pass: unknown pass");
         }
     };
@@ -1308,10 +1467,10 @@ static double time_pass_v(Ctx& c, int kind, int B, int reps, double* bytes)
     return ms / reps;
 }
 
-// The positivity loop's own sequence (x, forward y, z + data consistency, inverse y) run `iters` times
-// on the context's volume, each launch carrying its own start/end events (hipExtLaunchKernel): per-pass
-// average durations in the context they run in (each pass reads what the previous one wrote), with the
-// tuned choices.
+// The positivity loop's own sequence (xy, zy) run `iters` times on the context's volume, each launch carrying
+// its own start/end events (hipExtLaunchKernel): average durations in the context the passes run in (each reads
+// what the previous one wrote), with the tuned choices; and the y pass that precedes the loop, `iters` times on a
+// volume of its own.
 // Stand-in data-consistency list for timing before any reconstruction at this V: `per` entries per
 // pencil spread evenly over z (a 60-angle cell lands 20-30 samples on a typical pencil).
 __global__ void k_dc_synth(DcList dc, int V, int per)
@@ -1351,23 +1510,25 @@ static void time_loop_v(Ctx& c, int iters, double ms[3], double bytes[3])
     bytes[0] = vb;
     bytes[1] = vb;
     bytes[2] = vb + sizeof(int) * (double)VV + nent * (sizeof(float2) + sizeof(short));
-    const int nk = 4 * iters;
+    fill(c, nbuf, 2 * (long long)vol, 0.f);
+    const int nk = 3 * iters;
     std::vector<hipEvent_t> ev(2 * nk);
     for (auto& e : ev) CTDM_HIP(hipEventCreate(&e));
-    Vol<V>::x(c, 1, W, nbuf, p, 1.f / (float)vol, true);  // warm-up of the sequence
     auto arm = [&](int k) {
         c.tev[0] = ev[2 * k];
         c.tev[1] = ev[2 * k + 1];
     };
+    Vol<V>::y(c, nbuf, +1);  // warm-up
+    for (int it = 0; it < iters; ++it) {  // zeros, so that repeating the unnormalised transform keeps its values
+        arm(3 * it + 1);
+        Vol<V>::y(c, nbuf, +1);
+    }
+    Vol<V>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true);  // warm-up of the sequence
     for (int it = 0; it < iters; ++it) {
-        arm(4 * it);
-        Vol<V>::x(c, 1, W, nbuf, p, 1.f / (float)vol, true);
-        arm(4 * it + 1);
-        Vol<V>::y(c, W, -1);
-        arm(4 * it + 2);
-        Vol<V>::zdc(c, W, dc);
-        arm(4 * it + 3);
-        Vol<V>::y(c, W, +1);
+        arm(3 * it);
+        Vol<V>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true);
+        arm(3 * it + 2);
+        Vol<V>::zy(c, W, dc);
     }
     c.tev[0] = c.tev[1] = nullptr;
     CTDM_HIP(hipEventSynchronize(ev[2 * nk - 1]));
@@ -1375,13 +1536,10 @@ static void time_loop_v(Ctx& c, int iters, double ms[3], double bytes[3])
     for (int k = 0; k < nk; ++k) {
         float t = 0;
         CTDM_HIP(hipEventElapsedTime(&t, ev[2 * k], ev[2 * k + 1]));
-        const int kind = k % 4 == 0 ? 0 : (k % 4 == 2 ? 2 : 1);
-        acc[kind] += t;
+        acc[k % 3] += t;
     }
     for (auto& e : ev) hipEventDestroy(e);
-    ms[0] = acc[0] / iters;
-    ms[1] = acc[1] / (2.0 * iters);
-    ms[2] = acc[2] / iters;
+    for (int k = 0; k < 3; ++k) ms[k] = acc[k] / iters;
 }
 
 void time_loop(Ctx& c, int V, int iters, double ms[3], double bytes[3])

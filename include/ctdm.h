@@ -322,12 +322,12 @@ typedef struct ctdm_batch_opts {
 ctdm_status ctdm_reconstruct(ctdm_ctx *ctx, ctdm_cell *cells, int ncells,
                              const ctdm_batch_opts *opts);
 
-/* Times the three fused volume passes (x with projection, y, z with data consistency) of each
- * listed volume side V with 8 and 16 pencils per workgroup on this device, inside the positivity
- * loop's own pass sequence, and caches the choice in the context: the faster one, except that y and
- * z take 8 pencils only when at least 3 % faster (their 8-pencil tiles write half lines). Then times the
- * loop iteration with the x or the y passes sweeping the z planes backwards (kept when at least 1 %
- * faster), the y pass with its alternative radix plan (kept when at least 1 % faster) and the gridding
+/* Times the three fused volume passes (x with projection and z with data consistency, which hold half of
+ * the y transform each, and the y pass that precedes the loop) of each listed volume side V with both tile
+ * sizes on this device, inside the positivity loop's own pass sequence, and caches the choice in the
+ * context: the faster one, except that y and z take choice 8 only when at least 3 % faster. Then times the
+ * sequence with the x or the y pass sweeping the z planes backwards (kept when at least 1 %
+ * faster), the y pass with its alternative radix plan (kept when at least 10 % faster) and the gridding
  * pass with 8 and 16 pencils for 60 angles (16 when at least 3 % faster). The choices also serve contexts
  * created later in the process on the same GPU architecture. No reference counterpart. Every listed
  * side is re-timed, also one tuned before. Synchronises. `report` (HOST, may be NULL) receives a text
@@ -335,8 +335,9 @@ ctdm_status ctdm_reconstruct(ctdm_ctx *ctx, ctdm_cell *cells, int ncells,
 ctdm_status ctdm_autotune(ctdm_ctx *ctx, const int *sizes, int nsizes, char *report,
                           size_t report_len);
 
-/* The tuning table entry of volume side V (no reference counterpart): values[0..6] = pencils per workgroup
- * of the x, y, z+dc and gridding passes (8 or 16), the sweep direction of the x and y passes (0 forward,
+/* The tuning table entry of volume side V (no reference counterpart): values[0..6] = tile size of the x,
+ * y, z+dc and gridding passes (8 or 16: pencils per workgroup of y and gridding; the x and z+dc passes take two
+ * groups of pencils at 16, the default, and four at 8), the sweep direction of the x and y passes (0 forward,
  * 1 backwards over the z planes), and the radix plan of the y pass (0 the base factorisation, 1 the
  * alternative: 32 = 4x8, 64 = 4x4x4, 128 = 16x8, 192 = 16x12, 256 = 4x4x16). Pencil grouping and sweep
  * order compute bit-identical values; the two radix plans agree to FP32 rounding. ctdm_get_tuning reads the
@@ -347,18 +348,17 @@ ctdm_status ctdm_set_tuning(ctdm_ctx *ctx, int V, const int *values, int n);
 
 /* Average duration [ms] of one launch of a fused volume pass (pass 0: x with projection, 1: y,
  * 2: z with data consistency; 4: a plain streaming copy of the V^3 complex64 volume, the bandwidth
- * yardstick) at volume side V with `pencils` pencils per workgroup (8 or 16;
+ * yardstick) at volume side V with tile size `pencils` (8 or 16, as in ctdm_get_tuning;
  * <= 0 = the tuned choice), timed with hipEvents on the context stream over `reps` launches on the
  * context's volume buffer (no reference counterpart: the measuring primitive of ctdm_autotune).
  * *bytes receives the algorithmic bytes of one launch. Synchronises. */
 ctdm_status ctdm_time_pass(ctdm_ctx *ctx, int pass, int V, int pencils, int reps, double *avg_ms,
                            double *bytes);
 
-/* Runs `iters` iterations of the fused positivity loop's pass sequence (x with projection, forward y,
- * z with data consistency, inverse y) on the context's volume of side V, each launch carrying its own
- * start and end events (hipExtLaunchKernel), and returns the average duration [ms] of each pass in that
- * sequence
- * (avg_ms[0] x, [1] y, [2] z + data consistency; host arrays of 3) and its algorithmic bytes per
+/* Runs `iters` iterations of the fused positivity loop's pass sequence (x with projection, z with data
+ * consistency; each with its half of the y transform) on the context's volume of side V, each launch carrying its
+ * own start and end events (hipExtLaunchKernel), and `iters` launches of the y pass that precedes the loop, and
+ * returns the average duration [ms] of each pass (avg_ms[0] x, [1] y, [2] z + data consistency; host arrays of 3) and its algorithmic bytes per
  * launch (bytes[3]). Uses the data-consistency list of the last reconstruction at this V, when there is
  * one. No reference counterpart: the per-kernel measurement of the loop as it runs. Synchronises. */
 ctdm_status ctdm_time_loop(ctdm_ctx *ctx, int V, int iters, double *avg_ms, double *bytes);
