@@ -433,9 +433,13 @@ __device__ __forceinline__ float2 modify_f(float2 n, const Proj& p)
     return make_float2(-p.k2 * re, -p.k2 * im);
 }
 
-// modify_f(est_n(scale * f)) in one step, as the fused x pass applies it: with (a, b) = sqrt(1 - f/k^2) and
-// the positivity clamps a >= 1, b >= 0 (Re n >= n_m, Im n >= 0 without the n_m factor),
-// f' = -k^2 ((a - 1)(a + 1) - b^2) - i k^2 2ab, the same value as the two operators in exact arithmetic.
+// modify_f(est_n(scale * f)) in one step, as the fused x pass applies it: with (a, b) = sqrt(c + i d) = sqrt(1 - f/k^2)
+// and the positivity clamps a >= 1, b >= 0 (Re n >= n_m, Im n >= 0 without the n_m factor),
+// f' = -k^2 ((a^2 - 1) - b^2) - i k^2 2ab, the same value as the two operators in exact arithmetic. For c >= 0,
+// a^2 = h = (|z| + c) / 2 and, for d > 0, b = d / (2 sqrt h): a^2 - 1 with its clamp is max(h, 1) - 1, and 2ab is d where
+// a is not clamped (h >= 1) and 2b = d / sqrt h where it is, that is max(d, d / sqrt h). This needs neither a nor b:
+// two hardware roots per voxel instead of three and 20 other operations instead of 27 (the xy pass, bound by vector issue,
+// 50 -> 47 us at 256^3, 34 -> 31 at 192^3). The rare c < 0 (and a NaN) takes the general form.
 __device__ __forceinline__ float2 project(float2 f, const Proj& p, float scale)
 {
     const float ik = scale * p.inv_k2;
@@ -443,12 +447,15 @@ __device__ __forceinline__ float2 project(float2 f, const Proj& p, float scale)
     const float d = -f.y * ik;
     const float r = __builtin_amdgcn_sqrtf(c * c + d * d);
     const float h = 0.5f * (r + fabsf(c));
-    const float big = __builtin_amdgcn_sqrtf(h);
-    const float small = h > 0.f ? 0.5f * fabsf(d) * __builtin_amdgcn_rsqf(h) : 0.f;
-    float a = c >= 0.f ? big : small;
-    float b = d > 0.f ? (c >= 0.f ? small : big) : 0.f;  // b < 0 (d < 0) and b = 0 (d = 0) both clamp to 0
-    a = fmaxf(a, 1.f);
-    return make_float2(-p.k2 * ((a - 1.f) * (a + 1.f) - b * b), -p.k2 * (2.f * a * b));
+    if (__builtin_expect(!(c >= 0.f), 0)) {
+        const float big = __builtin_amdgcn_sqrtf(h);
+        const float small = h > 0.f ? 0.5f * fabsf(d) * __builtin_amdgcn_rsqf(h) : 0.f;
+        const float a = fmaxf(small, 1.f), b = d > 0.f ? big : 0.f;
+        return make_float2(-p.k2 * ((a - 1.f) * (a + 1.f) - b * b), -p.k2 * (2.f * a * b));
+    }
+    const float dp = fmaxf(d, 0.f);  // b < 0 (d < 0) and b = 0 (d = 0) both clamp to 0
+    const float dq = dp * __builtin_amdgcn_rsqf(fmaxf(h, 1.17549435e-38f));  // d / sqrt h, 0 at c = d = 0
+    return make_float2(-p.k2 * ((fmaxf(h, 1.f) - 1.f) - 0.25f * dq * dq), -p.k2 * fmaxf(dp, dq));
 }
 
 __global__ void k_est_n(const float2* __restrict__ f, float2* __restrict__ n, long long cnt, Proj p)
@@ -670,9 +677,9 @@ using PlanAfter = std::conditional_t<V == 64 || V == 256, Plan<V>, PlanAlt<V>>;
 // zy pass. OUT 0: on to the zy pass; 1: n = est_n, octant shift, to `out`.
 // The inverse x transform's last stage leaves each thread the elements that the forward one's first stage reads, so
 // the projection happens in registers. T lanes of one wave share a row: only the two changes between
-// columns and rows are workgroup barriers. Bound by vector issue (1645 instructions a wave at 256^3, about 45 us of
-// issue of the 50 us it takes). Y = 2 leaves two workgroups on a CU at 256^3, one loading while the other
-// computes; Y = 4 one: 50 and 73 us (192^3: 34 and 38, 128^3: 11.8 and 13.5). It writes through (see
+// columns and rows are workgroup barriers. Bound by vector issue and the copy itself (about 40 us each of
+// the 47 us it takes at 256^3). Y = 2 leaves two workgroups on a CU at 256^3, one loading while the other
+// computes; Y = 4 one: 50 and 73 us (192^3: 34 and 38, 128^3: 11.8 and 13.5, before the projection's last change). It writes through (see
 // store_through), since the zy pass reads every line on another XCD: with ordinary stores 128^3 takes 16.8 us and the
 // zy pass after it 18.8 instead of 14.7, 256^3 52.
 template <int V, int Y, int IN, int OUT>

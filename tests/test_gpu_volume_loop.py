@@ -80,3 +80,30 @@ def test_two_pass_loop(ctx, V, iters, fill):
             assert torch.equal(n, first), (px, pz, off)  # tile sizes and directions change no value
     finally:
         ctx.set_tuning(V, saved["pencils"], saved["sweep"], saved["yplan"])
+
+
+def test_projection_over_its_branches(ctx):
+    """One iteration with nothing measured gives est_n of the projection of f: 1 - f / k^2 over [-2, 3] x [-2, 2], with
+    zeros and the branch point, and a NaN voxel, which projects to 0. The volume's rms is 2 k^2, so its two
+    transforms leave 1.34 * 0.5 * 2 * 5 * 3e-7 * sqrt(2) = 3e-6 in n (|sqrt| >= 1 after the clamps); the bar is twice that."""
+    V = 64
+    k2 = (2 * np.pi * NM / LAM) ** 2
+    rng = np.random.default_rng(3)
+    c, d = rng.uniform(-2, 3, (V, V, V)), rng.uniform(-2, 2, (V, V, V))
+    f = (k2 * ((1 - c) - 1j * d)).astype(np.complex64)
+    f[0, 0, :3] = 0, np.float32(k2), np.float32(2 * k2)
+    f[1, 0, 0] = complex(0.5 * k2, 0)
+    g = f.copy()
+    g[2, 0, 0] = complex(np.nan, np.nan)
+    f[2, 0, 0] = 0
+    z = f.astype(np.complex128)
+    z.imag[z.imag == 0] = 0.0
+    want = est_n(z, k2)
+    none = torch.zeros((V, V, V), dtype=torch.float32, device="cuda")
+    o = ctdm_amd.Optics(LAM, NM, 0.1e-6)
+    for src in (f, g):
+        n = ctx.positivity(cuda(src), torch.zeros_like(cuda(f)), none, 1, o, ctdm_amd.POS_NO_SHIFT).cpu().numpy()
+        e = np.abs(n - want)
+        e[0, 0, 1:3] = 0  # at the cut itself the sign of a zero decides
+        print(f"max|dn| {e.max():.1e}")
+        assert e.max() <= 6e-6
