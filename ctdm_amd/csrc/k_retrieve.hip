@@ -83,6 +83,10 @@ __host__ __device__ inline CropDev make_crop_dev(int row, int col, int radius, i
     return d;
 }
 
+// Row pitch of the band arrays R and G, in columns: rows start on 64-byte boundaries, so that the column pass's
+// 8 columns are one half line per row and never the ends of two (60 pairs of 1024^2, 173 columns: 241.6 -> 238.2 us in all).
+__host__ __device__ inline int band_pitch(int n) { return (n + 7) & ~7; }
+
 __global__ void k_set_crop(CropDev* __restrict__ slot, int row, int col, int radius, int M, int H, int W)
 {
     *slot = make_crop_dev(row, col, radius, M, H, W);
@@ -91,7 +95,7 @@ __global__ void k_set_crop(CropDev* __restrict__ slot, int row, int col, int rad
 // ---------------------------------------------------------------- 1. real row FFT, pruned output
 // Each row of W reals is read as W/2 complex z[n] = x[2n] + i x[2n+1]; Z = FFT_{W/2}(z);
 // X[k] = (Z[k] + conj Z[-k]) / 2 - i/2 * exp(-2 pi i k / W) * (Z[k] - conj Z[-k]).
-// Output: out[(img*H + y)*nout + q] = X[(k_lo + q) mod W], q < nout. Images img < n0 come from
+// Output: out[(img*H + y)*band_pitch(nout) + q] = X[(k_lo + q) mod W], q < nout. Images img < n0 come from
 // src0, the others from src1 (sample holograms first, then backgrounds). PX: the pixel type.
 template <int W, int G, class PX>
 __global__ __launch_bounds__(G* Plan<W / 2>::T) void k_row_real(
@@ -144,7 +148,7 @@ __global__ __launch_bounds__(G* Plan<W / 2>::T) void k_row_real(
     auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
     Plan<NH>::template run<-1>(t, s, twp, x, gs);
     __syncthreads();
-    float2* dst = out + ((long long)img * H + y) * nout;
+    float2* dst = out + ((long long)img * H + y) * band_pitch(nout);
     auto emit = [&](int q, float2 w) {
         int k = (k_lo + q) % W;
         if (k < 0) k += W;
@@ -235,13 +239,14 @@ __global__ __launch_bounds__(C* Plan<H>::T) void k_col_band(
     const int img = blk / tiles;
     const int q = (blk % tiles) * C + cidx;
     const bool valid = q < nin && img < nimg;
+    const int np = band_pitch(nin);
     float2* s = lds + cidx * LS;
     if constexpr (HALF) {
-        // Element offsets within an image fit 32 bits (H * nin < 2^31); the image base is uniform.
-        const float2* base = in + (long long)(img < nimg ? img : 0) * H * nin;
-        const unsigned lane = (unsigned)t * nin + (valid ? q : 0);
+        // Element offsets within an image fit 32 bits (H * pitch < 2^31); the image base is uniform.
+        const float2* base = in + (long long)(img < nimg ? img : 0) * H * np;
+        const unsigned lane = (unsigned)t * np + (valid ? q : 0);
         auto gl = [&](int r) -> float2 {
-            return valid ? base[lane + (unsigned)(32 * r * nin)] : make_float2(0.f, 0.f);
+            return valid ? base[lane + (unsigned)(32 * r * np)] : make_float2(0.f, 0.f);
         };
         float2 v[32];
         col_fft1024_half_lds(t, s, tw_h, gl, v);
@@ -261,8 +266,8 @@ __global__ __launch_bounds__(C* Plan<H>::T) void k_col_band(
             s[e < q_n ? lds_pad(qq < 0 ? qq + M : qq) : spare] = v[k];
         }
     } else {
-        const float2* col = in + (long long)img * H * nin + (valid ? q : 0);
-        auto gl = [&](int i) -> float2 { return valid ? col[(long long)i * nin] : make_float2(0.f, 0.f); };
+        const float2* col = in + (long long)img * H * np + (valid ? q : 0);
+        auto gl = [&](int i) -> float2 { return valid ? col[(long long)i * np] : make_float2(0.f, 0.f); };
         auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
         Plan<H>::template run<-1>(t, s, tw_h, gl, gs);
     }
@@ -277,9 +282,9 @@ __global__ __launch_bounds__(C* Plan<H>::T) void k_col_band(
         if (ky < 0) ky += H;
         return s[lds_pad(ky)];
     };
-    float2* dst = out + (long long)img * M * nin + (valid ? q : 0);
+    float2* dst = out + (long long)img * M * np + (valid ? q : 0);
     auto gs2 = [&](int i, float2 v) {
-        if (valid) dst[(long long)i * nin] = v;
+        if (valid) dst[(long long)i * np] = v;
     };
     Plan<M>::template run<+1>(t, s, tw_m, gl2, gs2);
 }
@@ -317,7 +322,7 @@ __global__ __launch_bounds__(2 * GR * Plan<M>::T) void k_row_final(
     const int pair = blockIdx.x / tiles;
     const int y = (blockIdx.x % tiles) * GR + r;
     const long long img = (long long)pair + (long long)which * batch;
-    const float2* row = in + (img * M + y) * (long long)nin;
+    const float2* row = in + (img * M + y) * (long long)band_pitch(nin);
     float2* s = lds + tr * LdsSize<M>::value;
     auto gl = [&](int i) -> float2 {
         const int pp = i < M / 2 ? i : i - M;  // p'
@@ -467,15 +472,27 @@ static void row_real(Ctx& c, Pixels src0, int n0, Pixels src1, int nimg, int H, 
     });
 }
 
+template <int H, int M, int C>
+static void launch_col_band_c(Ctx& c, const float2* in, int nimg, int nin, int r0, const Band& qb, const CropDev* cd,
+                              float2* out)
+{
+    const int tiles = (nin + C - 1) / C;  // with a device crop, nin is the widest band (M)
+    hipLaunchKernelGGL((k_col_band<H, M, C>), dim3(tiles * nimg), dim3(C * Plan<H>::T), 0, c.stream,
+                       in, nimg, nin, tiles, c.tw(H), c.tw(M), r0, qb.lo, qb.n, cd, out);
+    CTDM_CHECK_LAUNCH("k_col_band");
+}
+
+// 256 threads per workgroup, or 128 while those leave three quarters of the CUs idle: one 1024^2 pair (44 workgroups,
+// 88) takes 39.1 and 38.3 us in all, four pairs with 131 columns (136, 264) 48.1 and 48.5, 60 pairs 238 and 257.
 template <int H, int M>
 static void launch_col_band(Ctx& c, const float2* in, int nimg, int nin, int r0, const Band& qb,
                             const CropDev* cd, float2* out)
 {
     constexpr int C = 256 / Plan<H>::T;
-    const int tiles = (nin + C - 1) / C;  // with a device crop, nin is the widest band (M)
-    hipLaunchKernelGGL((k_col_band<H, M, C>), dim3(tiles * nimg), dim3(C * Plan<H>::T), 0, c.stream,
-                       in, nimg, nin, tiles, c.tw(H), c.tw(M), r0, qb.lo, qb.n, cd, out);
-    CTDM_CHECK_LAUNCH("k_col_band");
+    if ((long long)((nin + C - 1) / C) * nimg * 4 < c.cus)
+        launch_col_band_c<H, M, C / 2>(c, in, nimg, nin, r0, qb, cd, out);
+    else
+        launch_col_band_c<H, M, C>(c, in, nimg, nin, r0, qb, cd, out);
 }
 
 template <int M>
@@ -519,9 +536,9 @@ static void retrieve_core(Ctx& c, Pixels holo, Pixels bg, int batch, int H, int 
                           float* refph)
 {
     const int nimg = 2 * batch;
-    const int nmax = cd ? M : pb.n;
-    float2* R = (float2*)c.buf("ret.R", sizeof(float2) * (size_t)nimg * H * nmax);
-    float2* G = (float2*)c.buf("ret.G", sizeof(float2) * (size_t)nimg * M * nmax);
+    const int nmax = cd ? M : pb.n, np = band_pitch(nmax);
+    float2* R = (float2*)c.buf("ret.R", sizeof(float2) * (size_t)nimg * H * np);
+    float2* G = (float2*)c.buf("ret.G", sizeof(float2) * (size_t)nimg * M * np);
     row_real(c, holo, batch, bg, nimg, H, W, k_lo, pb.n, cd, R);
     switch (H) {
     case 256: col_band_m<256>(c, M, R, nimg, nmax, r0, pb, cd, G); break;
