@@ -8,12 +8,15 @@
 //      concurrently, which is racy; the raster order makes it reproducible): k_gs_pair (one workgroup per
 //      map) pairs the residues, with rows side by side where no decision can reach another's, and k_gs_draw
 //      draws the chosen cuts in parallel.
-//   3. flood fill: level-synchronous breadth-first search over non-cut pixels from a fixed start; each
-//                     new pixel takes k from its first neighbour of the previous level in the order
-//                     right, left, below, above. Maps whose cut bits fit in LDS (up to 1.3 M pixels):
+//   3. fill           a pixel's 2 pi count is the sum of the steps along the path by which a level-synchronous
+//                     breadth-first search over non-cut pixels reaches it from a fixed start, each new pixel
+//                     from its first neighbour of the previous level in the order right, left, below,
+//                     above. Maps whose cut bits fit in LDS (up to 1.3 M pixels): a spanning forest gives the
+//                     counts without a search (k_gs_tile, k_gs_merge, k_gs_anchor; whole device), and every
+//                     step is checked against them; a map whose counts would depend on the path takes the search:
 //                     k_gs_bfs_lev (one workgroup per map, one barrier per level) stores each pixel's
-//                     level, k_gs_par_lev takes the parents from the levels, and k_gs_ptr_init /
-//                     k_gs_ptr_jump (whole device) sum the steps along the parent chains by pointer
+//                     level, k_gs_ptr_init takes the parents from the levels and k_gs_ptr_jump
+//                     (whole device) sums the steps along the parent chains by pointer
 //                     jumping. Larger maps: k_gs_bfs, with k along the levels.
 //   4. k_gs_finish    one thread per pixel: interior cut pixels next to a reached pixel take k from
 //                     it (same order); unwrapped = phi + 2 pi k, or 0 where unreached.
@@ -316,7 +319,7 @@ __device__ __forceinline__ unsigned ring_key(int dx, int dy)
 template <bool LDSW>
 __global__ __launch_bounds__(64 * GS_WAVES) void k_gs_pair(const int8_t* __restrict__ res, int H, int W,
                                                            unsigned* __restrict__ gwords, int2* __restrict__ pairs,
-                                                           int* __restrict__ rowpairs)
+                                                           int* __restrict__ rowpairs, int* __restrict__ flags)
 {
     extern __shared__ unsigned lwords[];
     // prog[first lane of a group]: its published index (the other lanes write the words beside it, which
@@ -328,6 +331,10 @@ __global__ __launch_bounds__(64 * GS_WAVES) void k_gs_pair(const int8_t* __restr
     const long long n = (long long)H * W;
     const int nw = (int)((n + 31) / 32);
     const int8_t* r = res + blockIdx.x * n;
+    if (tid == 0) {  // the fill's flag of this map, and behind the last one the longest chain
+        flags[blockIdx.x] = 0;
+        if (blockIdx.x == 0) flags[gridDim.x] = 0;
+    }
     int2* out = pairs + blockIdx.x * n;  // row y's choices start at out[y W], nrow[y] of them
     int* nrow = rowpairs + (long long)blockIdx.x * H;
     const Charges<LDSW> ch{(LDSW ? lwords : gwords + (long long)blockIdx.x * 2 * (nw + 3)) + 1, nw};
@@ -607,16 +614,246 @@ __global__ __launch_bounds__(1024) void k_gs_bfs(const float* __restrict__ phi, 
 // Bit p of a bit mask.
 __device__ __forceinline__ bool tbit(const unsigned* b, long long p) { return (b[p >> 5] >> (p & 31)) & 1u; }
 
-// ---------------------------------------------------------------- 3b. flood fill in two stages
-// For maps whose cut bits fit in LDS (up to 1.3 M pixels in 160 KiB). Stage 1 (k_gs_bfs_lev, one workgroup
-// per map, then k_gs_par_lev over every pixel) finds the levels of the search of k_gs_bfs and each reached
-// pixel's parent (the first neighbour of the previous level in the order right, left, below, above) as a
-// byte. Stage 2 (k_gs_ptr_init, k_gs_ptr_jump; the whole device) gives every reached pixel the pair
-// (parent, -step2pi(phi - phi_parent)) and contracts the parent chains by pointer jumping, (ptr, sum) <-
-// (ptr[ptr], sum + sum[ptr]), until each pointer is the start pixel, whose pair is (itself, 0). Then sum
+// ---------------------------------------------------------------- 3b. fill without a search
+// The 2 pi count of a reached pixel is the sum of the steps along the search's path to it. Where every loop of free
+// (not cut) pixels has steps that sum to zero, which is what the cuts are for, any path gives the same count, and the
+// paths need no levels: a spanning forest of the free pixels does. k_gs_tile joins the pixels of a tile in LDS,
+// k_gs_merge the tiles' trees over the tile borders, k_gs_anchor lets each tile's roots point to the map's root and
+// finds the start pixel's; k_gs_finish then adds two offsets per pixel. Each pixel's pair (ptr, sum), k(p) =
+// sum + k(ptr), is read and written as one 64-bit word; a root points to itself. Roots are hooked to roots of smaller
+// index by compare-and-swap, so pointers only fall, every walk ends, and a failed swap means that another one joined that root.
+// Every edge between free pixels is then checked (k_gs_tile within tiles, k_gs_anchor across their borders). A map with
+// an edge that disagrees, or with a step outside 32 bits, is flagged and takes the search of 3c, whose kernels return at
+// once for the others: whatever the input, the counts are the search's own. 64 maps of 512^2 (noise 0.8 rad; a map in
+// about 100 is flagged): fill and outputs 0.41 ms in place of 1.92 (k_gs_tile 0.10, merge 0.04, anchor 0.03, the idle search
+// 0.03, finish 0.21), 1.22 with a flagged map among them; one map of 256^2 60 us in place of 320. Tiles of 16 rows: 0.42,
+// of 64 (1024 threads) 0.41.
+constexpr int GS_TX = 64, GS_TY = 32;  // a tile: a wave's width, four rows for each of eight waves
+__device__ __forceinline__ unsigned long long gs_pack(int ptr, unsigned sum)
+{
+    return (unsigned long long)(unsigned)ptr | ((unsigned long long)sum << 32);
+}
+template <int SCOPE>
+__device__ __forceinline__ unsigned long long gs_pair_load(const unsigned long long* p)
+{
+    if constexpr (SCOPE == 0)
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int SCOPE>
+__device__ __forceinline__ void gs_pair_store(unsigned long long* p, unsigned long long v)
+{
+    if constexpr (SCOPE == 0)
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Root of node a; off gains the sums on the way. Pointers fall strictly, so the walk ends.
+template <int SCOPE>
+__device__ __forceinline__ int gs_root(const unsigned long long* node, int a, unsigned& off)
+{
+    for (;;) {
+        const unsigned long long v = gs_pair_load<SCOPE>(node + a);
+        const int up = (int)(unsigned)v;
+        if (up == a) return a;
+        off += (unsigned)(v >> 32);
+        a = up;
+    }
+}
+// Joins the trees of p and q, given k(p) = k(a) + oa, k(q) = k(b) + ob and k(q) = k(p) - s.
+template <int SCOPE>
+__device__ __forceinline__ void gs_unite(unsigned long long* node, int a, unsigned oa, int b, unsigned ob, unsigned s)
+{
+    for (;;) {
+        a = gs_root<SCOPE>(node, a, oa);
+        b = gs_root<SCOPE>(node, b, ob);
+        if (a == b) return;
+        const unsigned d = oa - s - ob;  // k(b) - k(a)
+        const int hi = a < b ? b : a;
+        unsigned long long self = gs_pack(hi, 0);
+        const unsigned long long link = a < b ? gs_pack(a, d) : gs_pack(b, 0u - d);
+        bool done;
+        if constexpr (SCOPE == 0)
+            done = __hip_atomic_compare_exchange_strong(node + hi, &self, link, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP);
+        else
+            done = __hip_atomic_compare_exchange_strong(node + hi, &self, link, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT);
+        if (done) return;
+    }
+}
+// A step outside 32 bits (the conversion saturates): its two directions are not each other's negative.
+__device__ __forceinline__ bool gs_step_bad(int s) { return s == INT_MIN || s == INT_MAX; }
+
+// One tile per workgroup, a row at a time per wave: the offsets within a run of free pixels are a prefix sum of the
+// row's steps, so the nodes are the runs (at their first pixels) and the edges to join the first of each overlap of a
+// run with one of the row above.
+__global__ __launch_bounds__(512) void k_gs_tile(const float* __restrict__ phi, const uint8_t* __restrict__ cuts, int H,
+                                                 int W, unsigned long long* __restrict__ pr, int* __restrict__ flag)
+{
+    constexpr int RW = GS_TY / 8;  // rows per wave
+    __shared__ unsigned long long node[GS_TX * GS_TY];
+    const long long n = (long long)H * W, b = blockIdx.z;
+    const float* ph = phi + b * n;
+    const uint8_t* cut = cuts + b * n;
+    const int lane = threadIdx.x & 63, r0 = (threadIdx.x >> 6) * RW;
+    const int x = blockIdx.x * GS_TX + lane, y0 = blockIdx.y * GS_TY;
+    float f[RW + 1];
+    unsigned long long m[RW + 1];  // free pixels of rows r0 - 1 .. r0 + RW - 1 (none above the tile's first row)
+    unsigned off[RW + 1];          // k(p) - k(first pixel of p's run)
+    int st[RW + 1];                // node of p's run
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i <= RW; ++i) {
+        const int row = r0 + i - 1, y = y0 + row;
+        const bool in = row >= 0 && y < H && x < W;
+        const long long g = in ? (long long)y * W + x : 0;
+        f[i] = ph[g];
+        const bool fr = in && cut[g] == 0;
+        m[i] = __ballot(fr);
+    }
+#pragma unroll
+    for (int i = 0; i <= RW; ++i) {
+        const float left = __shfl_up(f[i], 1);
+        const unsigned long long joined = m[i] & (m[i] << 1);  // free with a free left neighbour
+        const int s = (joined >> lane) & 1 ? gs_step2pi(__fsub_rn(f[i], left)) : 0;
+        bad |= gs_step_bad(s);
+        unsigned v = 0u - (unsigned)s;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned u = __shfl_up(v, o);
+            if (lane >= o) v += u;
+        }
+        const unsigned long long first = m[i] & ~joined & (~0ull >> (63 - lane));  // run starts up to this lane
+        const int sl = first ? 63 - __clzll(first) : lane;
+        off[i] = v - __shfl(v, sl);
+        st[i] = max(r0 + i - 1, 0) * GS_TX + sl;
+        if (i > 0 && sl == lane && ((m[i] >> lane) & 1)) node[st[i]] = gs_pack(st[i], 0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 1; i <= RW; ++i) {
+        const unsigned long long e = m[i] & m[i - 1];
+        if (((e & ~(e << 1)) >> lane) & 1)
+            gs_unite<0>(node, st[i - 1], off[i - 1], st[i], off[i], (unsigned)gs_step2pi(__fsub_rn(f[i], f[i - 1])));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 1; i <= RW; ++i) {
+        if (((m[i] >> lane) & 1) && (st[i] & 63) == lane) {
+            unsigned o = 0;
+            const int r = gs_root<0>(node, st[i], o);
+            gs_pair_store<0>(node + st[i], gs_pack(r, o));
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 1; i <= RW; ++i) {
+        const int y = y0 + r0 + i - 1;
+        if (x >= W || y >= H) continue;
+        unsigned long long out = gs_pack(-1, 0);
+        if ((m[i] >> lane) & 1) {
+            const unsigned long long v = node[st[i]];
+            const int r = (int)(unsigned)v;
+            const unsigned k = off[i] + (unsigned)(v >> 32);
+            if ((m[i - 1] >> lane) & 1) {
+                const int s = gs_step2pi(__fsub_rn(f[i], f[i - 1]));
+                bad |= gs_step_bad(s) || k != off[i - 1] + (unsigned)(node[st[i - 1]] >> 32) - (unsigned)s;
+            }
+            out = gs_pack((y0 + r / GS_TX) * W + (int)blockIdx.x * GS_TX + r % GS_TX, k);
+        }
+        pr[b * n + (long long)y * W + x] = out;
+    }
+    if (__any(bad) && lane == 0) atomicOr(flag + b, 1);
+}
+
+// Edge e of a map's tile borders: pixels p and q = right of or below p, of two tiles. `before`: how far back the pair before it
+// along the border lies when it joins the same two tiles (else 0): where that pair is free too the edge joins nothing new.
+__device__ __forceinline__ bool gs_border_edge(long long e, int H, int W, int& p, int& q, int& before)
+{
+    const long long nv = (long long)((W - 1) / GS_TX) * H, nh = (long long)((H - 1) / GS_TY) * W;
+    if (e >= nv + nh) return false;
+    if (e < nv) {
+        const int y = (int)(e % H), x = ((int)(e / H) + 1) * GS_TX;
+        q = y * W + x;
+        p = q - 1;
+        before = y % GS_TY ? W : 0;
+    } else {
+        const int x = (int)((e - nv) % W), y = ((int)((e - nv) / W) + 1) * GS_TY;
+        q = y * W + x;
+        p = q - W;
+        before = x % GS_TX ? 1 : 0;
+    }
+    return true;
+}
+
+__global__ __launch_bounds__(256) void k_gs_merge(const float* __restrict__ phi, const uint8_t* __restrict__ cuts, int H,
+                                                  int W, unsigned long long* __restrict__ pr)
+{
+    const long long n = (long long)H * W, base = blockIdx.y * n;
+    int p, q, before;
+    if (!gs_border_edge((long long)blockIdx.x * 256 + threadIdx.x, H, W, p, q, before)) return;
+    const uint8_t* cut = cuts + base;
+    if (cut[p] || cut[q] || (before && !cut[p - before] && !cut[q - before])) return;
+    const unsigned s = (unsigned)gs_step2pi(__fsub_rn(phi[base + q], phi[base + p]));
+    gs_unite<1>(pr + base, p, 0, q, 0, s);
+}
+
+// After the merge: every border edge is checked and its pixels, with the tile roots that they point to, are pointed to
+// the map's root; the last workgroup of a map writes the root of its start pixel with the start's offset (-1: none).
+__global__ __launch_bounds__(256) void k_gs_anchor(const float* __restrict__ phi, const uint8_t* __restrict__ cuts, int H,
+                                                   int W, unsigned long long* __restrict__ pr,
+                                                   unsigned long long* __restrict__ start, int* __restrict__ flag)
+{
+    const long long n = (long long)H * W, base = blockIdx.y * n;
+    const uint8_t* cut = cuts + base;
+    unsigned long long* node = pr + base;
+    if (blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x != 0) return;
+        int sx = W / 2, sy = min(20, H - 1);
+        while (sx >= 0 && sy < H && cut[sx + (long long)W * sy]) {
+            --sx;
+            ++sy;
+        }
+        unsigned long long v = gs_pack(-1, 0);
+        if (sx >= 0 && sy < H) {
+            unsigned o = 0;
+            const int r = gs_root<1>(node, sx + W * sy, o);
+            v = gs_pack(r, o);
+        }
+        start[blockIdx.y] = v;
+        return;
+    }
+    int p, q, before;
+    if (!gs_border_edge((long long)blockIdx.x * 256 + threadIdx.x, H, W, p, q, before) || cut[p] || cut[q]) return;
+    const int s = gs_step2pi(__fsub_rn(phi[base + q], phi[base + p]));
+    // the pixel's own pair, then the node it points to: both get the root
+    auto settle = [&](int a, unsigned& k) {
+        const unsigned long long v = gs_pair_load<1>(node + a);
+        const int t = (int)(unsigned)v;
+        unsigned o = 0;
+        const int r = gs_root<1>(node, t, o);
+        k = (unsigned)(v >> 32) + o;
+        if (t != r) {
+            gs_pair_store<1>(node + t, gs_pack(r, o));
+            gs_pair_store<1>(node + a, gs_pack(r, k));
+        }
+        return r;
+    };
+    unsigned kp, kq;
+    const int rp = settle(p, kp), rq = settle(q, kq);
+    if (gs_step_bad(s) || rp != rq || kq != kp - (unsigned)s) atomicOr(flag + blockIdx.y, 1);
+}
+
+// ---------------------------------------------------------------- 3c. flood fill in two stages
+// For flagged maps (see 3b) whose cut bits fit in LDS (up to 1.3 M pixels in 160 KiB). Stage 1 (k_gs_bfs_lev, one
+// workgroup per map) finds the levels of the search of k_gs_bfs. Stage 2 (the whole device): k_gs_ptr_init gives every
+// reached pixel the pair (parent, -step2pi(phi - phi_parent)), the parent being the first neighbour of the previous
+// level in the order right, left, below, above, and k_gs_ptr_jump contracts the parent chains by pointer jumping,
+// (ptr, sum) <- (ptr[ptr], sum + sum[ptr]), until each pointer is the start pixel, whose pair is (itself, 0). Then sum
 // is the pixel's 2 pi count: the same integers k_gs_bfs adds level by level, in another order (integer
-// sums do not depend on it). Unreached pixels keep ptr = -1. Parent codes: 0 unreached, 1..4 right, left,
-// below, above, 5 the start pixel.
+// sums do not depend on it). Unreached pixels keep ptr = -1.
 //
 // The search keeps one bit per pixel in LDS, set for cut pixels and for visited ones, so that an atomic
 // OR claims a pixel (the returned word tells whether it was still free; a level is one pass and one
@@ -625,8 +862,10 @@ __device__ __forceinline__ bool tbit(const unsigned* b, long long p) { return (b
 // pixel, the same whatever order the search claims pixels in.
 __global__ __launch_bounds__(1024) void k_gs_bfs_lev(const uint8_t* __restrict__ cuts, int H, int W, int Q,
                                                      int* __restrict__ level, int* __restrict__ qa,
-                                                     int* __restrict__ qb, int* __restrict__ maxdepth)
+                                                     int* __restrict__ qb, int* __restrict__ maxdepth,
+                                                     const int* __restrict__ flag)
 {
+    if (!flag[blockIdx.x]) return;
     extern __shared__ unsigned sm[];
     __shared__ int cnt[3];  // entries of levels d, d + 1, d + 2 (mod 3)
     const long long n = (long long)H * W;
@@ -634,7 +873,8 @@ __global__ __launch_bounds__(1024) void k_gs_bfs_lev(const uint8_t* __restrict__
     unsigned* blk = sm;  // cut or visited
     int* lq[2] = {reinterpret_cast<int*>(sm + nb), reinterpret_cast<int*>(sm + nb) + Q};
     const uint8_t* cut = cuts + blockIdx.x * n;
-    int* lev = level + blockIdx.x * n;  // all -1 (unreached) on entry
+    int* lev = level + blockIdx.x * n;
+    for (long long p = threadIdx.x; p < n; p += blockDim.x) lev[p] = -1;  // unreached
     int* gq[2] = {qa + blockIdx.x * n, qb + blockIdx.x * n};
     auto qget = [&](int which, int i) -> int { return i < Q ? lq[which][i] : ld_wg(gq[which] + i); };
     auto qput = [&](int which, int i, int v) {
@@ -688,62 +928,37 @@ __global__ __launch_bounds__(1024) void k_gs_bfs_lev(const uint8_t* __restrict__
     if (threadIdx.x == 0 && d > 1) atomicMax(maxdepth, d - 1);  // longest parent chain of the map
 }
 
-// Parent codes from the levels of k_gs_bfs_lev: a reached pixel of level d + 1 takes its first neighbour
-// of level d in the order right, left, below, above (cut and unreached pixels have level -1); the start
-// pixel (level 0) gets 5, unreached pixels 0.
-__global__ void k_gs_par_lev(const int* __restrict__ level, int batch, int H, int W, uint8_t* __restrict__ par)
+// Pair (ptr, sum) per pixel of a flagged map from its levels, map-local ptr: a reached pixel of level d + 1 points to
+// its first neighbour of level d in the order right, left, below, above (cut and unreached pixels have level -1), the
+// start pixel (level 0) to itself.
+__global__ __launch_bounds__(256) void k_gs_ptr_init(const float* __restrict__ phi, const int* __restrict__ level, int H,
+                                                     int W, unsigned long long* __restrict__ pr,
+                                                     const int* __restrict__ flag)
 {
+    const int b = blockIdx.y;
+    if (!flag[b]) return;
     const long long n = (long long)H * W;
-    int x, y;
-    long long b;
-    pixel_of_grid(W, x, y, b);
-    if (x >= W) return;
-    const int p = x + W * y;
-    const long long g = b * n + p;
     const int* lev = level + b * n;
-    const int d = lev[p];
-    uint8_t code = 0;
-    if (d == 0) {
-        code = 5;
-    } else if (d > 0) {
-        if (x + 1 < W && lev[p + 1] == d - 1)
-            code = 1;
-        else if (x > 0 && lev[p - 1] == d - 1)
-            code = 2;
-        else if (y + 1 < H && lev[p + W] == d - 1)
-            code = 3;
-        else if (y > 0 && lev[p - W] == d - 1)
-            code = 4;
+    const float* ph = phi + b * n;
+    for (long long p = (long long)blockIdx.x * 256 + threadIdx.x; p < n; p += (long long)gridDim.x * 256) {
+        const int x = (int)(p % W), y = (int)(p / W), d = lev[p];
+        unsigned long long v = gs_pack(-1, 0);
+        if (d == 0) {
+            v = gs_pack((int)p, 0);
+        } else if (d > 0) {
+            long long pp = -1;
+            if (x + 1 < W && lev[p + 1] == d - 1)
+                pp = p + 1;
+            else if (x > 0 && lev[p - 1] == d - 1)
+                pp = p - 1;
+            else if (y + 1 < H && lev[p + W] == d - 1)
+                pp = p + W;
+            else if (y > 0 && lev[p - W] == d - 1)
+                pp = p - W;
+            v = gs_pack((int)pp, 0u - (unsigned)gs_step2pi(__fsub_rn(ph[p], ph[pp])));
+        }
+        pr[b * n + p] = v;
     }
-    par[g] = code;
-}
-
-__global__ void k_gs_fill_i32(int* __restrict__ p, long long n, int v)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-// Pair (ptr, sum) per pixel, map-local ptr; the start pixel points to itself.
-__global__ void k_gs_ptr_init(const float* __restrict__ phi, const uint8_t* __restrict__ par, int batch, int H,
-                              int W, int2* __restrict__ pr)
-{
-    const long long n = (long long)H * W;
-    int x, y;
-    long long b;
-    pixel_of_grid(W, x, y, b);
-    if (x >= W) return;
-    const int p = x + W * y;
-    const long long g = b * n + p;
-    const int code = par[g];
-    int2 v = make_int2(-1, 0);
-    if (code == 5) {
-        v = make_int2(p, 0);
-    } else if (code >= 1 && code <= 4) {
-        const int pp = p + (code == 1 ? 1 : code == 2 ? -1 : code == 3 ? W : -W);
-        v = make_int2(pp, -gs_step2pi(__fsub_rn(phi[g], phi[b * n + pp])));
-    }
-    pr[g] = v;
 }
 
 // Pointer jumping, in place: each pixel follows its pointer GS_HOPS times, reading the pairs as they are,
@@ -753,14 +968,14 @@ __global__ void k_gs_ptr_init(const float* __restrict__ phi, const uint8_t* __re
 // at least GS_HOPS + 1 (the pairs read within it may be older than the launch's own updates), so launch
 // `step` is needed only while (GS_HOPS + 1)^step is below the longest chain (maxdepth, from the search);
 // later launches return at once.
-constexpr int GS_HOPS = 3;
-__global__ __launch_bounds__(256) void k_gs_ptr_jump(int2* __restrict__ pr, long long n, int step,
-                                                     const int* __restrict__ maxdepth)
+constexpr int GS_HOPS = 15;
+__global__ __launch_bounds__(256) void k_gs_ptr_jump(unsigned long long* __restrict__ a, long long n, int step,
+                                                     const int* __restrict__ maxdepth, const int* __restrict__ flag)
 {
+    if (!flag[blockIdx.y]) return;
     long long reach = 1;
     for (int i = 0; i < step; ++i) reach *= GS_HOPS + 1;
     if (reach >= (long long)*maxdepth) return;
-    unsigned long long* a = reinterpret_cast<unsigned long long*>(pr);
     const long long base = (long long)blockIdx.y * n;  // the grid's y is the map
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         const long long g = base + i;
@@ -780,11 +995,12 @@ __global__ __launch_bounds__(256) void k_gs_ptr_jump(int2* __restrict__ pr, long
 }
 
 // ---------------------------------------------------------------- 4. cut fill + outputs
-// k of a pixel: from the fill's int32 counts, or (PTR) from the contracted pairs (ptr < 0: unreached).
+// k of a pixel: from the fill's int32 counts, or (PTR) from the pairs. A flagged map's are contracted (ptr < 0:
+// unreached), the others' lead to the map's root in two steps at most.
 template <bool PTR>
 __global__ void k_gs_finish(const float* __restrict__ phi, const uint8_t* __restrict__ cuts, const int* __restrict__ kk,
-                            const int2* __restrict__ pr, int batch, int H, int W, int* __restrict__ kout,
-                            float* __restrict__ unwrapped)
+                            const int2* __restrict__ pr, const int2* __restrict__ start, const int* __restrict__ flag,
+                            int H, int W, int* __restrict__ kout, float* __restrict__ unwrapped)
 {
     const long long n = (long long)H * W;
     int x, y;
@@ -795,35 +1011,40 @@ __global__ void k_gs_finish(const float* __restrict__ phi, const uint8_t* __rest
     const long long g = b * n + p;
     const uint8_t* cut = cuts + b * n;
     const float* ph = phi + b * n;
-    auto kat = [&](int q) -> int {
+    const int2 anchor = PTR ? start[b] : make_int2(0, 0);
+    const bool searched = PTR ? flag[b] != 0 : false;
+    // k of four pixels, or fewer (q < 0: none, INT_MIN): every load of a level is under way before the next level's
+    auto kat = [&](const int (&q)[4], int (&kv)[4]) {
         if constexpr (PTR) {
-            const int2 v = pr[b * n + q];
-            return v.x < 0 ? INT_MIN : v.y;
+            int2 v[4], u[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) v[t] = q[t] >= 0 ? pr[b * n + q[t]] : make_int2(-1, 0);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) u[t] = v[t].x >= 0 && !searched ? pr[b * n + v[t].x] : make_int2(anchor.x, anchor.y);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                kv[t] = v[t].x >= 0 && u[t].x == anchor.x ? (int)((unsigned)v[t].y + (unsigned)u[t].y - (unsigned)anchor.y) : INT_MIN;
         } else {
-            return kk[b * n + q];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) kv[t] = q[t] >= 0 ? kk[b * n + q[t]] : INT_MIN;
         }
     };
-    int kv = kat(p);
-    if (cut[p] && x > 0 && x < W - 1 && y > 0 && y < H - 1 &&
-        !(cut[p + 1] && cut[p - 1] && cut[p + W] && cut[p - W])) {
+    const bool is_cut = cut[p];
+    int own[4] = {p, -1, -1, -1}, kp[4];
+    kat(own, kp);
+    int kv = kp[0];
+    if (is_cut && x > 0 && x < W - 1 && y > 0 && y < H - 1) {
         const int nb[4] = {p + 1, p - 1, p + W, p - W};
-        for (int t = 0; t < 4; ++t) {
-            const int q = nb[t];
-            const int kq = kat(q);
-            if (!cut[q] && kq != INT_MIN) {  // reached by the fill
-                kv = kq - gs_step2pi(__fsub_rn(ph[p], ph[q]));
-                break;
-            }
-        }
+        int q[4], kq[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) q[t] = cut[nb[t]] ? -1 : nb[t];
+        kat(q, kq);
+#pragma unroll
+        for (int t = 3; t >= 0; --t)  // the first one that the fill reached
+            if (kq[t] != INT_MIN) kv = kq[t] - gs_step2pi(__fsub_rn(ph[p], ph[nb[t]]));
     }
     if (kout) kout[g] = kv;
     unwrapped[g] = kv == INT_MIN ? 0.f : __fadd_rn(ph[p], __fmul_rn((float)kv, kTWO_PI_F));
-}
-
-__global__ void k_gs_fill_u8(uint8_t* __restrict__ p, long long n)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
 }
 
 void goldstein(Ctx& c, const float* wrapped, int batch, int H, int W, int8_t* res, uint8_t* cuts, int32_t* k2pi,
@@ -847,52 +1068,64 @@ void goldstein(Ctx& c, const float* wrapped, int batch, int H, int W, int8_t* re
     const size_t words = 2 * ((size_t)nw + 3) * sizeof(unsigned);  // the charges' two bit arrays
     int* npairs = (int*)c.buf("gs.npairs", sizeof(int) * (size_t)batch * H);
     int2* pairs = (int2*)c.buf("gs.pairs", sizeof(int2) * (size_t)tot);
+    int* flag = (int*)c.buf("gs.flag", sizeof(int) * ((size_t)batch + 1));
+    int* maxd = flag + batch;
     if (words + 4096 <= lds_max) {  // beside the kernel's own 3 KiB
         hipLaunchKernelGGL(k_gs_pair<true>, dim3(batch), dim3(64 * GS_WAVES), words, c.stream, r, H, W, nullptr,
-                           pairs, npairs);
+                           pairs, npairs, flag);
     } else {
         unsigned* gw = (unsigned*)c.buf("gs.words", words * batch);
         hipLaunchKernelGGL(k_gs_pair<false>, dim3(batch), dim3(64 * GS_WAVES), 0, c.stream, r, H, W, gw, pairs,
-                           npairs);
+                           npairs, flag);
     }
     CTDM_CHECK_LAUNCH("k_gs_pair");
     hipLaunchKernelGGL(k_gs_draw, pgrid, dim3(256), 0, c.stream, pairs, npairs, H, W, ct);
     CTDM_CHECK_LAUNCH("k_gs_draw");
     const size_t bits = sizeof(unsigned) * (size_t)nb;  // cut-or-visited bits
+    const bool searchable = bits + 64 + 2 * sizeof(int) * 256 <= lds_max && W < 65536 && H < 65536;
     // the queues get what LDS has left (>= 256 each); their entries pack x and y in 16 bits each
-    if (bits + 64 + 2 * sizeof(int) * 256 <= lds_max && W < 65536 && H < 65536) {
-        // two-stage fill: levels by the search and parent directions from them, 2 pi counts by pointer jumping
-        const int Q = (int)std::min<long long>(n, (long long)((lds_max - 64 - bits) / (2 * sizeof(int))));
-        uint8_t* par = (uint8_t*)c.buf("gs.par", (size_t)tot);
-        int2* pr = (int2*)c.buf("gs.pr", sizeof(int2) * (size_t)tot);
-        int* maxd = (int*)c.buf("gs.maxd", sizeof(int));
+    if (searchable) {
+        unsigned long long* pr = (unsigned long long*)c.buf("gs.pr", sizeof(unsigned long long) * (size_t)tot);
+        unsigned long long* start = (unsigned long long*)c.buf("gs.start", sizeof(unsigned long long) * (size_t)batch);
         int* lev = (int*)c.buf("gs.level", sizeof(int) * tot);
-        hipLaunchKernelGGL(k_gs_fill_u8, dim3(1), dim3(256), 0, c.stream, (uint8_t*)maxd, (long long)sizeof(int));
-        hipLaunchKernelGGL(k_gs_fill_i32, dim3(grid1d(tot, 256)), dim3(256), 0, c.stream, lev, tot, -1);
+        hipLaunchKernelGGL(k_gs_tile, dim3((unsigned)((W + GS_TX - 1) / GS_TX), (unsigned)((H + GS_TY - 1) / GS_TY), (unsigned)batch),
+                           dim3(512), 0, c.stream, wrapped, ct, H, W, pr, flag);
+        CTDM_CHECK_LAUNCH("k_gs_tile");
+        const long long edges = (long long)((W - 1) / GS_TX) * H + (long long)((H - 1) / GS_TY) * W;
+        if (edges) {
+            hipLaunchKernelGGL(k_gs_merge, dim3((unsigned)grid1d(edges, 256), (unsigned)batch), dim3(256), 0, c.stream,
+                               wrapped, ct, H, W, pr);
+            CTDM_CHECK_LAUNCH("k_gs_merge");
+        }
+        hipLaunchKernelGGL(k_gs_anchor, dim3((unsigned)(edges ? grid1d(edges, 256) : 0) + 1, (unsigned)batch), dim3(256), 0,
+                           c.stream, wrapped, ct, H, W, pr, start, flag);
+        CTDM_CHECK_LAUNCH("k_gs_anchor");
+        // the search, for flagged maps: levels, parents from them, 2 pi counts by pointer jumping
+        const int Q = (int)std::min<long long>(n, (long long)((lds_max - 64 - bits) / (2 * sizeof(int))));
         hipLaunchKernelGGL(k_gs_bfs_lev, dim3(batch), dim3(1024), bits + 2 * sizeof(int) * (size_t)Q, c.stream, ct,
-                           H, W, Q, lev, qa, qb, maxd);
+                           H, W, Q, lev, qa, qb, maxd, (const int*)flag);
         CTDM_CHECK_LAUNCH("k_gs_bfs_lev");
-        hipLaunchKernelGGL(k_gs_par_lev, pgrid, dim3(256), 0, c.stream, lev, batch, H, W, par);
-        hipLaunchKernelGGL(k_gs_ptr_init, pgrid, dim3(256), 0, c.stream, wrapped, par, batch, H, W, pr);
+        // about 8 workgroups per CU in all, split over the maps (the grid's y), but 128 for the one map of many that
+        // may be flagged
+        const long long per_map = std::max<long long>(128, (long long)std::max(c.cus, 1) * 8 / batch);
+        const dim3 jg((unsigned)std::min<long long>(grid1d(n, 256), per_map), (unsigned)batch);
+        hipLaunchKernelGGL(k_gs_ptr_init, jg, dim3(256), 0, c.stream, wrapped, lev, H, W, pr, (const int*)flag);
         // enough launches for any chain in a map ((GS_HOPS + 1)^launches >= n); launches past the longest
         // chain return at once
         int launches = 0;
         for (long long reach = 1; reach < n; reach *= GS_HOPS + 1) ++launches;
-        // about 8 workgroups per CU in all, split over the maps (the grid's y)
-        const long long per_map = std::max<long long>(1, (long long)std::max(c.cus, 1) * 8 / batch);
-        const dim3 jg((unsigned)std::min<long long>(grid1d(n, 256), per_map), (unsigned)batch);
         for (int r = 0; r < launches; ++r)
-            hipLaunchKernelGGL(k_gs_ptr_jump, jg, dim3(256), 0, c.stream, pr, n, r, (const int*)maxd);
+            hipLaunchKernelGGL(k_gs_ptr_jump, jg, dim3(256), 0, c.stream, pr, n, r, (const int*)maxd, (const int*)flag);
         CTDM_CHECK_LAUNCH("k_gs_ptr_jump");
-        hipLaunchKernelGGL(k_gs_finish<true>, pgrid, dim3(256), 0, c.stream, wrapped, ct, nullptr, pr, batch, H, W,
-                           k2pi, unwrapped);
+        hipLaunchKernelGGL(k_gs_finish<true>, pgrid, dim3(256), 0, c.stream, wrapped, ct, nullptr, (const int2*)pr,
+                           (const int2*)start, (const int*)flag, H, W, k2pi, unwrapped);
     } else {
         int* kk = (int*)c.buf("gs.k", sizeof(int) * tot);
         int* lev = (int*)c.buf("gs.level", sizeof(int) * tot);
         hipLaunchKernelGGL(k_gs_bfs, dim3(batch), dim3(1024), 0, c.stream, wrapped, ct, H, W, lev, kk, qa, qb);
         CTDM_CHECK_LAUNCH("k_gs_bfs");
-        hipLaunchKernelGGL(k_gs_finish<false>, pgrid, dim3(256), 0, c.stream, wrapped, ct, kk, nullptr, batch, H, W,
-                           k2pi, unwrapped);
+        hipLaunchKernelGGL(k_gs_finish<false>, pgrid, dim3(256), 0, c.stream, wrapped, ct, kk, nullptr, nullptr,
+                           nullptr, H, W, k2pi, unwrapped);
     }
     CTDM_CHECK_LAUNCH("k_gs_finish");
 }
