@@ -107,3 +107,17 @@ def test_projection_over_its_branches(ctx):
         e[0, 0, 1:3] = 0  # at the cut itself the sign of a zero decides
         print(f"max|dn| {e.max():.1e}")
         assert e.max() <= 6e-6
+
+
+@pytest.mark.parametrize("V,fill", [(32, 0.0), (32, 1.0), (64, 0.1), (192, 0.3)])
+def test_measured_list_by_value(ctx, V, fill):
+    """The list of CTDM_DC_REFCOMPAT: voxels whose real and imaginary parts both differ from zero, some with one zero part;
+    one iteration against the loop in double precision (tolerance as above)."""
+    f, Fm, mask, k2 = case(V, 7 + V, fill)
+    Fm[:, :, ::7] = 1j * Fm[:, :, ::7].imag
+    Fm[:, ::5] = Fm[:, ::5].real
+    mask = (Fm.real != 0) & (Fm.imag != 0)
+    want = loop(f.astype(np.complex128), Fm.astype(np.complex128), mask, 1, k2)
+    n = ctx.positivity(cuda(f), cuda(Fm), None, 1, ctdm_amd.Optics(LAM, NM, 0.1e-6),
+                       ctdm_amd.POS_NO_SHIFT | ctdm_amd.DC_REFCOMPAT)
+    assert float(np.abs(n.cpu().numpy() - want).max()) <= TOL
