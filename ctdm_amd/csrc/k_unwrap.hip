@@ -137,32 +137,14 @@ __device__ __forceinline__ float2 dct3_pair(const float2* s, int k, float2 w)
 // ---------------------------------------------------------------- 1. RHS + DCT-II along x
 enum : int { RHS_WRAP = 0, RHS_SIN = 1, RHS_NONE = 2 };  // RHS of a wrapped map, or the input as it is (adjoint)
 
-// A workgroup's 2 GP rows lie in one map. First each thread forms the right-hand side of blocks of 4 x 4 or 4 x 2 pixels
-// straight from the map (every difference within the block once: 2.5 or 2.75 per pixel instead of the 4 of the
-// stencil) and puts two rows of it as one complex line in Makhoul order; then the lines
-// are transformed. Bound by the chain load - differences - transform of one round of workgroups. 60 maps of
-// 256^2: 13.4 us, one map 7.3 us; 26.2 and 15.4 us when each thread evaluated the whole stencil for the 16 pixels
-// of its transform, with a division in each difference, in 80 KiB of unrolled code.
-template <int N, int RHS>
-__global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_fwd(const float* __restrict__ in,
-                                                            const float2* __restrict__ tw_n,
-                                                            const float2* __restrict__ tw_4n, float* __restrict__ out)
+// Rows y0 .. y0 + GR - 1 of a map's right-hand side as GR / 2 complex lines in Makhoul order, by NT threads: each forms
+// blocks of 4 x 4 or 4 x 2 pixels straight from the map (every difference within the block once: 2.5 or 2.75 per pixel
+// instead of the 4 of the stencil).
+template <int N, int RHS, int GR, int NT>
+__device__ __forceinline__ void rhs_lines(const float* __restrict__ map, int y0, float2* lds)
 {
-    using PR = Pair<N>;
-    constexpr int T = PR::T, GP = PR::GP, NT = PR::NT, GR = 2 * GP, Q = N / 4;
-    constexpr int CR = Q * GR / 4 >= NT ? 4 : 2;  // rows of a thread's block
+    constexpr int Q = N / 4, CR = Q * GR / 4 >= NT ? 4 : 2;  // CR: rows of a thread's block
     static_assert(N % GR == 0 && GR % CR == 0, "a workgroup's rows lie in one map");
-    __shared__ float2 lds[GP * LdsSize<N>::value];
-    __shared__ float2 twl[LdsSize<N>::value];
-    TwStager<N, NT> tws;
-    tws.fetch(tw_n);
-    const int g = threadIdx.x / T, t = threadIdx.x % T;
-    const long long row0 = (long long)blockIdx.x * GR;
-    const int y0 = (int)(row0 % N);
-    const float* map = in + (row0 - y0) * N;
-    float2 w[PR::J];
-#pragma unroll
-    for (int j = 0; j < PR::J; ++j) w[j] = tw_4n[t + j * T];
     for (int e = threadIdx.x; e < Q * (GR / CR); e += NT) {
         const int x = 4 * (e % Q), r = CR * (e / Q), y = y0 + r;
         const float* p = map + (long long)y * N + x;
@@ -216,6 +198,30 @@ __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_fwd(const float* __rest
                 lds[(r / 2 + h) * LdsSize<N>::value + lds_pad(mk_pos(x + i, N))] =
                     make_float2(rho[2 * h][i], rho[2 * h + 1][i]);
     }
+}
+
+// A workgroup's 2 GP rows lie in one map: their right-hand side as complex lines of two rows, then the transforms. Bound by the chain load - differences - transform of one round of workgroups. 60 maps of
+// 256^2: 13.4 us, one map 7.3 us; 26.2 and 15.4 us when each thread evaluated the whole stencil for the 16 pixels
+// of its transform, with a division in each difference, in 80 KiB of unrolled code.
+template <int N, int RHS>
+__global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_fwd(const float* __restrict__ in,
+                                                            const float2* __restrict__ tw_n,
+                                                            const float2* __restrict__ tw_4n, float* __restrict__ out)
+{
+    using PR = Pair<N>;
+    constexpr int T = PR::T, GP = PR::GP, NT = PR::NT, GR = 2 * GP;
+    __shared__ float2 lds[GP * LdsSize<N>::value];
+    __shared__ float2 twl[LdsSize<N>::value];
+    TwStager<N, NT> tws;
+    tws.fetch(tw_n);
+    const int g = threadIdx.x / T, t = threadIdx.x % T;
+    const long long row0 = (long long)blockIdx.x * GR;
+    const int y0 = (int)(row0 % N);
+    const float* map = in + (row0 - y0) * N;
+    float2 w[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) w[j] = tw_4n[t + j * T];
+    rhs_lines<N, RHS, GR, NT>(map, y0, lds);
     tws.put(twl);
     const TwPad twp{twl};
     __syncthreads();
@@ -257,6 +263,25 @@ __device__ __forceinline__ void idct_refcompat(int t, const float* X, float2* s,
         if (i < N) put(i, v.x);
     };
     Plan<2 * N>::template run<+1>(t, s, tw_2n, gl, gs);
+}
+
+// Coefficients ky of columns 2c and 2c + 1 over the eigenvalue: a product with the hardware reciprocal (v_rcp_f32,
+// about 1 ulp) of the eigenvalue sum formed in double, two ulps at most, in place of a double division. With `num`
+// (the adjoint) also times the stencil's own eigenvalue.
+__device__ __forceinline__ float2 solve_pair(float2 X, int c, int ky, bool refeig, double e0, double e1, double ey,
+                                             const double* __restrict__ num)
+{
+    const double l0 = refeig ? e0 + ey - 4.0 : -4.0 * (e0 + ey);
+    const double l1 = refeig ? e1 + ey - 4.0 : -4.0 * (e1 + ey);
+    float2 v;
+    v.x = c == 0 && ky == 0 ? 0.f : X.x * __builtin_amdgcn_rcpf((float)l0);
+    v.y = X.y * __builtin_amdgcn_rcpf((float)l1);
+    if (num) {
+        const double n = num[ky];
+        v.x *= (float)(-4.0 * (num[2 * c] + n));
+        v.y *= (float)(-4.0 * (num[2 * c + 1] + n));
+    }
+    return v;
 }
 
 // ---------------------------------------------------------------- 2. columns: DCT-II, / lambda, DCT-III
@@ -308,17 +333,7 @@ __global__ __launch_bounds__(Pair<N>::NC) void k_uw_cols(const float2* __restric
     for (int j = 0; j < PR::J; ++j) {
         const int ky = t + j * T;
         const float2 X = dct2_pair<N>(s, ky, w[j]);
-        const double l0 = refeig ? e0 + ey[j] - 4.0 : -4.0 * (e0 + ey[j]);
-        const double l1 = refeig ? e1 + ey[j] - 4.0 : -4.0 * (e1 + ey[j]);
-        // X / lambda as a product with the hardware reciprocal (v_rcp_f32, about 1 ulp) of the eigenvalue sum
-        // formed in double: two ulps at most, in place of a double division
-        xv[j].x = c == 0 && ky == 0 ? 0.f : X.x * __builtin_amdgcn_rcpf((float)l0);
-        xv[j].y = X.y * __builtin_amdgcn_rcpf((float)l1);
-        if (num) {
-            const double n = num[ky];
-            xv[j].x *= (float)(-4.0 * (num[2 * c] + n));
-            xv[j].y *= (float)(-4.0 * (num[2 * c + 1] + n));
-        }
+        xv[j] = solve_pair(X, c, ky, refeig, e0, e1, ey[j], num);
         if (dc && c == 0 && ky == 0) dc[b] = X.x * (1.f / N);
     }
     __syncthreads();  // every read of the transform's output precedes the coefficients' writes
@@ -524,6 +539,105 @@ __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_inv_rytov(const float* 
     }
 }
 
+// ---------------------------------------------------------------- the three passes in one workgroup
+// A map of 32^2 or 64^2 fits a workgroup: all its row pairs at once, the coefficients as a matrix in LDS, all its column
+// pairs, the row pairs again; the same operations in the same order as the three kernels, and the same bits. For a few
+// maps the three are launches and latency, for many they write and read the coefficients: 1 map of 64^2 12.4 us in
+// three launches, 8.3 in one; 256 17.0 and 9.3; 4096 81 and 62; 32^2 11.8 and 6.5, 30 and 23. One 256^2 hologram pair to an
+// unwrapped 64^2 map 28.8 and 21.8.
+template <int N, int RHS>
+__global__ __launch_bounds__(N / 2 * Pair<N>::T) void k_uw_map(const float* __restrict__ in, const float* __restrict__ wrapped,
+                                                            unsigned flags, const double* __restrict__ eig,
+                                                            const float2* __restrict__ tw_n,
+                                                            const float2* __restrict__ tw_4n, float* __restrict__ out,
+                                                            const double* __restrict__ num, float* __restrict__ dc)
+{
+    using PR = Pair<N>;
+    constexpr int T = PR::T, NT = N / 2 * T, LS = LdsSize<N>::value, MS = N + 2, Q = N / 4;
+    static_assert(64 % T == 0, "a pair's threads lie in one wave");
+    __shared__ float2 lds[N / 2 * LS];
+    __shared__ float2 twl[LS];
+    __shared__ __align__(8) float mat[N * MS];
+    TwStager<N, NT> tws;
+    tws.fetch(tw_n);
+    const int g = threadIdx.x / T, t = threadIdx.x % T;  // a pair of rows (2g, 2g + 1) or of columns
+    const long long base = (long long)blockIdx.x * N * N;
+    float2 w[PR::J];
+    double ey[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) {
+        w[j] = tw_4n[t + j * T];
+        ey[j] = eig[t + j * T];
+    }
+    const double e0 = eig[2 * g], e1 = eig[2 * g + 1];
+    rhs_lines<N, RHS, N, NT>(in + base, 0, lds);
+    tws.put(twl);
+    const TwWave twp{{twl}};
+    __syncthreads();
+    float2* s = lds + g * LS;
+    auto gl = [&](int n) -> float2 { return s[lds_pad(n)]; };
+    auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
+    PR::template run<-1>(t, s, twp, gl, gs);
+    stage_sync(twp);
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) {
+        const int k = t + j * T;
+        const float2 X = dct2_pair<N>(s, k, w[j]);
+        mat[2 * g * MS + k] = X.x;
+        mat[(2 * g + 1) * MS + k] = X.y;
+    }
+    __syncthreads();
+    StageRegs<N, T, PR::R0> x;
+    float2* col = reinterpret_cast<float2*>(mat) + g;  // (a column pair's float2 of row y at y MS / 2)
+#pragma unroll
+    for (int r = 0; r < PR::R0; ++r) x.v[0][r] = col[mk_src(t + r * T, N) * (MS / 2)];
+    PR::template run<-1>(t, s, twp, x, gs);
+    stage_sync(twp);
+    const bool refeig = flags & F_REF_EIG;
+    float2 xv[PR::J];
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) {
+        const int ky = t + j * T;
+        const float2 X = dct2_pair<N>(s, ky, w[j]);
+        xv[j] = solve_pair(X, g, ky, refeig, e0, e1, ey[j], num);
+        if (dc && g == 0 && ky == 0) dc[blockIdx.x] = X.x * (1.f / N);
+    }
+    stage_sync(twp);
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) s[lds_pad(t + j * T)] = xv[j];
+    stage_sync(twp);
+#pragma unroll
+    for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
+    auto gc = [&](int n, float2 v) { col[mk_src(n, N) * (MS / 2)] = cscale(v, 1.f / N); };
+    PR::template run<+1>(t, s, twp, x, gc);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PR::J; ++j) {
+        const int k = t + j * T;
+        s[lds_pad(k)] = make_float2(mat[2 * g * MS + k], mat[(2 * g + 1) * MS + k]);
+    }
+    stage_sync(twp);
+#pragma unroll
+    for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
+    auto gr = [&](int n, float2 v) { s[lds_pad(mk_src(n, N))] = cscale(v, 1.f / N); };
+    PR::template run<+1>(t, s, twp, x, gr);
+    stage_sync(twp);
+    for (int e = t; e < Q; e += T) {  // both rows of the pair, four pixels at a time
+        const int c = 4 * e;
+        const float2 v0 = s[lds_pad(c)], v1 = s[lds_pad(c + 1)], v2 = s[lds_pad(c + 2)], v3 = s[lds_pad(c + 3)];
+        const long long o = base + 2 * g * N + c;
+        float4 a = make_float4(v0.x, v1.x, v2.x, v3.x), b = make_float4(v0.y, v1.y, v2.y, v3.y);
+        if (wrapped) {
+            const float4 wa = *reinterpret_cast<const float4*>(wrapped + o);
+            const float4 wb = *reinterpret_cast<const float4*>(wrapped + o + N);
+            a = make_float4(congruent(a.x, wa.x), congruent(a.y, wa.y), congruent(a.z, wa.z), congruent(a.w, wa.w));
+            b = make_float4(congruent(b.x, wb.x), congruent(b.y, wb.y), congruent(b.z, wb.z), congruent(b.w, wb.w));
+        }
+        *reinterpret_cast<float4*>(out + o) = a;
+        *reinterpret_cast<float4*>(out + o + N) = b;
+    }
+}
+
 // Adjoint of the right-hand side at a solution v = P g: the zero-flux stencil sum_nbr w_pn (v_n - v_p) with
 // weights cos(phi_n - phi_p). With `g` and `mean` (P exact) the unweighted part is known, as the stencil undoes
 // P up to the mean, and only sum (cos - 1) (v_n - v_p) is taken from v: v is smooth and large where g is rough,
@@ -711,7 +825,7 @@ static void run_rows_inv(Ctx& c, const float* in, int batch, unsigned flags, con
         constexpr int G = 256 / Plan<2 * N>::T;
         hipLaunchKernelGGL((k_uw_rows_inv_ref<N, G>), dim3(grid1d((long long)batch * N, G)), dim3(G * Plan<2 * N>::T),
                            0, c.stream, in, batch, wrapped, c.tw(2 * N), c.tw(4 * N), out);
-    } else {
+    } else if constexpr (N > 64) {  // (smaller maps: k_uw_map)
         using PR = Pair<N>;
         hipLaunchKernelGGL((k_uw_rows_inv<N>), dim3((unsigned)((long long)batch * N / (2 * PR::GP))), dim3(PR::NT), 0,
                            c.stream, in, wrapped, c.tw(N), c.tw(4 * N), out);
@@ -734,6 +848,25 @@ template <int N>
 static void solve(Ctx& c, const float* in, int batch, unsigned flags, int mode, const float* wrapped,
                   float* out, Work w)
 {
+    if constexpr (N <= 64) {
+        if (!(flags & F_REF_IDCT)) {  // (the reference's IDCT has its own kernels)
+            const double* eig = eig_table(c, N, flags & F_REF_EIG, w.existing);
+            const dim3 grid(batch), block(N / 2 * Pair<N>::T);
+            const float* cong = flags & F_CONGRUENT ? wrapped : nullptr;
+            const float2 *tw = c.tw(N), *tw4 = c.tw(4 * N);
+            if (mode == 1)
+                hipLaunchKernelGGL((k_uw_map<N, RHS_NONE>), grid, block, 0, c.stream, in, cong, flags, eig, tw, tw4, out,
+                                   w.num, w.dc);
+            else if (flags & F_SINCOS)
+                hipLaunchKernelGGL((k_uw_map<N, RHS_SIN>), grid, block, 0, c.stream, in, cong, flags, eig, tw, tw4, out,
+                                   w.num, w.dc);
+            else
+                hipLaunchKernelGGL((k_uw_map<N, RHS_WRAP>), grid, block, 0, c.stream, in, cong, flags, eig, tw, tw4, out,
+                                   w.num, w.dc);
+            CTDM_CHECK_LAUNCH("k_uw_map");
+            return;
+        }
+    }
     if (!w.D1) {
         w.D1 = (float*)c.buf("uw.D1", sizeof(float) * (size_t)batch * N * N);
         w.D2 = (float*)c.buf("uw.D2", sizeof(float) * (size_t)batch * N * N);
