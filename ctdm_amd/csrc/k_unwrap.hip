@@ -107,7 +107,7 @@ struct Pair<128> : PairOf<128, 32, 8, 4, 4, 8> {};
 template <>
 struct Pair<192> : PairOf<192, 24, 8, 8, 8, 3> {};
 template <>
-struct Pair<256> : PairOf<256, 32, 8, 8, 8, 4> {};
+struct Pair<256> : PairOf<256, 64, 2, 4, 4, 4, 4> {};  // one map 38.2 us from hologram to phase with 32 threads and 8 pairs, 34.2
 
 // The DCT-II coefficients k of two lines a, b from Z = FFT(v_a + i v_b): V_a = (Z[k] + conj Z[-k]) / 2,
 // V_b = (Z[k] - conj Z[-k]) / 2i, X = s Re(w V) with w = exp(-i pi k / 2N).
@@ -200,8 +200,9 @@ __device__ __forceinline__ void rhs_lines(const float* __restrict__ map, int y0,
     }
 }
 
-// A workgroup's 2 GP rows lie in one map: their right-hand side as complex lines of two rows, then the transforms. Bound by the chain load - differences - transform of one round of workgroups. 60 maps of
-// 256^2: 13.4 us, one map 7.3 us; 26.2 and 15.4 us when each thread evaluated the whole stencil for the 16 pixels
+// A workgroup's 2 GP rows lie in one map: their right-hand side as complex lines of two rows, then the transforms.
+// Bound by the chain load - differences - transform of one round of workgroups. 60 maps of
+// 256^2: 12.4 us, one map 5.3 us; 26.2 and 15.4 us when each thread evaluated the whole stencil for the 16 pixels
 // of its transform, with a division in each difference, in 80 KiB of unrolled code.
 template <int N, int RHS>
 __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_fwd(const float* __restrict__ in,
@@ -286,7 +287,8 @@ __device__ __forceinline__ float2 solve_pair(float2 X, int c, int ky, bool refei
 
 // ---------------------------------------------------------------- 2. columns: DCT-II, / lambda, DCT-III
 // C pairs of neighbouring columns per workgroup, one float2 per row of a pair (C * 8 bytes of a row side by
-// side). 60 maps of 256^2: 14.7 us (22.8 with one real column per transform), one map 7.1 us (9.5). The coefficient pairs between the two transforms are held in registers while the area is read, then
+// side). 60 maps of 256^2: 14.3 us (22.8 with one real column per transform), one map 6.4 us (9.5). The
+// coefficient pairs between the two transforms are held in registers while the area is read, then
 // written into it: the DCT-III reads them before its first write. For the adjoint: `num`, the exact sin^2 table,
 // also multiplies by the stencil's own eigenvalue (the Laplacian of the solution, without the stencil), and
 // `dc` receives each map's mean.
