@@ -647,8 +647,9 @@ __global__ __launch_bounds__(B* Plan<V>::T) void k_vol_x(const float2* __restric
 // {y0 + R2 r} of one z plane (pass xy, which transforms those rows along x), the DFTs over y0 within the
 // (x, k1) pencils of all y0 and z (pass zy, which transforms them along z). One iteration reads and writes the
 // volume twice; with a y pass of its own in each direction it was four times. Per iteration, before (x + y + z +
-// y) and now (xy + zy), the streaming copy of the volume in brackets: 256^3 177 and 110 us (38.5), 192^3 92 and 70,
-// 128^3 31 and 26.5, 64^3 17.5 and 8.3.
+// y) and now (xy + zy), the streaming copy of the volume in brackets: 256^3 177 and 107 us (38.5), 192^3 92 and 63,
+// 128^3 31 and 25, 64^3 17.5 and 8.3. On real data the fit's iteration takes 121 us at 256^3 (zy 68: 44 without list and
+// transforms, 61 without the list, 65 without the transforms).
 // Between the passes element (z, y0, k1, x) stands in the row pair of y0 and its neighbour y0 ^ 1, at slot k1:
 //   W[(z V + (y0 & ~1) + R2 k1) V + 2 x + (y0 & 1)],
 // rows that one xy workgroup both reads and writes, so the volume is transformed in place. Pairing two y0 doubles
