@@ -12,13 +12,33 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace ctdm {
+
+// Butterflies take their elements as float2, or as double2 (see Wide).
+template <class V>
+__device__ __forceinline__ V to(float2 a)
+{
+    if constexpr (std::is_same_v<V, float2>)
+        return a;
+    else
+        return make_double2(a.x, a.y);
+}
+__device__ __forceinline__ float2 to_float(float2 a) { return a; }
+__device__ __forceinline__ float2 to_float(double2 a) { return make_float2((float)a.x, (float)a.y); }
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ float2 cmul(float2 a, float2 b)
 {
     return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ double2 cmul(double2 a, double2 b)
+{
+    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 __device__ __forceinline__ float2 cmulc(float2 a, float2 b)  // a * conj(b)
 {
@@ -32,6 +52,11 @@ template <int DIR>
 __device__ __forceinline__ float2 mul_i(float2 a)
 {
     return DIR > 0 ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
+}
+template <int DIR>
+__device__ __forceinline__ double2 mul_i(double2 a)
+{
+    return DIR > 0 ? make_double2(-a.y, a.x) : make_double2(a.y, -a.x);
 }
 
 // cos / sin of 2*pi*k/32, k = 0..31 (exact to double rounding).
@@ -52,14 +77,16 @@ struct DFT;
 
 template <int DIR>
 struct DFT<1, DIR> {
-    __device__ __forceinline__ static void run(float2*) {}
+    template <class V>
+    __device__ __forceinline__ static void run(V*) {}
 };
 
 template <int DIR>
 struct DFT<2, DIR> {
-    __device__ __forceinline__ static void run(float2* a)
+    template <class V>
+    __device__ __forceinline__ static void run(V* a)
     {
-        const float2 t = a[1];
+        const V t = a[1];
         a[1] = csub(a[0], t);
         a[0] = cadd(a[0], t);
     }
@@ -67,14 +94,19 @@ struct DFT<2, DIR> {
 
 template <int DIR>
 struct DFT<3, DIR> {
-    __device__ __forceinline__ static void run(float2* a)
+    template <class V>
+    __device__ __forceinline__ static void run(V* a)
     {
         // W = exp(DIR*2*pi*i/3) = -1/2 + DIR*i*sqrt(3)/2
-        const float h = 0.86602540378443865f;
-        const float2 t = cadd(a[1], a[2]);
-        const float2 d = csub(a[1], a[2]);
-        const float2 m = make_float2(a[0].x - 0.5f * t.x, a[0].y - 0.5f * t.y);
-        const float2 r = mul_i<DIR>(cscale(d, h));
+        const decltype(a->x) h = 0.86602540378443865, half = 0.5;
+        const V t = cadd(a[1], a[2]);
+        const V d = csub(a[1], a[2]);
+        V m, r;
+        m.x = a[0].x - half * t.x;
+        m.y = a[0].y - half * t.y;
+        r.x = d.x * h;
+        r.y = d.y * h;
+        r = mul_i<DIR>(r);
         a[0] = cadd(a[0], t);
         a[1] = cadd(m, r);
         a[2] = csub(m, r);
@@ -83,12 +115,13 @@ struct DFT<3, DIR> {
 
 template <int DIR>
 struct DFT<4, DIR> {
-    __device__ __forceinline__ static void run(float2* a)
+    template <class V>
+    __device__ __forceinline__ static void run(V* a)
     {
-        const float2 t0 = cadd(a[0], a[2]);
-        const float2 t1 = csub(a[0], a[2]);
-        const float2 t2 = cadd(a[1], a[3]);
-        const float2 t3 = mul_i<DIR>(csub(a[1], a[3]));
+        const V t0 = cadd(a[0], a[2]);
+        const V t1 = csub(a[0], a[2]);
+        const V t2 = cadd(a[1], a[3]);
+        const V t3 = mul_i<DIR>(csub(a[1], a[3]));
         a[0] = cadd(t0, t2);
         a[2] = csub(t0, t2);
         a[1] = cadd(t1, t3);
@@ -101,9 +134,10 @@ struct DFT<4, DIR> {
 // so four-point DFTs over n2 followed by three-point DFTs over n1 give the twelve-point DFT.
 template <int DIR>
 struct DFT<12, DIR> {
-    __device__ __forceinline__ static void run(float2* a)
+    template <class V>
+    __device__ __forceinline__ static void run(V* a)
     {
-        float2 b[3][4];
+        V b[3][4];
 #pragma unroll
         for (int n1 = 0; n1 < 3; ++n1) {
 #pragma unroll
@@ -112,7 +146,7 @@ struct DFT<12, DIR> {
         }
 #pragma unroll
         for (int k2 = 0; k2 < 4; ++k2) {
-            float2 c[3] = {b[0][k2], b[1][k2], b[2][k2]};
+            V c[3] = {b[0][k2], b[1][k2], b[2][k2]};
             DFT<3, DIR>::run(c);
 #pragma unroll
             for (int k1 = 0; k1 < 3; ++k1) a[(4 * k1 + 9 * k2) % 12] = c[k1];
@@ -124,9 +158,10 @@ struct DFT<12, DIR> {
 template <int R, int DIR>
 struct DFT {
     static_assert(R >= 8 && R <= 32 && (R & (R - 1)) == 0, "register DFT supports 2^k <= 32, 3 and 12");
-    __device__ __forceinline__ static void run(float2* a)
+    template <class V>
+    __device__ __forceinline__ static void run(V* a)
     {
-        float2 e[R / 2], o[R / 2];
+        V e[R / 2], o[R / 2];
 #pragma unroll
         for (int k = 0; k < R / 2; ++k) {
             e[k] = a[2 * k];
@@ -136,16 +171,17 @@ struct DFT {
         DFT<R / 2, DIR>::run(o);
 #pragma unroll
         for (int k = 0; k < R / 2; ++k) {
-            float2 t;
+            V t;
             if (k == 0) {
                 t = o[k];
             } else if (4 * k == R) {
                 t = mul_i<DIR>(o[k]);
             } else {
                 const int m = k * (32 / R);
-                const float c = (float)Tw32::c[m];
-                const float s = (float)(DIR * Tw32::c[(m + 24) & 31]);  // sin(x) = cos(x - pi/2)
-                t = cmul(o[k], make_float2(c, s));
+                using S = decltype(t.x);
+                const S c = (S)Tw32::c[m];
+                const S s = (S)(DIR * Tw32::c[(m + 24) & 31]);  // sin(x) = cos(x - pi/2)
+                t = cmul(o[k], V{c, s});
             }
             a[k] = cadd(e[k], t);
             a[k + R / 2] = csub(e[k], t);
@@ -190,6 +226,12 @@ __device__ __forceinline__ void stage_twiddles(float2* dst, const float2* __rest
 struct TwPad {
     const float2* p;
     __device__ __forceinline__ float2 operator[](int m) const { return p[lds_pad(m)]; }
+};
+
+// The table in global memory.
+struct TwTable {
+    const float2* p;
+    __device__ __forceinline__ float2 operator[](int m) const { return p[m]; }
 };
 
 // Twiddle from a per-N table tw[m] = exp(-2*pi*i*m/N) (float2, computed in double on the host): a
@@ -283,6 +325,24 @@ __device__ __forceinline__ void stage_sync(const TwWave&)
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
+// A twiddle table whose transforms compute each stage in double, from and to floats: an exchange rounds an element
+// once, in place of the stage's additions and products each. (FP64 vector operations issue at the rate of unpacked FP32 ones.)
+template <class TW>
+struct Wide : TW {};
+template <class TW>
+__device__ __forceinline__ void stage_sync(const Wide<TW>& tw)
+{
+    stage_sync(static_cast<const TW&>(tw));
+}
+template <class TW>
+struct StageVec {
+    using type = float2;
+};
+template <class TW>
+struct StageVec<Wide<TW>> {
+    using type = double2;
+};
+
 // Cooperative N-point transform by T threads of one transform; threads with t >= T only take part
 // in the barriers (so a workgroup sized for a longer transform can run a shorter one).
 // gload(i) supplies input element i (called in the first stage), gstore(i, v) receives output
@@ -304,7 +364,8 @@ struct Stockham {
         if constexpr (REG_IN) static_assert(GLoad::P == P && GLoad::R == R, "register input must match the stage");
         constexpr bool REG_OUT = LAST && IsRegFile<GStore>::value;
         if constexpr (REG_OUT) static_assert(GStore::P == P && GStore::R == R, "register output must match the stage");
-        float2 v[P][R];
+        using V = typename StageVec<TW>::type;
+        V v[P][R];
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const int j = t + p * T;
@@ -316,15 +377,15 @@ struct Stockham {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     if constexpr (REG_IN)
-                        v[p][r] = gload.v[p][r];
+                        v[p][r] = to<V>(gload.v[p][r]);
                     else if constexpr (FIRST)
-                        v[p][r] = gload(j + r * S);
+                        v[p][r] = to<V>(gload(j + r * S));
                     else if constexpr (L == 12 && S == 12)
-                        v[p][r] = sj[13 * r];
+                        v[p][r] = to<V>(sj[13 * r]);
                     else if constexpr (S % 16 == 0 || 16 % S == 0)
-                        v[p][r] = sj[lds_pad(r * S)];
+                        v[p][r] = to<V>(sj[lds_pad(r * S)]);
                     else
-                        v[p][r] = s[lds_pad(j + r * S)];
+                        v[p][r] = to<V>(s[lds_pad(j + r * S)]);
                 }
             }
         }
@@ -337,7 +398,7 @@ struct Stockham {
                 if constexpr (L > 1) {
 #pragma unroll
                     for (int r = 1; r < R; ++r)
-                        v[p][r] = cmul(v[p][r], twiddle<DIR>(tw, r * k * (N / (L * R))));
+                        v[p][r] = cmul(v[p][r], to<V>(twiddle<DIR>(tw, r * k * (N / (L * R)))));
                 }
                 DFT<R, DIR>::run(v[p]);
                 const int base = (j - k) * R + k;
@@ -353,15 +414,15 @@ struct Stockham {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     if constexpr (REG_OUT)
-                        gstore.v[p][r] = v[p][r];
+                        gstore.v[p][r] = to_float(v[p][r]);
                     else if constexpr (LAST)
-                        gstore(base + r * L, v[p][r]);
+                        gstore(base + r * L, to_float(v[p][r]));
                     else if constexpr (WR == 1 || WR == 2)
-                        sb[lds_pad(r * L)] = v[p][r];
+                        sb[lds_pad(r * L)] = to_float(v[p][r]);
                     else if constexpr (WR == 3 || WR == 4)
-                        sb[r * L] = v[p][r];
+                        sb[r * L] = to_float(v[p][r]);
                     else
-                        s[lds_pad(base + r * L)] = v[p][r];
+                        s[lds_pad(base + r * L)] = to_float(v[p][r]);
                 }
             }
         }

@@ -7,7 +7,8 @@
 //           (the trigonometric right-hand side of FastUnwrapping.cu:37-96 on the same stencil)
 //   phi   = IDCT2( DCT2(rho) / lambda ),  lambda_ij = -4 (sin^2(pi i/2N) + sin^2(pi j/2N)), DC := 0
 //           (REFCOMPAT_EIG: 2cos(4 pi i/(4N-1)) + 2cos(4 pi j/(4N-1)) - 4, DCT_Unwrapping.cu:310)
-//   the division is done in FP64 (lambda -> 0 at low frequencies amplifies any rounding).
+//   lambda is formed in FP64 (-> 0 at low frequencies, where any rounding is amplified). The batched path multiplies by
+//   its reciprocal in FP32, rounded once (with the reference's IDCT: the hardware reciprocal); the plain path divides in FP64.
 // Orthonormal DCT-II along a line via one N-point complex FFT (Makhoul reordering):
 //   v[n] = x[2n], v[N-1-n] = x[2n+1];  X[k] = s_k Re(exp(-i pi k / 2N) FFT(v)[k]),
 //   s_0 = sqrt(1/N), s_k = sqrt(2/N).
@@ -109,25 +110,55 @@ struct Pair<192> : PairOf<192, 24, 8, 8, 8, 3> {};
 template <>
 struct Pair<256> : PairOf<256, 64, 2, 4, 4, 4, 4> {};  // one map 38.2 us from hologram to phase with 32 threads and 8 pairs, 34.2
 
-// The DCT-II coefficients k of two lines a, b from Z = FFT(v_a + i v_b): V_a = (Z[k] + conj Z[-k]) / 2,
-// V_b = (Z[k] - conj Z[-k]) / 2i, X = s Re(w V) with w = exp(-i pi k / 2N).
+// Which of a solve's transforms compute their stages in double (Wide). Two lines in one transform take on each other's
+// rounding, and the plans of Pair have more stages than Plan's: the solve's error against 64 bits was 6 to 22 % larger than with
+// one real line per transform. The rows' right-hand side matters most, since 1 / lambda raises what its transform adds to the low
+// frequencies; then the inverse transforms, whose error is the result's. These are as many as bring it below. Mean relative error
+// over 64 maps, in 1e-7, for the wrapped and the sine right-hand side, one line per transform | pairs in floats | now:
+// 64^2 1.82 1.91 | 1.91 2.07 | 1.62 1.75, 128^2 1.75 1.82 | 1.97 2.05 | 1.52 1.69, 192^2 2.13 2.24 | 2.56 2.71 | 2.05 2.12,
+// 256^2 2.88 2.83 | 3.06 3.15 | 2.50 2.58. At 32^2 and 64^2 leaving the factors s_k out is enough. The cost: 60 maps of 256^2
+// 33.8 -> 35.1 us, of 192^2 30.3 -> 32.4, of 128^2 18.6 -> 19.8 (55.5, 39.5 and 22.7 with one line per transform); in
+// double throughout 38.5, 34.2, 20.2.
+template <int N>
+struct InDouble {
+    static constexpr bool rhs = N >= 128, cols_inv = N == 128, rows_inv = N == 128 || N == 192;
+};
+template <bool W, class TW>
+__device__ __forceinline__ auto wide(const TW& tw)
+{
+    if constexpr (W)
+        return Wide<TW>{tw};
+    else
+        return tw;
+}
+
+// The solve's transforms leave the DCT's factors s_k out, which cancel between a DCT-II and its inverse, and scale each
+// forward transform by 1 / DctScale<N> instead: a power of two near N, so that no rounding comes from it and the
+// coefficients keep the magnitude of orthonormal ones. What is left of 1 / N^2 joins the eigenvalue (solve_pair).
+template <int N>
+struct DctScale {
+    static constexpr int value = N == 192 ? 128 : N;
+    static constexpr double rest = (double)N * N / ((double)value * value);  // 1 for a power of two
+};
+
+// The DCT-II coefficients k of two lines a, b, over s_k DctScale<N>, from Z = FFT(v_a + i v_b):
+// V_a = (Z[k] + conj Z[-k]) / 2, V_b = (Z[k] - conj Z[-k]) / 2i, X = s_k Re(w V) with w = exp(-i pi k / 2N).
 template <int N>
 __device__ __forceinline__ float2 dct2_pair(const float2* s, int k, float2 w)
 {
     const float2 z = s[lds_pad(k)], m = s[lds_pad(k == 0 ? 0 : N - k)];
-    const float sc = 0.5f * (k == 0 ? sqrtf(1.f / N) : sqrtf(2.f / N));
+    constexpr float sc = 0.5f / DctScale<N>::value;
     const float ax = z.x + m.x, ay = z.y - m.y, bx = z.y + m.y, by = m.x - z.x;
     return make_float2((ax * w.x - ay * w.y) * sc, (bx * w.x - by * w.y) * sc);
 }
 
 // Element k of the DCT-III's transform input of two lines whose coefficients c = (a, b) stand in s:
-// V_a + i V_b with V = exp(i pi k / 2N) (C_k - i C_{N-k}), C = X / s, C_N = 0.
+// V_a + i V_b with V = exp(i pi k / 2N) (C_k - i C_{N-k}), C_N = 0.
 template <int N>
 __device__ __forceinline__ float2 dct3_pair(const float2* s, int k, float2 w)
 {
-    const float r0 = 1.f / sqrtf(1.f / N), r1 = 1.f / sqrtf(2.f / N);
-    const float2 c = cscale(s[lds_pad(k)], k == 0 ? r0 : r1);
-    const float2 n = k == 0 ? make_float2(0.f, 0.f) : cscale(s[lds_pad(N - k)], r1);
+    const float2 c = s[lds_pad(k)];
+    const float2 n = k == 0 ? make_float2(0.f, 0.f) : s[lds_pad(N - k)];
     // (c - i n) (w.x - i w.y) for each line
     const float ar = c.x * w.x - n.x * w.y, ai = -c.x * w.y - n.x * w.x;
     const float br = c.y * w.x - n.y * w.y, bi = -c.y * w.y - n.y * w.x;
@@ -202,7 +233,7 @@ __device__ __forceinline__ void rhs_lines(const float* __restrict__ map, int y0,
 
 // A workgroup's 2 GP rows lie in one map: their right-hand side as complex lines of two rows, then the transforms.
 // Bound by the chain load - differences - transform of one round of workgroups. 60 maps of
-// 256^2: 12.4 us, one map 5.3 us; 26.2 and 15.4 us when each thread evaluated the whole stencil for the 16 pixels
+// 256^2: 15.2 us (12.5 with its stages in floats), one map 4.9 us; 26.2 and 15.4 us when each thread evaluated the whole stencil for the 16 pixels
 // of its transform, with a division in each difference, in 80 KiB of unrolled code.
 template <int N, int RHS>
 __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_fwd(const float* __restrict__ in,
@@ -229,7 +260,7 @@ __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_fwd(const float* __rest
     float2* s = lds + g * LdsSize<N>::value;
     auto gl = [&](int n) -> float2 { return s[lds_pad(n)]; };
     auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
-    PR::template run<-1>(t, s, twp, gl, gs);
+    PR::template run<-1>(t, s, wide<RHS != RHS_NONE && InDouble<N>::rhs>(twp), gl, gs);
     __syncthreads();
     float* dst = out + (row0 + 2 * g) * N;
 #pragma unroll
@@ -266,17 +297,25 @@ __device__ __forceinline__ void idct_refcompat(int t, const float* X, float2* s,
     Plan<2 * N>::template run<+1>(t, s, tw_2n, gl, gs);
 }
 
-// Coefficients ky of columns 2c and 2c + 1 over the eigenvalue: a product with the hardware reciprocal (v_rcp_f32,
-// about 1 ulp) of the eigenvalue sum formed in double, two ulps at most, in place of a double division. With `num`
-// (the adjoint) also times the stencil's own eigenvalue.
+// 1 / l to one rounding: the hardware reciprocal of l's float and a Newton step on what it and the float leave.
+__device__ __forceinline__ float reciprocal(double l)
+{
+    const float hi = (float)l, lo = (float)(l - (double)hi), r = __builtin_amdgcn_rcpf(hi);
+    return fmaf(r, fmaf(-lo, r, fmaf(-hi, r, 1.f)), r);
+}
+
+// Coefficients ky of columns 2c and 2c + 1 over the eigenvalue, which is formed in double. With `num` (the adjoint)
+// also times the stencil's own eigenvalue.
+template <int N>
 __device__ __forceinline__ float2 solve_pair(float2 X, int c, int ky, bool refeig, double e0, double e1, double ey,
                                              const double* __restrict__ num)
 {
-    const double l0 = refeig ? e0 + ey - 4.0 : -4.0 * (e0 + ey);
-    const double l1 = refeig ? e1 + ey - 4.0 : -4.0 * (e1 + ey);
+    constexpr double F = DctScale<N>::rest;
+    const double l0 = refeig ? F * (e0 + ey - 4.0) : -4.0 * F * (e0 + ey);
+    const double l1 = refeig ? F * (e1 + ey - 4.0) : -4.0 * F * (e1 + ey);
     float2 v;
-    v.x = c == 0 && ky == 0 ? 0.f : X.x * __builtin_amdgcn_rcpf((float)l0);
-    v.y = X.y * __builtin_amdgcn_rcpf((float)l1);
+    v.x = c == 0 && ky == 0 ? 0.f : X.x * reciprocal(l0);
+    v.y = X.y * reciprocal(l1);
     if (num) {
         const double n = num[ky];
         v.x *= (float)(-4.0 * (num[2 * c] + n));
@@ -335,8 +374,8 @@ __global__ __launch_bounds__(Pair<N>::NC) void k_uw_cols(const float2* __restric
     for (int j = 0; j < PR::J; ++j) {
         const int ky = t + j * T;
         const float2 X = dct2_pair<N>(s, ky, w[j]);
-        xv[j] = solve_pair(X, c, ky, refeig, e0, e1, ey[j], num);
-        if (dc && c == 0 && ky == 0) dc[b] = X.x * (1.f / N);
+        xv[j] = solve_pair<N>(X, c, ky, refeig, e0, e1, ey[j], num);
+        if (dc && c == 0 && ky == 0) dc[b] = X.x * (float)(1.0 / DctScale<N>::rest);
     }
     __syncthreads();  // every read of the transform's output precedes the coefficients' writes
 #pragma unroll
@@ -345,8 +384,8 @@ __global__ __launch_bounds__(Pair<N>::NC) void k_uw_cols(const float2* __restric
 #pragma unroll
     for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
     float2* dcol = out + b * N * H + c;
-    auto gs2 = [&](int n, float2 v) { dcol[mk_src(n, N) * H] = cscale(v, 1.f / N); };
-    PR::template run<+1>(t, s, twp, x, gs2);
+    auto gs2 = [&](int n, float2 v) { dcol[mk_src(n, N) * H] = v; };
+    PR::template run<+1>(t, s, wide<InDouble<N>::cols_inv>(twp), x, gs2);
 }
 
 // The same for one column per transform with the reference's 2N-point IDCT.
@@ -373,7 +412,9 @@ __global__ __launch_bounds__(C* Plan<2 * N>::T) void k_uw_cols_ref(const float* 
     auto gs = [&](int i, float2 v) { s[lds_pad(i)] = v; };
     Plan<N>::template run<-1>(t, s, tw_n, gl, gs);
     __syncthreads();
-    const float s0 = sqrtf(1.f / N), s1 = sqrtf(2.f / N);
+    // s_kx s_ky and the rows' scale in one factor
+    constexpr double u = (double)DctScale<N>::value / N, r2 = 1.41421356237309505;
+    const float s0 = (float)(kx == 0 ? u : r2 * u), s1 = (float)(kx == 0 ? r2 * u : 2.0 * u);
     const bool refeig = flags & F_REF_EIG;
     float xv[J];
 #pragma unroll
@@ -444,8 +485,8 @@ __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_inv(const float* __rest
     StageRegs<N, T, PR::R0> x;
 #pragma unroll
     for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
-    auto gs = [&](int n, float2 v) { s[lds_pad(mk_src(n, N))] = cscale(v, 1.f / N); };
-    PR::template run<+1>(t, s, twp, x, gs);
+    auto gs = [&](int n, float2 v) { s[lds_pad(mk_src(n, N))] = v; };
+    PR::template run<+1>(t, s, wide<InDouble<N>::rows_inv>(twp), x, gs);
     __syncthreads();
     for (int e = threadIdx.x; e < Q * GP; e += PR::NT) {
         const int gg = e / Q, c = 4 * (e % Q);
@@ -516,7 +557,7 @@ __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_inv_rytov(const float* 
     float* pb = reinterpret_cast<float*>(s + LS);
     auto gs = [&](int n, float2 v) {
         const int c = mk_src(n, N);
-        float a = v.x * (1.f / N), b = v.y * (1.f / N);
+        float a = v.x, b = v.y;
         if (wrapped) {
             a = congruent(a, wrapped[ra + c]);
             b = congruent(b, wrapped[ra + N + c]);
@@ -528,7 +569,7 @@ __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_inv_rytov(const float* 
             out[ra + N + c] = b;
         }
     };
-    PR::template run<+1>(t, s, tw_n, x, gs);
+    PR::template run<+1>(t, s, wide<InDouble<N>::rows_inv>(TwTable{tw_n}), x, gs);
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -601,8 +642,8 @@ __global__ __launch_bounds__(N / 2 * Pair<N>::T) void k_uw_map(const float* __re
     for (int j = 0; j < PR::J; ++j) {
         const int ky = t + j * T;
         const float2 X = dct2_pair<N>(s, ky, w[j]);
-        xv[j] = solve_pair(X, g, ky, refeig, e0, e1, ey[j], num);
-        if (dc && g == 0 && ky == 0) dc[blockIdx.x] = X.x * (1.f / N);
+        xv[j] = solve_pair<N>(X, g, ky, refeig, e0, e1, ey[j], num);
+        if (dc && g == 0 && ky == 0) dc[blockIdx.x] = X.x * (float)(1.0 / DctScale<N>::rest);
     }
     stage_sync(twp);
 #pragma unroll
@@ -610,7 +651,7 @@ __global__ __launch_bounds__(N / 2 * Pair<N>::T) void k_uw_map(const float* __re
     stage_sync(twp);
 #pragma unroll
     for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
-    auto gc = [&](int n, float2 v) { col[mk_src(n, N) * (MS / 2)] = cscale(v, 1.f / N); };
+    auto gc = [&](int n, float2 v) { col[mk_src(n, N) * (MS / 2)] = v; };
     PR::template run<+1>(t, s, twp, x, gc);
     __syncthreads();
 #pragma unroll
@@ -621,7 +662,7 @@ __global__ __launch_bounds__(N / 2 * Pair<N>::T) void k_uw_map(const float* __re
     stage_sync(twp);
 #pragma unroll
     for (int r = 0; r < PR::R0; ++r) x.v[0][r] = dct3_pair<N>(s, t + r * T, w[r]);
-    auto gr = [&](int n, float2 v) { s[lds_pad(mk_src(n, N))] = cscale(v, 1.f / N); };
+    auto gr = [&](int n, float2 v) { s[lds_pad(mk_src(n, N))] = v; };
     PR::template run<+1>(t, s, twp, x, gr);
     stage_sync(twp);
     for (int e = t; e < Q; e += T) {  // both rows of the pair, four pixels at a time
