@@ -6,8 +6,8 @@
 //                     double promotions, summed in float, thresholded at +-6.
 //   2. branch cuts, deterministic raster order (the reference runs its search for all residues
 //      concurrently, which is racy; the raster order makes it reproducible): k_gs_pair (one workgroup per
-//      map) pairs the residues, with rows side by side where no decision can reach another's, and k_gs_draw
-//      draws the chosen cuts in parallel.
+//      map) pairs the residues, with rows side by side where no decision can reach another's (maps of few
+//      columns: k_gs_walk, one residue after the other), and k_gs_draw draws the chosen cuts in parallel.
 //   3. fill           a pixel's 2 pi count is the sum of the steps along the path by which a level-synchronous
 //                     breadth-first search over non-cut pixels reaches it from a fixed start, each new pixel
 //                     from its first neighbour of the previous level in the order right, left, below,
@@ -152,11 +152,12 @@ __device__ __forceinline__ uint2 charge_bits(const int8_t* __restrict__ m, long 
 // flight. Each group publishes the pixel up to which its row is decided (raster index; a wave's LDS
 // operations execute in order, so removals precede the index that covers them). With c the first column the
 // row above has not published and rho a bound on every reach, a residue at column x takes a hit on ring r
-// once x + r + rho < c, and a row publishes at most c - rho - 1. If every reach is at most rho, its scan then
+// once x + r + rho < c, and a row publishes at most c. If every reach is at most rho, its scan then
 // sees
-//   - every earlier residue's removals: undecided ones lie at columns >= c in the row above and further right
+//   - every earlier residue's removals: undecided ones lie at columns >= c in the row above and no further left
 //     in the rows before, so they change columns >= c - rho only;
-//   - no later residue's: those decided changed columns < x - rho.
+//   - no later residue's: one decided in a row below, at x' on ring r', had x' + r' + rho < c' with c' at most what this row
+//     had published, which is at most x, so it changed columns < x - rho.
 // so all decisions are those of the raster order. A hit beyond rho ends the attempt, and the map starts again
 // with 4 rho, then with R, which no reach exceeds. A small rho keeps the rows close together and more of them
 // in flight; it follows the residue density, as the nearest opposite charges are close where residues are
@@ -164,13 +165,13 @@ __device__ __forceinline__ uint2 charge_bits(const int8_t* __restrict__ m, long 
 // one in 150 000 is 6) and 0.20 (0.7), 10 at 0.10 (0.6, 256^2), 12 at 0.09, 16 at 0.04 (0.55), each ring
 // further 3 to 15 times rarer, so a second attempt stays below one map in a hundred.
 //
-// Bound: the chain of dependent decisions along the front (about 2 300 steps for 512 rows of density 0.28,
-// 13 decisions side by side). In a step a group reads the row above's index, its row's next 31 pixels and the
+// Bound: the chain of dependent decisions along the front (about 1 900 steps for 512 rows of density 0.28,
+// 19 decisions side by side). In a step a group reads the row above's index, its row's next 31 pixels and the
 // opposite charges on rings 1-3 of the pixel it stands on (one LDS round trip), looks the first hit up (another)
 // and removes the pair; the work of a step is done on vectors of rows, one instruction for the eight rows of a
 // wave, since a wavefront alone on its SIMD takes about five cycles per instruction whatever its lanes do.
-// Measured: 64 maps of 512^2 at density 0.28 in 1.0 ms, one 256^2 map at 0.10 in 0.46 ms, against 7.6 and
-// 0.74 ms for one wavefront per map that visited the residues one after the other.
+// Measured: 64 maps of 512^2 at density 0.28 in 0.97 ms, one 256^2 map at 0.09 in 0.40 ms, against 7.1 and
+// 0.60 ms one residue after the other (2c). (With a row publishing c - rho - 1 at most: 1.03 and 0.46 ms.)
 constexpr int GS_LANES = 8;                       // lanes per row: rows -3 .. 3 around it (the last lane idle)
 constexpr int GS_WAVES = 4;                       // wavefronts per map
 constexpr int GS_ROWS = GS_WAVES * 64 / GS_LANES; // rows in flight
@@ -225,10 +226,10 @@ __device__ __forceinline__ void ring_position(int r, int q, int& dx, int& dy)
 // The scan of one residue beyond ring 3 by a whole wavefront, 64 positions of the scan order per round (the
 // first hit is the lowest lane with one). Returns the hit's pixel, -1 for no hit; sets `far` for a hit beyond ring
 // rho, or none up to it. No ring is clipped before the one that touches the border, which holds a hit, so the
-// first round (ring 4 and 32 positions of ring 5, fixed offsets) needs no look at the borders.
-template <bool LDSW>
-__device__ int gs_scan(const Charges<LDSW>& ch, int H, int W, int R, int p, int i, int j, int opp, int lane, int rho,
-                       bool& far)
+// first round (ring 4 and 32 positions of ring 5, fixed offsets) needs no look at the borders. at(q): whether pixel q, at most five
+// rows outside the map, is a hit.
+template <class At>
+__device__ int gs_scan(const At& at, int H, int W, int R, int p, int i, int j, int lane, int rho, bool& far)
 {
     if (R <= 4) return -1;
     int rc = 4, o0 = 0;  // next position: ring rc, index o0
@@ -236,8 +237,7 @@ __device__ int gs_scan(const Charges<LDSW>& ch, int H, int W, int R, int p, int 
         int dx, dy;
         ring_position(lane < 32 ? 4 : 5, lane & 31, dx, dy);
         const int q = p + dx + W * dy;
-        const unsigned wq = min((unsigned)(q >> 5), (unsigned)ch.nw);
-        const unsigned long long hit = __ballot((ch.ld(opp + (int)wq) >> (q & 31)) & 1u);
+        const unsigned long long hit = __ballot(at(q));
         if (hit) {
             const int l = __builtin_ctzll(hit);
             return __builtin_amdgcn_readlane(q, l);
@@ -279,7 +279,7 @@ __device__ int gs_scan(const Charges<LDSW>& ch, int H, int W, int R, int p, int 
             const int nn = left ? n1 + lq : (mid ? ((q2 & 1) ? n2 : n1) : n1 + (q2 - nmid));
             const int q = mm + W * nn;
             c = q;
-            here = (ch.ld(opp + (q >> 5)) >> (q & 31)) & 1u;
+            here = at(q);
         }
         const unsigned long long hit = __ballot(here);
         if (hit) {
@@ -420,9 +420,12 @@ __global__ __launch_bounds__(64 * GS_WAVES) void k_gs_pair(const int8_t* __restr
                 slow &= ~(((1ull << GS_LANES) - 1) << (f & ~(GS_LANES - 1)));
                 bool beyond = false;
                 const int sp = __builtin_amdgcn_readlane(pos, f);
-                const int c = gs_scan(ch, H, W, R, sp, sp - __builtin_amdgcn_readlane(row0, f),
-                                      __builtin_amdgcn_readlane(y, f), __builtin_amdgcn_readlane(opp, f), lane, rho,
-                                      beyond);
+                const int so = __builtin_amdgcn_readlane(opp, f);
+                auto at = [&](int q) -> bool {
+                    return (ch.ld(so + (int)min((unsigned)(q >> 5), (unsigned)nw)) >> (q & 31)) & 1u;
+                };
+                const int c = gs_scan(at, H, W, R, sp, sp - __builtin_amdgcn_readlane(row0, f),
+                                      __builtin_amdgcn_readlane(y, f), lane, rho, beyond);
                 if ((lane ^ f) < GS_LANES) {
                     t = c;
                     const int tx = c % W, ty = c / W;
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(64 * GS_WAVES) void k_gs_pair(const int8_t* __restr
             const int nx = known ? __builtin_ctz(any) : nb;
             qn = (neg >> nx) & 1u;
             pos += nx;
-            pub = pub == GS_LEFT ? GS_LEFT : max(pub, min(pos, lim - rho - 1));
+            pub = pub == GS_LEFT ? GS_LEFT : max(pub, min(pos, lim));
             if (active && all && pos >= hi) {
                 pub = row0 + W;
                 if (l == 0) nrow[y] = np;
@@ -478,6 +481,117 @@ __global__ __launch_bounds__(64 * GS_WAVES) void k_gs_pair(const int8_t* __restr
     }
     for (int y = tid; y < H; y += NT)
         if (nres == 0 || y == 0 || y == H - 1) nrow[y] = 0;
+}
+
+// ---------------------------------------------------------------- 2c. branch cuts: one residue after the other
+// Maps of few columns leave the pipeline no room, since each row stays more than rho columns behind the one above: the
+// search as it is stated, by one wavefront, with a residue's first 64 positions (rings 1-3 and 16 of ring 4) side by side and
+// the rest by gs_scan. The pixels' states stand in LDS in two bits each (1, 2: a present charge of either sign, 3: border),
+// with zeros for five rows before and after, so that one read tells a position's state and no position needs a look at the
+// map's edges (no ring is clipped before the one that touches the border, which holds a hit).
+// Bound by the instructions from one residue to the next, about 90 ns a residue, hence the common case as a loop of its
+// own. Against the pipeline, at noise of 0.6 and 0.8 pi (density 0.09 and 0.28), in us: one map of 4000 x 16 560 and 1619 (2445,
+// 4265), 2000 x 40 734 and 2061 (1924, 2764), 520 x 48 239 and 637 (557, 737), 520 x 64 330 and 869 (515, 780): up to 48
+// columns it is the faster one at every density.
+constexpr int GS_WALK = 48;
+constexpr __host__ __device__ int gs_ahead(int W) { return 5 * (W + 1) / 16 + 2; }
+__device__ __forceinline__ unsigned spread_bits(unsigned v)  // bit b of the low half to bit 2 b
+{
+    v = (v | (v << 8)) & 0x00ff00ffu;
+    v = (v | (v << 4)) & 0x0f0f0f0fu;
+    v = (v | (v << 2)) & 0x33333333u;
+    return (v | (v << 1)) & 0x55555555u;
+}
+
+__global__ __launch_bounds__(256) void k_gs_walk(const int8_t* __restrict__ res, int H, int W, int2* __restrict__ pairs,
+                                                 int* __restrict__ rowpairs, int* __restrict__ flags)
+{
+    extern __shared__ unsigned lwords[];
+    __shared__ int total;
+    const int tid = threadIdx.x, lane = tid & 63, R = min(901, W / 2), ahead = gs_ahead(W);
+    const long long n = (long long)H * W;
+    const int nw = (int)((n + 15) / 16);
+    unsigned* const state = lwords + ahead;
+    const int8_t* r = res + blockIdx.x * n;
+    if (tid == 0) {  // the fill's flag of this map, and behind the last one the longest chain
+        flags[blockIdx.x] = 0;
+        if (blockIdx.x == 0) flags[gridDim.x] = 0;
+    }
+    int2* out = pairs + blockIdx.x * n;
+    for (int w = tid; w < ahead; w += 256) lwords[w] = state[nw + w] = 0;
+    for (int w = tid; w < (nw + 1) / 2; w += 256) {
+        const uint2 b = charge_bits(r, n, w);
+        state[2 * w] = spread_bits(b.x & 0xffffu) | spread_bits(b.y & 0xffffu) << 1;
+        if (2 * w + 1 < nw) state[2 * w + 1] = spread_bits(b.x >> 16) | spread_bits(b.y >> 16) << 1;
+    }
+    __syncthreads();
+    auto border = [&](int p) { atomicOr(state + (p >> 4), 3u << (2 * (p & 15))); };
+    for (int y = tid; y < H; y += 256) {
+        border(y * W);
+        border(y * W + W - 1);
+    }
+    for (int x = tid; x < W; x += 256) {
+        border(x);
+        border((H - 1) * W + x);
+    }
+    __syncthreads();
+    if (tid < 64) {
+        auto ld = [&](int w) { return __hip_atomic_load(state + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+        const int ring = lane < 8 ? 1 : (lane < 24 ? 2 : (lane < 48 ? 3 : 4));
+        int dx, dy;
+        ring_position(ring, lane - (lane < 8 ? 0 : (lane < 24 ? 8 : (lane < 48 ? 24 : 48))), dx, dy);
+        const int off = 2 * (dx + W * dy);  // positions as bit numbers, two a pixel
+        const unsigned in = ring < R ? 3u : 0u;
+        int2* o = out;
+        for (int c = 0; c < nw; c += 64) {
+            const unsigned w = c + lane < nw ? ld(c + lane) : 0u;
+            unsigned m = (w ^ (w >> 1)) & 0x55555555u;  // charges left to visit (at their lower bits)
+            const int base = 32 * (c + lane);
+            int p = 0;  // the residue visited
+            unsigned opp = 0, self = 0;
+            auto settle = [&](int t, bool pair) {  // lane 0 removes the residue, lane 1 the charge that it takes
+                const int gone = pair ? t : p;
+                if (lane < 2) {
+                    const int x = lane ? gone : p;
+                    atomicAnd(state + (x >> 5), ~(3u << (x & 31)));
+                    reinterpret_cast<int*>(o)[lane] = (lane ? t : p) >> 1;
+                }
+                ++o;
+                const unsigned x = gone - base, taken = x < 32u ? 1u << x : 0u;
+                m = m & ~self & ~taken;
+                asm volatile("" ::: "memory");  // the removals before later reads (in order in the LDS)
+            };
+            for (;;) {
+                unsigned long long hit = ~0ull;
+                for (unsigned long long live; (live = __ballot(m != 0)) != 0;) {
+                    const int f = __builtin_ctzll(live), bit = __builtin_ctz(__builtin_amdgcn_readlane(m, f));
+                    p = 32 * (c + f) + bit;
+                    const int q = p + off;
+                    opp = ((unsigned)__builtin_amdgcn_readlane(w, f) >> (bit | 1)) & 1u ? 1u : 2u;
+                    const unsigned v = (ld(q >> 5) >> (q & 31)) & in;
+                    hit = __ballot((v & opp) != 0);
+                    const unsigned long long edge = __ballot(v == 3u);
+                    self = lane == f ? 1u << bit : 0u;
+                    if (__builtin_expect(hit == 0, 0)) break;
+                    const int k = __builtin_ctzll(hit);
+                    settle(__builtin_amdgcn_readlane(q, k), !((edge >> k) & 1u));
+                }
+                if (hit) break;
+                bool far = false;
+                auto at = [&](int x) { return ((ld(x >> 4) >> (2 * (x & 15))) & opp) != 0; };
+                const int pp = p >> 1, t = gs_scan(at, H, W, R, pp, pp % W, pp / W, lane, R, far);
+                if (t >= 0)
+                    settle(2 * t, t % W > 0 && t % W < W - 1 && t / W > 0 && t / W < H - 1);
+                else
+                    m &= ~self;  // nothing within reach: the residue stays unbalanced
+            }
+        }
+        const int np = (int)(o - out);
+        if (lane == 0) total = np;
+    }
+    __syncthreads();
+    // the choices are one list: rows of W of them
+    for (int y = tid; y < H; y += 256) rowpairs[(long long)blockIdx.x * H + y] = max(min(total - y * W, W), 0);
 }
 
 // The chosen cuts: one thread per choice, one grid row per row of the map (cut pixels are only set, so the
@@ -1070,7 +1184,11 @@ void goldstein(Ctx& c, const float* wrapped, int batch, int H, int W, int8_t* re
     int2* pairs = (int2*)c.buf("gs.pairs", sizeof(int2) * (size_t)tot);
     int* flag = (int*)c.buf("gs.flag", sizeof(int) * ((size_t)batch + 1));
     int* maxd = flag + batch;
-    if (words + 4096 <= lds_max) {  // beside the kernel's own 3 KiB
+    // up to GS_WALK columns one residue after the other (where a map's states fit in LDS beside the kernel's own word)
+    const size_t states = sizeof(unsigned) * ((size_t)(n + 15) / 16 + 2 * (size_t)gs_ahead(W));
+    if (W <= GS_WALK && states + 64 <= lds_max) {
+        hipLaunchKernelGGL(k_gs_walk, dim3(batch), dim3(256), states, c.stream, r, H, W, pairs, npairs, flag);
+    } else if (words + 4096 <= lds_max) {  // beside the kernel's own 3 KiB
         hipLaunchKernelGGL(k_gs_pair<true>, dim3(batch), dim3(64 * GS_WAVES), words, c.stream, r, H, W, nullptr,
                            pairs, npairs, flag);
     } else {
