@@ -1,11 +1,12 @@
 // Autotuner: for every requested volume side, times each fused volume pass (xy with projection,
-// y, zy with data consistency) with both tile sizes on this device, inside the
+// y, zy with data consistency) with both tile sizes on this device, xy and zy inside the
 // positivity loop's own pass sequence (ctdm_time_loop; each pass reads what the previous one wrote),
 // and keeps the faster choice (for y and zy, 8 only when clearly faster) in the context
-// (used by every later launch of that side, including graph captures made afterwards); then the sweep
-// direction of the xy and y passes (forward, or one of them walking the z planes backwards so that it
-// starts on the planes the previous pass wrote last), the radix plan of the y pass and the pencils per
-// workgroup of the gridding pass. An explicit call re-times every side; a reconstruction asking for
+// (used by every later launch of that side, including graph captures made afterwards); then the radix plan of the
+// y pass and the pencils per workgroup of the gridding pass. The xy and y passes walk the z planes forward: the
+// zy pass between two xy passes walks all planes at once, and the y pass runs once per volume, so that either
+// direction takes the same time (volumes of 64^3 to 256^3 with 1 and 10 iterations: within 0.7 %, the timings' own
+// spread). An explicit call re-times every side; a reconstruction asking for
 // tuning only times sides not tuned yet. The choices are also kept per (device architecture, side) for
 // the rest of the process, so contexts created later start from them. The other passes keep one radix
 // plan per length (fft_dev.hpp).
@@ -52,13 +53,13 @@ std::string autotune(Ctx& c, const int* sizes, int nsizes, bool force)
             for (int b = 0; b < 2; ++b) {  // this pass at 8 / 16 pencils, the others at their current choice
                 t.pencils[k] = b ? 16 : 8;
                 double ms[3];
-                time_loop(c, V, kIters, ms, bytes);
+                time_loop(c, V, kIters, ms, bytes, k == 1 ? TIME_Y : TIME_XY_ZY);
                 m[b] = ms[k];
             }
             t.ms[k][0] = m[0];
             t.ms[k][1] = m[1];
             // 8 y pencils write 64-byte halves of 128-byte lines, which costs more inside a replayed
-            // reconstruction than in this short timed sequence, and the zy pass's two tiles lie within the
+            // reconstruction than in these short timings, and the zy pass's two tiles lie within the
             // timing's spread at the sides where both fill the device (128^3: 14.3 and 14.7 us). These
             // take 8 only on a clear margin.
             const double margin = k == 0 ? 1.0 : 0.97;
@@ -68,24 +69,9 @@ std::string autotune(Ctx& c, const int* sizes, int nsizes, bool force)
                           names[k], m[0], m[1], t.pencils[k], bytes[k] / (1e6 * std::min(m[0], m[1])));
             rep << line;
         }
-        // Sweep directions: the sequence timed with the xy pass, then the y pass, walking the z
-        // planes backwards (outputs are identical; only the order of the tiles changes), kept when
-        // the three together are at least 1 % faster than with both forward.
-        static const int combos[3][2] = {{0, 0}, {1, 0}, {0, 1}};
-        int best = 0;
-        for (int v = 0; v < 3; ++v) {
-            t.rev[0] = combos[v][0];
-            t.rev[1] = combos[v][1];
-            double ms[3], bytes[3];
-            time_loop(c, V, kIters, ms, bytes);
-            t.sweep_ms[v] = ms[0] + ms[1] + ms[2];
-            if (t.sweep_ms[v] < (best == 0 ? 0.99 : 1.0) * t.sweep_ms[best]) best = v;
-        }
-        t.rev[0] = combos[best][0];
-        t.rev[1] = combos[best][1];
+        t.rev[0] = t.rev[1] = 0;
         char line[240];
-        std::snprintf(line, sizeof line, "V=%d sweep  fwd %.4f ms  x-rev %.4f ms  y-rev %.4f ms -> %s\n", V,
-                      t.sweep_ms[0], t.sweep_ms[1], t.sweep_ms[2], best == 0 ? "fwd" : (best == 1 ? "x-rev" : "y-rev"));
+        std::snprintf(line, sizeof line, "V=%d sweep  -> fwd\n", V);
         rep << line;
         // Radix plan of the y pass: the alternative factorisation is kept when its slowest of three timings leads
         // the base plan's fastest by 10 %. It rounds differently, so the choice must not hang on the timing's own
@@ -94,7 +80,7 @@ std::string autotune(Ctx& c, const int* sizes, int nsizes, bool force)
         for (int r = 0; r < 6; ++r) {
             t.yplan = r & 1;
             double ms[3], bytes[3];
-            time_loop(c, V, 4 * kIters, ms, bytes);
+            time_loop(c, V, 4 * kIters, ms, bytes, TIME_Y);
             if (r < 2 || (t.yplan == 0 ? ms[1] < t.yplan_ms[0] : ms[1] > t.yplan_ms[1]))
                 t.yplan_ms[t.yplan] = ms[1];
         }

@@ -62,7 +62,6 @@ struct Tune {
     int yplan = 0;                     // radix plan of the y pass: 0 Plan<V>, 1 PlanAlt<V>
     bool tuned = false;
     double ms[4][2] = {};               // measured ms per launch for B = 8, 16 (after tuning)
-    double sweep_ms[3] = {};            // xy + y + zy for sweeps (fwd, fwd), (rev, fwd), (fwd, rev)
     double yplan_ms[2] = {};            // y pass per launch with either radix plan
     double grid_ms[2] = {};             // gridding pass per launch with 8 / 16 pencils
 };
@@ -261,7 +260,9 @@ void fit_pgd(Ctx& c, float2* f, const float2* spec, const ctdm_angle* ang, int A
 double time_pass(Ctx& c, int kind, int V, int B, int reps, double* bytes);
 // Average ms of one gridding pass at side V with B pencils per workgroup for A synthetic angles.
 double time_grid(Ctx& c, int V, int B, int A, int reps);
-void time_loop(Ctx& c, int V, int iters, double ms[3], double bytes[3]);
+// `parts`: the loop's passes (ms[0], ms[2]), the y pass (ms[1]) or both; the others' entries are 0.
+enum : int { TIME_XY_ZY = 1, TIME_Y = 2 };
+void time_loop(Ctx& c, int V, int iters, double ms[3], double bytes[3], int parts = TIME_XY_ZY | TIME_Y);
 
 // Pipeline (pipeline.cpp)
 void reconstruct(Ctx& c, ctdm_cell* cells, int ncells, const ctdm_batch_opts& opts);

@@ -1253,8 +1253,7 @@ enum PassKind { PASS_X = 0, PASS_Y = 1, PASS_ZDC = 2, PASS_GRID = 3, NPASS = 4, 
 template <int V>
 struct Vol {
     static int pick(Ctx& c, PassKind k) { return c.tuning(V).pencils[k] == 8 ? 8 : 16; }
-    // Sweep direction of the xy and y passes (tuned): both walk the z planes in tile order, so running
-    // one of them backwards starts it on the planes the previous pass wrote last.
+    // Sweep direction of the xy and y passes (a tuning entry): both walk the z planes in tile order, or backwards.
     template <int IN, int OUT>
     static void xy(Ctx& c, float2* W, float2* out, const Proj& p, float scale, bool shift)
     {
@@ -1535,7 +1534,7 @@ __global__ void k_dc_synth(DcList dc, int V, int per)
 }
 
 template <int V>
-static void time_loop_v(Ctx& c, int iters, double ms[3], double bytes[3])
+static void time_loop_v(Ctx& c, int iters, double ms[3], double bytes[3], int parts)
 {
     const size_t vol = (size_t)V * V * V, VV = (size_t)V * V;
     const std::string wname = "vol.W";
@@ -1559,48 +1558,54 @@ static void time_loop_v(Ctx& c, int iters, double ms[3], double bytes[3])
     bytes[0] = vb;
     bytes[1] = vb;
     bytes[2] = vb + sizeof(int) * (double)VV + nent * (sizeof(float2) + sizeof(short));
-    fill(c, nbuf, 2 * (long long)vol, 0.f);
-    const int nk = 3 * iters;
-    std::vector<hipEvent_t> ev(2 * nk);
-    for (auto& e : ev) CTDM_HIP(hipEventCreate(&e));
+    std::vector<hipEvent_t> ev;
+    std::vector<int> pass;  // of each pair of events
     auto arm = [&](int k) {
-        c.tev[0] = ev[2 * k];
-        c.tev[1] = ev[2 * k + 1];
+        for (int i = 0; i < 2; ++i) {
+            ev.push_back(nullptr);
+            CTDM_HIP(hipEventCreate(&ev.back()));
+            c.tev[i] = ev.back();
+        }
+        pass.push_back(k);
     };
-    Vol<V>::y(c, nbuf, +1);  // warm-up
-    for (int it = 0; it < iters; ++it) {  // zeros, so that repeating the unnormalised transform keeps its values
-        arm(3 * it + 1);
-        Vol<V>::y(c, nbuf, +1);
+    if (parts & TIME_Y) {  // zeros, so that repeating the unnormalised transform keeps its values
+        fill(c, nbuf, 2 * (long long)vol, 0.f);
+        Vol<V>::y(c, nbuf, +1);  // warm-up
+        for (int it = 0; it < iters; ++it) {
+            arm(1);
+            Vol<V>::y(c, nbuf, +1);
+        }
     }
-    Vol<V>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true);  // warm-up of the sequence
-    for (int it = 0; it < iters; ++it) {
-        arm(3 * it);
-        Vol<V>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true);
-        arm(3 * it + 2);
-        Vol<V>::zy(c, W, dc);
+    if (parts & TIME_XY_ZY) {
+        Vol<V>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true);  // warm-up of the sequence
+        for (int it = 0; it < iters; ++it) {
+            arm(0);
+            Vol<V>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true);
+            arm(2);
+            Vol<V>::zy(c, W, dc);
+        }
     }
     c.tev[0] = c.tev[1] = nullptr;
-    CTDM_HIP(hipEventSynchronize(ev[2 * nk - 1]));
-    double acc[3] = {0, 0, 0};
-    for (int k = 0; k < nk; ++k) {
+    CTDM_HIP(hipEventSynchronize(ev.back()));
+    for (int k = 0; k < 3; ++k) ms[k] = 0;
+    for (size_t k = 0; k < pass.size(); ++k) {
         float t = 0;
         CTDM_HIP(hipEventElapsedTime(&t, ev[2 * k], ev[2 * k + 1]));
-        acc[k % 3] += t;
+        ms[pass[k]] += t / iters;
     }
     for (auto& e : ev) hipEventDestroy(e);
-    for (int k = 0; k < 3; ++k) ms[k] = acc[k] / iters;
 }
 
-void time_loop(Ctx& c, int V, int iters, double ms[3], double bytes[3])
+void time_loop(Ctx& c, int V, int iters, double ms[3], double bytes[3], int parts)
 {
     CTDM_REQUIRE(!c.capturing, "time_loop during capture");
     CTDM_REQUIRE(iters > 0 && ms && bytes, "time_loop: bad arguments");
     switch (V) {
-    case 32: time_loop_v<32>(c, iters, ms, bytes); break;
-    case 64: time_loop_v<64>(c, iters, ms, bytes); break;
-    case 128: time_loop_v<128>(c, iters, ms, bytes); break;
-    case 192: time_loop_v<192>(c, iters, ms, bytes); break;
-    case 256: time_loop_v<256>(c, iters, ms, bytes); break;
+    case 32: time_loop_v<32>(c, iters, ms, bytes, parts); break;
+    case 64: time_loop_v<64>(c, iters, ms, bytes, parts); break;
+    case 128: time_loop_v<128>(c, iters, ms, bytes, parts); break;
+    case 192: time_loop_v<192>(c, iters, ms, bytes, parts); break;
+    case 256: time_loop_v<256>(c, iters, ms, bytes, parts); break;
     default: fail(CTDM_EUNSUPPORTED, "time_loop: volume side has no kernel");
     }
 }

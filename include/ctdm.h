@@ -325,9 +325,8 @@ ctdm_status ctdm_reconstruct(ctdm_ctx *ctx, ctdm_cell *cells, int ncells,
 /* Times the three fused volume passes (x with projection and z with data consistency, which hold half of
  * the y transform each, and the y pass that precedes the loop) of each listed volume side V with both tile
  * sizes on this device, inside the positivity loop's own pass sequence, and caches the choice in the
- * context: the faster one, except that y and z take choice 8 only when at least 3 % faster. Then times the
- * sequence with the x or the y pass sweeping the z planes backwards (kept when at least 1 %
- * faster), the y pass with its alternative radix plan (kept when at least 10 % faster) and the gridding
+ * context: the faster one, except that y and z take choice 8 only when at least 3 % faster. Then times
+ * the y pass with its alternative radix plan (kept when at least 10 % faster) and the gridding
  * pass with 8 and 16 pencils for 60 angles (16 when at least 3 % faster). The choices also serve contexts
  * created later in the process on the same GPU architecture. No reference counterpart. Every listed
  * side is re-timed, also one tuned before. Synchronises. `report` (HOST, may be NULL) receives a text
@@ -338,7 +337,7 @@ ctdm_status ctdm_autotune(ctdm_ctx *ctx, const int *sizes, int nsizes, char *rep
 /* The tuning table entry of volume side V (no reference counterpart): values[0..6] = tile size of the x,
  * y, z+dc and gridding passes (8 or 16: pencils per workgroup of y and gridding; the x and z+dc passes take two
  * groups of pencils at 16, the default, and four at 8), the sweep direction of the x and y passes (0 forward,
- * 1 backwards over the z planes), and the radix plan of the y pass (0 the base factorisation, 1 the
+ * 1 backwards over the z planes; the tuner leaves both forward), and the radix plan of the y pass (0 the base factorisation, 1 the
  * alternative: 32 = 4x8, 64 = 4x4x4, 128 = 16x8, 192 = 16x12, 256 = 4x4x16). Pencil grouping and sweep
  * order compute bit-identical values; the two radix plans agree to FP32 rounding. ctdm_get_tuning reads the
  * entry (defaults, or choices tuned earlier in the process on the same architecture); ctdm_set_tuning
