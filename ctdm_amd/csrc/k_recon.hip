@@ -576,8 +576,7 @@ struct Tile {
     // share lines and are kept on one XCD (xcd_block).
     static constexpr bool REMAP = BFAST && B * 8 < 128;
     static __device__ int block() { return REMAP ? xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x; }
-    // rev: tiles in reverse order (the volume swept from the last plane back), so that a pass can start
-    // on the planes the previous pass wrote last
+    // rev: tiles in reverse order (the volume swept from the last plane back)
     __device__ Tile(int rev = 0)
     {
         const int tid = threadIdx.x;
@@ -922,8 +921,8 @@ __global__ __launch_bounds__(P* Split<V>::R2* Split<V>::T, 4) void k_vol_zy(floa
     }
 }
 
-// Y pass (plain FFT along y).
-template <int V, int B, int DIR, int PV>
+// Y pass (inverse FFT along y).
+template <int V, int B, int PV>
 __global__ __launch_bounds__(B* Plan<V>::T) void k_vol_y(float2* __restrict__ W, const float2* __restrict__ tw,
                                                          int rev)
 {
@@ -945,7 +944,7 @@ __global__ __launch_bounds__(B* Plan<V>::T) void k_vol_y(float2* __restrict__ W,
     tws.put(twl);
     const TwPad twp{twl};
     auto gs = [&](int k, float2 v) { store_through(pen + (long long)k * tl.stride, v); };
-    PL::template run<DIR>(tl.t, s, twp, x, gs);
+    PL::template run<+1>(tl.t, s, twp, x, gs);
 }
 
 // Compact list from a dense measured spectrum (positivity API), entries in ascending z. 64 pencils side by side per
@@ -1194,20 +1193,12 @@ struct VolOps {
             vlaunch(c, &k_vol_x<V, B, 3>, grid(), dim3(NT), W, out, c.tw(V), p, scale, (int)shift);
         CTDM_CHECK_LAUNCH("k_vol_x");
     }
-    static void y(Ctx& c, float2* W, int dir, int rev = 0, int plan = 0)
+    static void y(Ctx& c, float2* W, int rev = 0, int plan = 0)
     {
-        const float2* tw = c.tw(V);
-        if (plan == 0) {
-            if (dir < 0)
-                vlaunch(c, &k_vol_y<V, B, -1, 0>, grid(), dim3(NT), W, tw, rev);
-            else
-                vlaunch(c, &k_vol_y<V, B, +1, 0>, grid(), dim3(NT), W, tw, rev);
-        } else {
-            if (dir < 0)
-                vlaunch(c, &k_vol_y<V, B, -1, 1>, grid(), dim3(NT), W, tw, rev);
-            else
-                vlaunch(c, &k_vol_y<V, B, +1, 1>, grid(), dim3(NT), W, tw, rev);
-        }
+        if (plan == 0)
+            vlaunch(c, &k_vol_y<V, B, 0>, grid(), dim3(NT), W, c.tw(V), rev);
+        else
+            vlaunch(c, &k_vol_y<V, B, 1>, grid(), dim3(NT), W, c.tw(V), rev);
         CTDM_CHECK_LAUNCH("k_vol_y");
     }
     // W == nullptr: the list only.
@@ -1261,11 +1252,11 @@ struct Vol {
         if (pick(c, PASS_X) == 8) LoopOps<V, 2>::template xy<IN, OUT>(c, W, out, p, scale, shift, rev);
         else LoopOps<V, 1>::template xy<IN, OUT>(c, W, out, p, scale, shift, rev);
     }
-    static void y(Ctx& c, float2* W, int dir)
+    static void y(Ctx& c, float2* W)
     {
         const int rev = c.tuning(V).rev[1], plan = c.tuning(V).yplan;
-        if (pick(c, PASS_Y) == 8) VolOps<V, 8>::y(c, W, dir, rev, plan);
-        else VolOps<V, 16>::y(c, W, dir, rev, plan);
+        if (pick(c, PASS_Y) == 8) VolOps<V, 8>::y(c, W, rev, plan);
+        else VolOps<V, 16>::y(c, W, rev, plan);
     }
     static unsigned zy_blocks(Ctx& c)
     {
@@ -1343,7 +1334,7 @@ static void volume_batched_v(Ctx& c, const float2* spec, const double* rows, int
     const DcList dc = dc_alloc(c, V, std::max(A, 1));
     float2* W = (float2*)c.buf("vol.W", sizeof(float2) * (size_t)V * V * V);
     Vol<V>::grid_pass(c, spec, rows, A, g, flags & CTDM_DC_REFCOMPAT, W, dc);
-    Vol<V>::y(c, W, +1);
+    Vol<V>::y(c, W);
     Vol<V>::loop(c, W, n_out, dc, make_proj(g), iters, !(flags & CTDM_POS_NO_SHIFT), true);
 }
 
@@ -1487,7 +1478,8 @@ static double time_pass_v(Ctx& c, int kind, int B, int reps, double* bytes)
     *bytes = vb + extra;
     const long long n4 = (long long)vol / 2;  // float4 = two complex values
     const int copy_grid = (int)std::min<long long>(grid1d(n4, 256), 8192);
-    auto launch = [&](int r) {
+    if (kind == PASS_Y) fill(c, nbuf, 2 * (long long)vol, 0.f);  // so that repeating the unnormalised transform keeps its values
+    auto launch = [&] {
         switch (kind) {
         case PASS_COPY:
             hipLaunchKernelGGL(k_copy_vol, dim3(copy_grid), dim3(256), 0, c.stream, (const float4*)W, (float4*)nbuf, n4);
@@ -1495,17 +1487,17 @@ static double time_pass_v(Ctx& c, int kind, int B, int reps, double* bytes)
             break;
         case PASS_X: B == 8 ? LoopOps<V, 2>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true, 0)
                             : LoopOps<V, 1>::template xy<2, 0>(c, W, nbuf, p, 1.f / (float)vol, true, 0); break;
-        case PASS_Y: B == 8 ? VolOps<V, 8>::y(c, W, (r & 1) ? 1 : -1) : VolOps<V, 16>::y(c, W, (r & 1) ? 1 : -1); break;
+        case PASS_Y: B == 8 ? VolOps<V, 8>::y(c, nbuf) : VolOps<V, 16>::y(c, nbuf); break;
         case PASS_ZDC: B == 8 ? LoopOps<V, 2>::zy(c, W, dc, 1.f) : LoopOps<V, 1>::zy(c, W, dc, 1.f); break;
         default: fail(CTDM_EINVAL, "time_pass: unknown pass");
         }
     };
-    launch(0);  // warm-up
+    launch();  // warm-up
     hipEvent_t e0, e1;
     CTDM_HIP(hipEventCreate(&e0));
     CTDM_HIP(hipEventCreate(&e1));
     CTDM_HIP(hipEventRecord(e0, c.stream));
-    for (int r = 0; r < reps; ++r) launch(r + 1);
+    for (int r = 0; r < reps; ++r) launch();
     CTDM_HIP(hipEventRecord(e1, c.stream));
     CTDM_HIP(hipEventSynchronize(e1));
     float ms = 0;
@@ -1570,10 +1562,10 @@ static void time_loop_v(Ctx& c, int iters, double ms[3], double bytes[3], int pa
     };
     if (parts & TIME_Y) {  // zeros, so that repeating the unnormalised transform keeps its values
         fill(c, nbuf, 2 * (long long)vol, 0.f);
-        Vol<V>::y(c, nbuf, +1);  // warm-up
+        Vol<V>::y(c, nbuf);  // warm-up
         for (int it = 0; it < iters; ++it) {
             arm(1);
-            Vol<V>::y(c, nbuf, +1);
+            Vol<V>::y(c, nbuf);
         }
     }
     if (parts & TIME_XY_ZY) {
@@ -1675,24 +1667,24 @@ static double time_pass_512(Ctx& c, int kind, int reps, double* bytes)
     const size_t vol = (size_t)V * V * V;
     float2* W = (float2*)c.buf("tp.W512", sizeof(float2) * vol);
     float2* dst = kind == PASS_COPY ? (float2*)c.buf("tp.n512", sizeof(float2) * vol) : nullptr;
-    fill(c, W, 2 * (long long)vol, 1.f);
+    fill(c, W, 2 * (long long)vol, 0.f);
     *bytes = 2.0 * sizeof(float2) * vol;
     const long long n4 = (long long)vol / 2;
     const int copy_grid = (int)std::min<long long>(grid1d(n4, 256), 8192);
-    auto launch = [&](int r) {
+    auto launch = [&] {
         if (kind == PASS_COPY) {
             hipLaunchKernelGGL(k_copy_vol, dim3(copy_grid), dim3(256), 0, c.stream, (const float4*)W, (float4*)dst, n4);
             CTDM_CHECK_LAUNCH("k_copy_vol");
         } else {
-            VolOps<V, 8>::y(c, W, (r & 1) ? 1 : -1);
+            VolOps<V, 8>::y(c, W);
         }
     };
-    launch(0);
+    launch();
     hipEvent_t e0, e1;
     CTDM_HIP(hipEventCreate(&e0));
     CTDM_HIP(hipEventCreate(&e1));
     CTDM_HIP(hipEventRecord(e0, c.stream));
-    for (int r = 0; r < reps; ++r) launch(r + 1);
+    for (int r = 0; r < reps; ++r) launch();
     CTDM_HIP(hipEventRecord(e1, c.stream));
     CTDM_HIP(hipEventSynchronize(e1));
     float ms = 0;

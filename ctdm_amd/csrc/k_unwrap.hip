@@ -54,24 +54,17 @@ __device__ __forceinline__ float wrapdiff(float t)
     return r;
 }
 
-// RHS at (i, j) of an N x N map.
-__device__ __forceinline__ float rhs_at(const float* __restrict__ p, int N, int i, int j, bool sincos)
+// Sine right-hand side at (i, j) of an N x N map.
+__device__ __forceinline__ float sin_rhs_at(const float* __restrict__ p, int N, int i, int j)
 {
     const int k = i + N * j;
     const float c = p[k];
-    if (sincos) {
-        float r = 0.f;
-        if (i < N - 1) r += sinf(p[k + 1] - c);
-        if (i > 0) r += sinf(p[k - 1] - c);
-        if (j < N - 1) r += sinf(p[k + N] - c);
-        if (j > 0) r += sinf(p[k - N] - c);
-        return r;
-    }
-    const float c1 = (i == N - 1) ? 0.f : wrapdiff(p[k + 1] - c);
-    const float c2 = (i == 0) ? 0.f : wrapdiff(c - p[k - 1]);
-    const float c3 = (j == N - 1) ? 0.f : wrapdiff(p[k + N] - c);
-    const float c4 = (j == 0) ? 0.f : wrapdiff(c - p[k - N]);
-    return (c1 - c2) + (c3 - c4);
+    float r = 0.f;
+    if (i < N - 1) r += sinf(p[k + 1] - c);
+    if (i > 0) r += sinf(p[k - 1] - c);
+    if (j < N - 1) r += sinf(p[k + N] - c);
+    if (j > 0) r += sinf(p[k - N] - c);
+    return r;
 }
 
 // Makhoul source index: position n of v holds x[src(n)].
@@ -837,8 +830,10 @@ static void run_rows_fwd(Ctx& c, const float* in, int batch, int rhs, float* out
         hipLaunchKernelGGL((k_uw_rows_fwd<N, RHS_WRAP>), grid, block, 0, c.stream, in, tw, tw4, out);
     else if (rhs == RHS_SIN)
         hipLaunchKernelGGL((k_uw_rows_fwd<N, RHS_SIN>), grid, block, 0, c.stream, in, tw, tw4, out);
-    else
+    else if constexpr (N > 64)
         hipLaunchKernelGGL((k_uw_rows_fwd<N, RHS_NONE>), grid, block, 0, c.stream, in, tw, tw4, out);
+    else
+        fail(CTDM_EUNSUPPORTED, "a right-hand side given as it is takes the one-workgroup solve at this size");
     CTDM_CHECK_LAUNCH("k_uw_rows_fwd");
 }
 
@@ -872,6 +867,8 @@ static void run_rows_inv(Ctx& c, const float* in, int batch, unsigned flags, con
         using PR = Pair<N>;
         hipLaunchKernelGGL((k_uw_rows_inv<N>), dim3((unsigned)((long long)batch * N / (2 * PR::GP))), dim3(PR::NT), 0,
                            c.stream, in, wrapped, c.tw(N), c.tw(4 * N), out);
+    } else {
+        fail(CTDM_EUNSUPPORTED, "rows of this size are solved with the whole map");
     }
     CTDM_CHECK_LAUNCH("k_uw_rows_inv");
 }
@@ -1081,16 +1078,12 @@ void unwrap_dct_adjoint(Ctx& c, const float* wrapped, const float* g_out, float*
             return;
         }
         Work w;
-        w.D1 = (float*)c.buf("uw.D1", sizeof(float) * n);
-        w.D2 = (float*)c.buf("uw.D2", sizeof(float) * n);
         w.num = eig_table(c, M, false);
         solve_any(c, g_out, batch, M, F_REF_EIG, 1, nullptr, g_in, w);
         return;
     }
     float* tmp = (float*)c.buf("uw.adj", sizeof(float) * n);
     Work w;
-    w.D1 = (float*)c.buf("uw.D1", sizeof(float) * n);
-    w.D2 = (float*)c.buf("uw.D2", sizeof(float) * n);
     if (!refeig) w.dc = (float*)c.buf("uw.dc", sizeof(float) * (size_t)batch);
     solve_any(c, g_out, batch, M, flags & F_REF_EIG, 1, nullptr, tmp, w);
     const long long quads = (long long)n / 4;
@@ -1132,7 +1125,7 @@ __global__ void k_sincos_rhs(float* __restrict__ o, const float* __restrict__ in
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
     if (i >= N || j >= N) return;
-    o[i + N * j] = rhs_at(in, N, i, j, true);
+    o[i + N * j] = sin_rhs_at(in, N, i, j);
 }
 
 // float2cufft (DCT_Unwrapping.cu:144-162): row mirror to length 2N.
