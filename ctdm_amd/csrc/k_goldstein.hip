@@ -491,9 +491,9 @@ __global__ __launch_bounds__(64 * GS_WAVES) void k_gs_pair(const int8_t* __restr
 // map's edges (no ring is clipped before the one that touches the border, which holds a hit).
 // Bound by the instructions from one residue to the next, about 90 ns a residue, hence the common case as a loop of its
 // own. Against the pipeline, at noise of 0.6 and 0.8 pi (density 0.09 and 0.28), in us: one map of 4000 x 16 560 and 1619 (2445,
-// 4265), 2000 x 40 734 and 2061 (1924, 2764), 520 x 48 239 and 637 (557, 737), 520 x 64 330 and 869 (515, 780): up to 48
-// columns it is the faster one at every density.
-constexpr int GS_WALK = 48;
+// 4265), 2000 x 40 734 and 2061 (1924, 2764), 520 x 48 239 and 637 (557, 737), 1000 x 60 561 and 1549 (1145, 1465), 520 x 64
+// 330 and 869 (515, 780). The line lies where the densest maps begin to lose more than the others gain.
+constexpr int GS_WALK = 60;
 constexpr __host__ __device__ int gs_ahead(int W) { return 5 * (W + 1) / 16 + 2; }
 __device__ __forceinline__ unsigned spread_bits(unsigned v)  // bit b of the low half to bit 2 b
 {

@@ -27,7 +27,7 @@ def _noisy(rng, shape, noise):
     return (p - 2 * np.pi * np.round(p / (2 * np.pi))).astype(np.float32)
 
 
-@pytest.mark.parametrize("W", [3, 4, 5, 8, 9, 10, 15, 16, 17, 31, 32, 33, 47, 48, 49])
+@pytest.mark.parametrize("W", [3, 4, 5, 8, 9, 10, 15, 16, 17, 31, 32, 33, 48, 59, 60, 61])
 @pytest.mark.parametrize("H", [3, 33, 64, 500])
 def test_few_columns(ctx, orc, H, W):
     """Widths around the words of 16 pixels, the rings that fit (W / 2) and the last width of this path, heights below and
@@ -37,7 +37,7 @@ def test_few_columns(ctx, orc, H, W):
         _equal(ctx, orc, _noisy(rng, (3, H, W), noise))
 
 
-@pytest.mark.parametrize("W", [20, 48])
+@pytest.mark.parametrize("W", [20, 60])
 def test_far_and_unreachable_charges(ctx, orc, W):
     """Vortices of one sign far from each other and from the borders: scans that go past the first 64 positions, and
     ones that end without a hit (a residue in the middle column, with the largest ring short of both borders)."""
