@@ -33,9 +33,9 @@ COMMON = [
 
 
 # Per-source flags. k_goldstein.hip: its floating-point results must match the host specification bit
-# for bit (no multiply-add contraction), and its single-lane LDS clears in the one-wavefront commit loop
-# must stay single instructions (the atomic optimizer would wrap each in lane-counting code; the module
-# aggregates its queue appends itself).
+# for bit (no multiply-add contraction), and the LDS atomics of one or two lanes with which k_gs_pair and
+# k_gs_walk remove a pair's charges must stay single instructions (the atomic optimizer would wrap each in
+# lane-counting code; the search aggregates its queue appends itself).
 EXACT_FP = {"k_goldstein.hip": ["-ffp-contract=off", "-mllvm", "-amdgpu-atomic-optimizer-strategy=None"]}
 
 

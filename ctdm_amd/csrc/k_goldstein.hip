@@ -178,7 +178,7 @@ constexpr int GS_ROWS = GS_WAVES * 64 / GS_LANES; // rows in flight
 constexpr int GS_LEFT = INT_MIN;                  // published by a group that leaves its rows undecided
 
 // The charges still present as two bit arrays, positive and negative, with the border's bits set in both; nw
-// words each, one spare word before them and two after. In LDS when they fit (maps up to 0.65 M pixels), else in global memory, read and
+// words each, one spare word before them and two after. In LDS when they fit (maps up to 0.63 M pixels), else in global memory, read and
 // cleared by atomics at device scope, which bypass the vector L1.
 template <bool LDSW>
 struct Charges {

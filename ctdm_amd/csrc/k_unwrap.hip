@@ -580,7 +580,7 @@ __global__ __launch_bounds__(Pair<N>::NT) void k_uw_rows_inv_rytov(const float* 
 // pairs, the row pairs again; the same operations in the same order as the three kernels, and the same bits. For a few
 // maps the three are launches and latency, for many they write and read the coefficients: 1 map of 64^2 12.4 us in
 // three launches, 8.3 in one; 256 17.0 and 9.3; 4096 81 and 62; 32^2 11.8 and 6.5, 30 and 23. One 256^2 hologram pair to an
-// unwrapped 64^2 map 28.8 and 21.8.
+// unwrapped 64^2 map 28.0 and 21.0.
 template <int N, int RHS>
 __global__ __launch_bounds__(N / 2 * Pair<N>::T) void k_uw_map(const float* __restrict__ in, const float* __restrict__ wrapped,
                                                             unsigned flags, const double* __restrict__ eig,

@@ -7,7 +7,7 @@
 //                   cudaMemcpy / cudaThreadSynchronize points, HilbertTransform.cu:785-1165,
 //                   1825-2047, FFT.cu:655-736).
 // batched (mode 1): all angles of a cell per launch, fused passes (3 retrieval, 3 unwrap,
-//                   2 Rytov, 3 + 4*iters volume kernels), optionally captured once into a hipGraph
+//                   2 Rytov, 3 + 2*iters volume kernels), optionally captured once into a hipGraph
 //                   and replayed.
 #include <algorithm>
 #include <cmath>
