@@ -738,10 +738,10 @@ __device__ __forceinline__ bool tbit(const unsigned* b, long long p) { return (b
 // index by compare-and-swap, so pointers only fall, every walk ends, and a failed swap means that another one joined that root.
 // Every edge between free pixels is then checked (k_gs_tile within tiles, k_gs_anchor across their borders). A map with
 // an edge that disagrees, or with a step outside 32 bits, is flagged and takes the search of 3c, whose kernels return at
-// once for the others: whatever the input, the counts are the search's own. 64 maps of 512^2 (noise 0.8 rad; a map in
-// about 100 is flagged): fill and outputs 0.41 ms in place of 1.92 (k_gs_tile 0.10, merge 0.04, anchor 0.03, the idle search
-// 0.03, finish 0.21), 1.22 with a flagged map among them; one map of 256^2 60 us in place of 320. Tiles of 16 rows: 0.42,
-// of 64 (1024 threads) 0.41.
+// once for the others: whatever the input, the counts are the search's own. 64 maps of 512^2 (noise +-0.8 pi; about one
+// map in 1000 is flagged): fill and outputs 0.41 ms in place of 1.92 (k_gs_tile 0.10, merge 0.04, anchor 0.03, the idle search
+// 0.03, finish 0.21), 1.2 to 1.5 with a flagged map among them; one map of 256^2 60 us in place of 320. Tiles of 16 rows:
+// 0.42, of 64 (1024 threads) 0.41.
 constexpr int GS_TX = 64, GS_TY = 32;  // a tile: a wave's width, four rows for each of eight waves
 __device__ __forceinline__ unsigned long long gs_pack(int ptr, unsigned sum)
 {
